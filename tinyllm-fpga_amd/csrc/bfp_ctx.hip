@@ -15,6 +15,7 @@
 #include "bfp_mx.h"
 #include "bfp_persist.h"
 #include "bfp_pipe.h"
+#include "bfp_prefill.h"
 
 using namespace bfp;
 
@@ -112,6 +113,14 @@ struct bfp_ctx {
     bool ok = false;
   };
   std::vector<PipeSched> pp_sched;   // by batch size (index batch - 1)
+  // the prompt pass (bfp_prefill.hip), made on its first use: activations of
+  // pf_rows rows
+  int pf_rows = 0;
+  int16_t *pf_h_m = nullptr, *pf_h1_m = nullptr, *pf_qkv_m = nullptr, *pf_att_m = nullptr, *pf_mlp_m = nullptr,
+          *pf_xn_m = nullptr;
+  int8_t *pf_h_e = nullptr, *pf_h1_e = nullptr, *pf_qkv_e = nullptr, *pf_att_e = nullptr, *pf_mlp_e = nullptr,
+         *pf_xn_e = nullptr;
+  double *pf_q = nullptr;
   std::vector<void *> allocs;
   // pinned, mapped host memory through which the single-layer boundary call
   // (bfp_layer_step_kv) passes its input and output, read and written by
@@ -393,10 +402,93 @@ int pipe_args(bfp_ctx *c, const bfp_ctx::PipeSched &ps, int batch, int16_t *dhm,
   return BFP_OK;
 }
 
-// The whole batch-1 decode as one persistent launch (bfp_persist.hip).
+// Positions of one prompt pass per sequence: as many as PF_ROWS rows hold,
+// the prompt in equal parts.
+int prefill_chunk(int batch, int n_prompt) {
+  const int most = PF_ROWS / batch;
+  if (most < 1) return 0;
+  const int parts = (n_prompt + most - 1) / most;
+  return (n_prompt + parts - 1) / parts;
+}
+
+// Steps 0 .. n_prompt-1 of a decode as passes over the prompt's positions
+// (bfp_prefill.hip): the cache rows and the history those steps leave.
+int prefill(bfp_ctx *c, const int *dprompt, int n_prompt, int batch, int16_t *dhm, int8_t *dhe, int steps) {
+  const bfp_dims &d = c->d;
+  hipStream_t s = c->stream;
+  const int n = prefill_chunk(batch, n_prompt), rows = batch * n;
+  if (rows > c->pf_rows) {
+    // the most rows any call of this context takes, at once
+    const size_t R = (size_t)std::min<long long>(PF_ROWS, (long long)c->max_batch * c->max_ctx);
+    const size_t D = d.D, nq = D + 2 * (size_t)d.H_KV * d.HD, F = d.FFN;
+    BFP_TRY(prepare_prefill_kernels());
+    BFP_TRY(c->alloc((void **)&c->pf_h_m, 2 * R * D));
+    BFP_TRY(c->alloc((void **)&c->pf_h_e, R * D / 16));
+    BFP_TRY(c->alloc((void **)&c->pf_h1_m, 2 * R * D));
+    BFP_TRY(c->alloc((void **)&c->pf_h1_e, R * D / 16));
+    BFP_TRY(c->alloc((void **)&c->pf_qkv_m, 2 * R * nq));
+    BFP_TRY(c->alloc((void **)&c->pf_qkv_e, R * nq / 16));
+    BFP_TRY(c->alloc((void **)&c->pf_att_m, 2 * R * D));
+    BFP_TRY(c->alloc((void **)&c->pf_att_e, R * D / 16));
+    BFP_TRY(c->alloc((void **)&c->pf_mlp_m, 2 * R * F));
+    BFP_TRY(c->alloc((void **)&c->pf_mlp_e, R * F / 16));
+    BFP_TRY(c->alloc((void **)&c->pf_xn_m, 2 * R * D));
+    BFP_TRY(c->alloc((void **)&c->pf_xn_e, R * D / 16));
+    BFP_TRY(c->alloc((void **)&c->pf_q, sizeof(double) * R * D));
+    c->pf_rows = (int)R;
+  }
+  if (rows > c->pf_rows) return set_err(BFP_EINVAL, "prefill: %d rows of %d", rows, c->pf_rows);
+  PrefillArgs a{};
+  a.batch = batch;
+  a.prompt = dprompt;
+  a.n_prompt = n_prompt;
+  a.VOCAB = d.VOCAB;
+  a.embed = c->embed;
+  a.qf = c->pf_q;
+  a.hist_m = dhm;
+  a.hist_e = dhe;
+  a.hist_steps = steps;
+  for (int p0 = 0; p0 < n_prompt; p0 += n) {
+    a.p0 = p0;
+    a.n = std::min(n, n_prompt - p0);
+    for (int l = 0; l < d.NL; ++l) {
+      LayerArgs &L = a.L = layer_args(c, l, batch * a.n);
+      L.h_m = c->pf_h_m;
+      L.h_e = c->pf_h_e;
+      L.h1_m = c->pf_h1_m;
+      L.h1_e = c->pf_h1_e;
+      L.qkv_m = c->pf_qkv_m;
+      L.qkv_e = c->pf_qkv_e;
+      L.att_m = c->pf_att_m;
+      L.att_e = c->pf_att_e;
+      L.mlp_m = c->pf_mlp_m;
+      L.mlp_e = c->pf_mlp_e;
+      L.xn_m = c->pf_xn_m;
+      L.xn_e = c->pf_xn_e;
+      if (l == 0) BFP_TRY(launch_prefill_embed(a, s));
+      BFP_TRY(launch_prefill_layer(a, s));
+    }
+  }
+  return BFP_OK;
+}
+
+// The steps a decode runs as prompt passes: the prompt's, when it is long
+// enough to pay for a pass and nothing asks for each step on its own (the
+// FPGA loop records every step's prediction; direct launches, step times,
+// traces and the abort hook are per step).
+int prefill_steps(int batch, int n_prompt, int flags, bool persist) {
+  const int per_step = BFP_DECODE_RTL_LOOP | BFP_DECODE_NO_GRAPH | BFP_DECODE_STEP_TIMES | BFP_DECODE_TRACE |
+                       BFP_DECODE_ABORT_TEST;
+  if (flags & per_step) return 0;
+  const int n = prefill_chunk(batch, n_prompt);
+  return n >= (persist ? PF_MIN_PERSIST : PF_MIN) ? n_prompt : 0;
+}
+
+// The whole batch-1 decode as one persistent launch (bfp_persist.hip);
+// its first step0 steps (0 or n_prompt) as prompt passes before it.
 int decode_persist(bfp_ctx *c, PersistArgs pa, int grid, const int *dprompt, int n_prompt,
                    int n_gen, int *dout, int16_t *dhm, int8_t *dhe, bool rtl_loop, bool trace,
-                   bool abort_test) {
+                   bool abort_test, int step0, int tok0) {
   const bfp_dims &d = c->d;
   hipStream_t s = c->stream;
   const int steps = n_prompt + n_gen;
@@ -435,6 +527,8 @@ int decode_persist(bfp_ctx *c, PersistArgs pa, int grid, const int *dprompt, int
   pa.n_prompt = n_prompt;
   pa.n_gen = n_gen;
   pa.rtl_loop = rtl_loop ? 1 : 0;
+  pa.step0 = step0;
+  pa.tok0 = tok0;
   pa.prompt = dprompt;
   pa.out = dout;
   pa.last = c->last;
@@ -453,7 +547,8 @@ int decode_persist(bfp_ctx *c, PersistArgs pa, int grid, const int *dprompt, int
   HIP_TRY(hipEventCreate(&ev0));
   HIP_TRY(hipEventCreate(&ev1));
   (void)hipEventRecord(ev0, s);
-  int rc = launch_decode_persist(pa, c->pt_args, grid, c->max_ctx, s);
+  int rc = step0 > 0 ? prefill(c, dprompt, n_prompt, 1, dhm, dhe, steps) : BFP_OK;
+  if (!rc) rc = launch_decode_persist(pa, c->pt_args, grid, c->max_ctx, s);
   (void)hipEventRecord(ev1, s);
   if (!rc) {
     hipError_t e = hipStreamSynchronize(s);
@@ -478,7 +573,10 @@ int decode_persist(bfp_ctx *c, PersistArgs pa, int grid, const int *dprompt, int
     c->last_decode_ms = ms;
     c->last_gen_ms = n_gen > 0 ? (float)((double)(clk[steps] - clk[n_prompt]) * tick_ms) : 0.f;
     c->step_ms.resize(steps);
-    for (int k = 0; k < steps; ++k) c->step_ms[k] = (float)((double)(clk[k + 1] - clk[k]) * tick_ms);
+    for (int k = step0; k < steps; ++k) c->step_ms[k] = (float)((double)(clk[k + 1] - clk[k]) * tick_ms);
+    // the steps of a prompt pass: equal shares of the time before the launch's first step
+    const double pre = ms - (double)(clk[steps] - clk[step0]) * tick_ms;
+    for (int k = 0; k < step0; ++k) c->step_ms[k] = (float)(std::max(pre, 0.0) / step0);
     c->last_path = BFP_PATH_PERSIST;
     c->last_form = BFP_FORM_PERSIST;
     if (dtrace) {
@@ -1279,19 +1377,25 @@ int bfp_decode(bfp_ctx *c, const int32_t *prompt, int n_prompt, int n_gen, int b
     BFP_TRY(tmp.alloc((void **)&dhe, (size_t)batch * steps * d.NL * d.D / 16));
   }
   HIP_TRY(hipMemcpyAsync(dprompt, prompt, sizeof(int) * batch * n_prompt, hipMemcpyHostToDevice, s));
-  std::vector<int> st(batch + 2, 0);   // step, next inputs, k_ctl_embed's arrival count
-  for (int b = 0; b < batch; ++b) st[1 + b] = prompt[b * n_prompt];
-  HIP_TRY(hipMemcpyAsync(c->state, st.data(), sizeof(int) * (batch + 2), hipMemcpyHostToDevice, s));
 
   PersistArgs pa{};
   int grid = 0;
   if (batch == 1 && !(flags & (BFP_DECODE_NO_GRAPH | BFP_DECODE_NO_PERSIST)) && persist_enabled() &&
       persist_plan(d, c->max_ctx, c->device, pa, grid)) {
+    const int step0 = prefill_steps(batch, n_prompt, flags, true);
     BFP_TRY(decode_persist(c, pa, grid, dprompt, n_prompt, n_gen, dout, dhm, dhe, rtl_loop,
-                           (flags & BFP_DECODE_TRACE) != 0, (flags & BFP_DECODE_ABORT_TEST) != 0));
+                           (flags & BFP_DECODE_TRACE) != 0, (flags & BFP_DECODE_ABORT_TEST) != 0, step0,
+                           prompt[step0 ? n_prompt - 1 : 0]));
     return decode_copy_out(c, batch, steps, n_out, dout, tokens_out, dhm, dhe, hist_m, hist_e);
   }
   c->last_path = (flags & BFP_DECODE_NO_GRAPH) ? BFP_PATH_EAGER : BFP_PATH_GRAPH;
+  // the first step0 steps as prompt passes; the step after them feeds the
+  // last prompt token once more
+  const int step0 = prefill_steps(batch, n_prompt, flags, false);
+  std::vector<int> st(batch + 2, 0);   // step, next inputs, k_ctl_embed's arrival count
+  st[0] = step0;
+  for (int b = 0; b < batch; ++b) st[1 + b] = prompt[b * n_prompt + (step0 ? n_prompt - 1 : 0)];
+  HIP_TRY(hipMemcpyAsync(c->state, st.data(), sizeof(int) * (batch + 2), hipMemcpyHostToDevice, s));
   // the pipelined step (one launch for the step's layers) unless the
   // per-stage launches are asked for or traced
   bfp_ctx::PipeSched *pipe = nullptr;
@@ -1357,7 +1461,8 @@ int bfp_decode(bfp_ctx *c, const int32_t *prompt, int n_prompt, int n_gen, int b
   hipGraph_t gr[2] = {nullptr, nullptr};
   int rc = BFP_OK;
   if (use_graph) {
-    for (int k = 0; k < 2 && !rc; ++k) {
+    // k = 0: a step without the head (before the prompt's end)
+    for (int k = step0 > 0 || rtl_loop ? 1 : 0; k < 2 && !rc; ++k) {
       HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
       rc = enqueue_step(k == 1);
       hipError_t e1 = hipStreamEndCapture(s, &gr[k]);
@@ -1380,8 +1485,9 @@ int bfp_decode(bfp_ctx *c, const int32_t *prompt, int n_prompt, int n_gen, int b
     (void)hipEventCreate(&ev1);
     (void)hipEventCreate(&evg);
     (void)hipEventRecord(ev0, s);
-    if (steps > 0) rc = launch_embed(ea, s);
-    for (int step = 0; step < steps && !rc; ++step) {
+    if (step0 > 0) rc = prefill(c, dprompt, n_prompt, batch, dhm, dhe, steps);
+    if (!rc && steps > step0) rc = launch_embed(ea, s);
+    for (int step = step0; step < steps && !rc; ++step) {
       const bool head = rtl_loop || step >= n_prompt - 1;
       if (step == n_prompt) (void)hipEventRecord(evg, s);
       if (per_step) (void)hipEventRecord(sev[step], s);

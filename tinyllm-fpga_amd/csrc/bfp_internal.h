@@ -75,6 +75,9 @@ struct EmbedArgs;
 // set_mx_trace names (batched decodes traced with BFP_DECODE_TRACE).
 int launch_layer(const LayerArgs &a, hipStream_t s, bool mx_traced = false);
 int set_mx_trace(unsigned long long *p);
+// A layer's stages around the attention for the rows of a prompt pass.
+int launch_rows_qkv(const LayerArgs &a, hipStream_t s);
+int launch_rows_post(const LayerArgs &a, hipStream_t s);
 // The launch form launch_layer takes for a (BFP_FORM_* bits).
 int layer_form(const LayerArgs &a);
 int prepare_layer_kernels(int max_ctx, int D, int FFN);

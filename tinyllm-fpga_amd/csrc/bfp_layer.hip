@@ -1308,6 +1308,23 @@ int launch_layer(const LayerArgs &a, hipStream_t s, bool mx_traced) {
   return launch_status("layer");
 }
 
+// The stages of a layer around the attention for the rows of a prompt pass
+// (bfp_prefill.hip): RMSNorm 1 and Q|K|V; O, RMSNorm 2, G/U and D.
+int launch_rows_qkv(const LayerArgs &a, hipStream_t s) {
+  const int nTD = a.D / 16, G = (a.batch + MX_SEQ - 1) / MX_SEQ, bq = (a.D + 2 * a.KV) / 16;
+  launch_norm_seq(a, 1, s);
+  hipLaunchKernelGGL(k_qkv_mx<false>, dim3(bq, G), dim3(64 * mx_waves(nTD, bq * G)), mx_lds_bytes(1, nTD), s, a);
+  return launch_status("rows qkv");
+}
+int launch_rows_post(const LayerArgs &a, hipStream_t s) {
+  const int nTD = a.D / 16, nTF = a.FFN / 16, G = (a.batch + MX_SEQ - 1) / MX_SEQ, bo = a.D / 16, bg = a.FFN / 16;
+  hipLaunchKernelGGL(k_o_res_mx<false>, dim3(bo, G), dim3(64 * mx_waves(nTD, bo * G)), mx_lds_bytes(1, nTD), s, a);
+  launch_norm_seq(a, 2, s);
+  hipLaunchKernelGGL(k_gu_mx<false>, dim3(bg, G), dim3(64 * mx_waves(nTD, bg * G)), mx_lds_bytes(2, nTD), s, a);
+  hipLaunchKernelGGL(k_d_res_mx<false>, dim3(bo, G), dim3(64 * mx_waves_d(a)), mx_lds_bytes(1, nTF), s, a);
+  return launch_status("rows post");
+}
+
 int launch_embed(const EmbedArgs &a, hipStream_t s) {
   hipLaunchKernelGGL(k_embed, dim3(a.batch), dim3(256), 0, s, a);
   return launch_status("embed");

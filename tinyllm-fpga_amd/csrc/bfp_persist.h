@@ -15,6 +15,7 @@ struct PersistArgs {
   int n_qkv, n_att;              // Q|K|V chunks; attention jobs per layer step
   int o0, g0, d0, n_d;           // first workgroup of the O, G/U and D roles; D chunks
   int steps, n_prompt, n_gen, rtl_loop;
+  int step0, tok0;               // first step of the launch and its input token
   const int *prompt;             // device, n_prompt ids
   int *out, *last;               // recorded argmaxes; the last head's argmax
   const float *embed;            // (VOCAB, D) float32, tied embedding and head

@@ -436,8 +436,8 @@ __device__ void role_qkv(const PT_CONST PersistArgs *pp, double *dsm, int c) {
   Gammas G1;
   load_chunk_rs(R, L[0].w_qkv_m + (long long)c * nT * 32, L[0].w_qkv_e + (long long)c * nT * 16, nT);
   load_gammas(G1, L[0].g1, D);
-  int tok = clamp_tok(p, p.prompt[0]);
-  for (int s = 0; s < p.steps; ++s) {
+  int tok = clamp_tok(p, p.tok0);
+  for (int s = p.step0; s < p.steps; ++s) {
     if (c == 0 && threadIdx.x == 0 && p.clock) put_clock(p.clock, s);
     const rsrc_t rq = rsrc(p.t_qkv + (s & 1) * nq);
     for (int l = 0; l < p.NL; ++l) {
@@ -510,8 +510,8 @@ __device__ void role_o(const PT_CONST PersistArgs *pp, double *dsm, int c) {
   __shared__ long long redA[PT_NW * 16];
   ChunkRegs<2> R;
   load_chunk_rs(R, L[0].w_o_m + (long long)c * nT * 32, L[0].w_o_e + (long long)c * nT * 16, nT);
-  int tok = clamp_tok(p, p.prompt[0]);
-  for (int s = 0; s < p.steps; ++s) {
+  int tok = clamp_tok(p, p.tok0);
+  for (int s = p.step0; s < p.steps; ++s) {
     const rsrc_t rh = rsrc(p.t_h + (s & 1) * D), ra = rsrc(p.t_att + (s & 1) * D);
     const rsrc_t r1 = rsrc(p.t_h1 + (s & 1) * D);
     for (int l = 0; l < p.NL; ++l) {
@@ -570,7 +570,7 @@ __device__ void role_gu(const PT_CONST PersistArgs *pp, double *dsm, int c) {
                   L[l].w_gu_e + (long long)(2 * c + 1) * nT * 16, nT);
   };
   load_w(0);
-  for (int s = 0; s < p.steps; ++s) {
+  for (int s = p.step0; s < p.steps; ++s) {
     const rsrc_t r1 = rsrc(p.t_h1 + (s & 1) * D), rmlp = rsrc(p.t_mlp + (s & 1) * p.FFN);
     for (int l = 0; l < p.NL; ++l) {
       const unsigned tg = tag_of(s, l, p.NL);
@@ -610,7 +610,7 @@ __device__ void role_d(const PT_CONST PersistArgs *pp, double *dsm, int c) {
   __shared__ long long redA[PT_NW * 16];
   ChunkRegs<3> R;
   load_chunk_rs(R, L[0].w_d_m + (long long)c * nT * 32, L[0].w_d_e + (long long)c * nT * 16, nT);
-  for (int s = 0; s < p.steps; ++s) {
+  for (int s = p.step0; s < p.steps; ++s) {
     const rsrc_t r1 = rsrc(p.t_h1 + (s & 1) * D), rmlp = rsrc(p.t_mlp + (s & 1) * p.FFN);
     const rsrc_t rh = rsrc(p.t_h + (s & 1) * D);
     for (int l = 0; l < p.NL; ++l) {
@@ -657,7 +657,7 @@ __device__ void role_d(const PT_CONST PersistArgs *pp, double *dsm, int c) {
 __device__ void role_head_only(const PT_CONST PersistArgs *pp, double *dsm) {
   PT_ENTER();
   (void)L;
-  for (int s = 0; s < p.steps; ++s) (void)end_of_step(p, s, dsm, w);
+  for (int s = p.step0; s < p.steps; ++s) (void)end_of_step(p, s, dsm, w);
 }
 
 // gp: the argument block in device memory (a global address, so it can be

@@ -1,0 +1,44 @@
+// The prompt of a decode as one pass over all its positions
+// (bfp_prefill.hip), instead of one step per position.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "bfp_layer.h"
+
+namespace bfp {
+
+// A pass over positions p0 .. p0 + n - 1 of `batch` sequences: row b*n + j
+// is position p0 + j of sequence b.  L holds one layer's weights, KV cache
+// and the row activations (L.batch = batch * n rows).
+struct PrefillArgs {
+  LayerArgs L;
+  int batch, n, p0;
+  const int *prompt;        // (batch, n_prompt) token ids, device
+  int n_prompt, VOCAB;
+  const float *embed;       // (VOCAB, D) float32
+  double *qf;               // (rows, D) rotated q as float64
+  int16_t *hist_m;          // optional: every layer's output, (batch, hist_steps, NL, D)
+  int8_t *hist_e;
+  int hist_steps;
+};
+
+// Most rows of one pass.
+constexpr int PF_ROWS = 1024;
+// Fewest positions a pass is made for, against the persistent batch-1 decode
+// and against a batch's steps.  Measured at SmolLM2's 30 layers, prompt part
+// of a decode, pass against steps: batch 1, 3 positions ~2.0 / 1.59 ms, 4
+// 1.99 / 2.10, 8 2.02 / 4.17; 2 positions at batch 2 1.72 / 1.82, batch 5
+// 1.76 / 3.17, batch 64 2.51 / 2.94.  (A pass of few rows is 8 launches a
+// layer, 66 us, whatever their number.)
+constexpr int PF_MIN_PERSIST = 4;
+constexpr int PF_MIN = 2;
+
+// Embedding rows of the pass's tokens into L.h_m / L.h_e.
+int launch_prefill_embed(const PrefillArgs &a, hipStream_t s);
+// One layer over the pass's rows: h in, h out, the cache rows written.
+int launch_prefill_layer(const PrefillArgs &a, hipStream_t s);
+// Raise the kernels' dynamic-LDS limits (outside any stream capture).
+int prepare_prefill_kernels();
+
+}  // namespace bfp
