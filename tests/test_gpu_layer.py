@@ -138,3 +138,37 @@ def test_second_context_keeps_lds_limit(gpu):
     assert (sim.tile_decode(om_[0].reshape(-1, 16), oe_[0]) == want).all()
     small.close()
     big.close()
+
+
+@pytest.mark.parametrize("spread", [6, 46, 50, 120])
+def test_batched_matvecs_exponent_spreads(gpu, spread):
+    """The matrix-core matvecs of a batch (float64 floor accumulation, with
+    and without the 47-bit window's test) against the batch-1 kernels'
+    64-bit shifts: full-range mantissas (sums to 2^34, -32768 among them),
+    weight exponents spread below, across and beyond the window, zero tiles."""
+    from bfp import Dims
+    from bfp.model import BfpModel
+    d = Dims(D=192, H_Q=3, H_KV=1, HD=64, FFN=272, NL=1, MAX_CTX=8, VOCAB=256)
+    B = 19   # a full group of 16 and a ragged one
+    rng = np.random.default_rng(spread)
+    gm = BfpModel(d, max_batch=B)
+    for name, (r, c) in {"Wq": (d.D, d.D), "Wk": (d.KV, d.D), "Wv": (d.KV, d.D), "Wo": (d.D, d.D),
+                         "Wg": (d.FFN, d.D), "Wu": (d.FFN, d.D), "Wd": (d.D, d.FFN)}.items():
+        m = rng.integers(-32768, 32768, size=(r, c // 16, 16)).astype(np.int16)
+        m[rng.random((r, c // 16)) < 0.05] = -32768
+        e = rng.integers(-spread // 2, spread - spread // 2 + 1, size=(r, c // 16)).astype(np.int8)
+        zero = rng.random((r, c // 16)) < 0.02
+        m[zero], e[zero] = 0, -127
+        gm.load_tensor(name, 0, m=m, e=e)
+    for name in ("g1", "g2"):
+        gm.load_tensor(name, 0, fp32=(1 + 0.1 * rng.standard_normal(d.D)).astype(np.float32))
+    hm = rng.integers(-32768, 32768, size=(B, d.D)).astype(np.int16)
+    he = rng.integers(-3, 4, size=(B, d.D // 16)).astype(np.int8)
+    om, oe, st = gm.layer_step_bfp(0, 0, hm, he, dump=True)
+    for b in range(B):
+        wm, we, ws = gm.layer_step_bfp(0, 0, hm[b], he[b], dump=True)
+        for name in st:
+            assert np.array_equal(st[name][0][b], ws[name][0][0]), (b, name)
+            assert np.array_equal(st[name][1][b], ws[name][1][0]), (b, name)
+        assert np.array_equal(om[b], wm[0]) and np.array_equal(oe[b], we[0])
+    gm.close()

@@ -87,3 +87,59 @@ def test_select_free_doubled_form():
         assert abs(hh) < 2 ** 20 and abs(cr) < 2 ** 22 and abs(ll) < 2 ** 20 and abs(lo) < 2 ** 31
         for d in (0, 1, 5, 16, 17, 33, 47):
             assert (2 * S) >> (d + 1) == S >> d
+
+
+def test_negated_operand_form():
+    """The per-stage kernels' form: the weight operand [Wh, Wl'] against
+    [xh, 0], [~xl', ~xh] + [-127, 1] and [0, ~xl'] + [0, -127] gives S with
+    128 sum x, each accumulator and the low part in int32."""
+    rng = np.random.default_rng(2)
+    ext = [-32768, -32767, -256, -129, -128, -1, 0, 1, 127, 128, 255, 256, 32767]
+    cases = [(rng.integers(-32768, 32768, 16), rng.integers(-32768, 32768, 16)) for _ in range(2000)]
+    cases += [(np.full(16, a), np.full(16, b)) for a in ext for b in ext]
+    cases += [(rng.choice(ext, 16), rng.choice(ext, 16)) for _ in range(1000)]
+    z, one = np.zeros(16, int), np.ones(16, int)
+    for W, x in cases:
+        Wh, Wl = _split(W)
+        xh, xl = _split(x)
+        A = np.concatenate([Wh, Wl])
+        cat = lambda a, b: np.concatenate([a, b])   # noqa: E731
+        hh = _mfma32(A, cat(xh, z))
+        cr = _mfma32(A, cat(-127 * one, one)) + _mfma32(A, cat(~np.asarray(xl), ~np.asarray(xh)))
+        ll = _mfma32(A, cat(z, -127 * one)) - 128 * int(np.sum(x)) + _mfma32(A, cat(z, ~np.asarray(xl)))
+        lo = (cr << 8) + ll
+        S = int((np.asarray(W, np.int64) * np.asarray(x, np.int64)).sum())
+        assert 65536 * hh - lo == S
+        assert abs(hh) <= 2 ** 18 and abs(cr) < 2 ** 20 and abs(ll) < 2 ** 27 and abs(lo) < 2 ** 29
+
+
+def test_floor_accumulation_in_float64():
+    """acc = fma(S, 2^E, acc) rounded toward minus infinity from acc = C =
+    1.5 * 2^(52 + M) adds 2^M floor(S 2^(E - M)): the bits of acc less C's are
+    the engine's sum.  The rounding is emulated with exact rationals."""
+    from fractions import Fraction
+    import struct
+    rng = np.random.default_rng(3)
+
+    def fma_down(s, scale, acc):
+        v = Fraction(s) * Fraction(scale) + Fraction(acc)
+        f = float(v)                      # nearest
+        if Fraction(f) > v:
+            f = np.nextafter(f, -np.inf)
+        return float(f)
+
+    def bits(f):
+        return struct.unpack("<q", struct.pack("<d", f))[0]
+
+    for M in (-254, -3, 0, 17, 254):
+        C = 1.5 * 2.0 ** 52 * 2.0 ** M
+        for _ in range(60):
+            d = rng.integers(0, 48, size=96)
+            d[rng.integers(96)] = 0
+            S = rng.integers(-2 ** 34, 2 ** 34 + 1, size=96)
+            S[:4] = (-2 ** 34, 2 ** 34, -1, 1)
+            acc = C
+            for s, k in zip(S, d):
+                acc = fma_down(int(s), 2.0 ** int(M - k), acc)
+            want = sum(int(s) >> int(k) for s, k in zip(S, d))
+            assert bits(acc) - bits(C) == want

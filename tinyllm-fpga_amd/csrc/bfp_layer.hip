@@ -432,7 +432,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES, (PPW == 3 ? 6 : 4)) void k_qkv_attn
   const int nT = a.D / 16, bq = nq / 16, c = blockIdx.x % bq, b0 = blockIdx.x / bq * MX_SEQ;
   const int ns = min(MX_SEQ, a.batch - b0);
   int8_t *mx_ex = reinterpret_cast<int8_t *>(dsm);
-  long long *Ao = reinterpret_cast<long long *>(mx_ex + mx_lds_bytes(1, nT));   // 32 nT bytes
+  long long *Ao = reinterpret_cast<long long *>(mx_ex + mx_lds_bytes(1, nT));   // 96 nT bytes
   int *Mo = reinterpret_cast<int *>(Ao + 16 * MX_SEQ);
   mx_block<1>(a.w_qkv_m + (long long)c * nT * 32, a.w_qkv_e + (long long)c * nT * 16, nT,
               a.xn_m + (long long)b0 * a.D, a.xn_e + (long long)b0 * nT, ns, Ao, Mo, mx_ex, mx_tr<TR>(a, MX_K_QKV));
@@ -506,7 +506,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES, 2) void k_qkv_attng_mx(LayerArgs a,
   const int nT = a.D / 16, bq = nq / 16, c = blockIdx.x % bq, b0 = blockIdx.x / bq * MX_SEQ;
   const int ns = min(MX_SEQ, a.batch - b0);
   int8_t *mx_ex = reinterpret_cast<int8_t *>(dsm);
-  long long *Ao = reinterpret_cast<long long *>(mx_ex + mx_lds_bytes(1, nT));   // 32 nT bytes
+  long long *Ao = reinterpret_cast<long long *>(mx_ex + mx_lds_bytes(1, nT));   // 96 nT bytes
   int *Mo = reinterpret_cast<int *>(Ao + 16 * MX_SEQ);
   mx_block<1>(a.w_qkv_m + (long long)c * nT * 32, a.w_qkv_e + (long long)c * nT * 16, nT,
               a.xn_m + (long long)b0 * a.D, a.xn_e + (long long)b0 * nT, ns, Ao, Mo, mx_ex, mx_tr<TR>(a, MX_K_QKV));

@@ -10,20 +10,37 @@
 // both in [-128, 127].  Over one 16-element tile
 //   S = 65536*Phh + 256*(Phl + Plh + 128*sum Wh) + (Pll + 128*sum Wl')
 //       + 128*sum x
-// where Pab = sum_k Wa*xb.  Every product sum is one v_mfma_i32_16x16x32_i8
+// where Pab = sum_k Wa*xb.  Every product sum is one v_mfma_i32_16x16x32_i8,
 // whose 32-deep k axis holds the tile twice (k-groups 0-1 and 2-3 of the
-// operand layout): Phh and Pll with the second copy of A zeroed, the cross
-// term as Wh.xl' over the first copy plus Wl'.xh over the second, and the
-// weight sums against a constant 64 operand over both copies (= 128 sum).
-// 128 sum x (one value per sequence, from the vector unit) is the initial
-// accumulator of the low-byte product sum.  |Phh| <= 2^18
-// and the rest fits in 29 bits, so S is formed exactly in 64 bits.  E =
-// W_e + x_e of the lane's four output rows comes from one LDS word (the four
-// rows' weight exponents, tile-major) and one byte, so every per-output
-// quantity is in the lane that owns the output: no lane exchange is needed.
-// (E through one more MFMA per tile and chunk, A = [W_e, 1], B = [1, x_e],
-// made the max-exponent pass a chain of dependent LDS reads and MFMAs: 1.9
-// against 1.0 us for the 576 x 3072 G/U block of 16 sequences.)
+// operand layout).  The weight operand of all of them is A = [Wh, Wl'] (first
+// copy high bytes, second low bytes); the input operand chooses the terms:
+//   Phh            A . [xh, 0]
+//   -(Phl + Plh + 128 sum Wh)   A . [~xl', ~xh] + A . [-127, 1]
+//   -(Pll + 128 sum Wl')        A . [0, ~xl'] + A . [0, -127]
+// with ~v = -v - 1, which stays in a signed byte: A . [~xl', ~xh] = -(Phl +
+// Plh) - sum Wh - sum Wl', so the constant operand adds -127 sum Wh + sum
+// Wl'; likewise for the low bytes.  The two constant products start the
+// accumulators, the low one from -128 sum x (one value per sequence, from
+// the vector unit).  |Phh| <= 2^18 and the rest fits in 29 bits.
+//
+// The aligned sum A is formed in float64 with the rounding mode toward minus
+// infinity: an accumulator starting at C = 1.5 * 2^(52 + M) has 2^M as the
+// unit of its last place, so fma(S, 2^E, acc) is acc + 2^M floor(S 2^(E - M))
+// exactly -- one instruction for the shift, the floor and the 64-bit add --
+// and A is the difference of the bit patterns of acc and C (|A| <= nT 2^34
+// < 2^51, so acc keeps its binade).  S itself is exact in float64 (35 bits:
+// fma(Phh, 65536, low part)), and 2^E is built from its exponent field: the
+// weights' exponents lie in LDS as 16-bit pairs and the inputs' as a pair of
+// one value, biased, so the largest and smallest E of pass 1 are formed two
+// rows an instruction and 2^E is one shift-add.  A wave that has a tile with
+// M - E > 47 (dropped by the engine) forms its sums with 2^E replaced by 0
+// there; without one it skips the test.
+//
+// Against a 64-bit shift and add per output and operand sets selected per
+// copy of the tile, the G/U launch of 64 sequences went from 13.4 to 12.2 us
+// (its tile sums from 5.5 to 4.2), Q|K|V 12.6 to 12.4, O 10.3 to 10.1, D 13.5
+// to 13.8.  (The input sums by three more products a tile instead of the
+// vector unit: G/U 15.9 us, its registers no longer fitting one round.)
 //
 // A block is NC adjacent 16-row chunks of the device layout by 16
 // sequences.  Lane l supplies row / sequence l % 16 and k-group l / 16
@@ -54,12 +71,6 @@ __device__ __forceinline__ void mx_split(const uint4 w, long &hi, long &lo) {
   const unsigned l1 = __builtin_amdgcn_perm(w.w, w.z, 0x06040200u) ^ 0x80808080u;
   hi = (long)(((unsigned long)h1 << 32) | h0);
   lo = (long)(((unsigned long)l1 << 32) | l0);
-}
-
-__device__ __forceinline__ int mx_sum8(const uint4 w) {
-  return (int)(short)(w.x & 0xffffu) + ((int)w.x >> 16) + (int)(short)(w.y & 0xffffu) +
-         ((int)w.y >> 16) + (int)(short)(w.z & 0xffffu) + ((int)w.z >> 16) +
-         (int)(short)(w.w & 0xffffu) + ((int)w.w >> 16);
 }
 
 __device__ __forceinline__ mx_v4 mx_mfma(long a, long b, mx_v4 c) {
@@ -109,11 +120,6 @@ __device__ __forceinline__ long long mx_align2(int hh, int lo, int q) {
   return q <= ALIGN_MAX + 1 ? t : 0;
 }
 
-// (The per-stage launches keep the form above with the second copy zeroed:
-// there the blocks are bound by the matrix cores, and the select-free form's
-// eight products a tile instead of five made G/U 5.5 -> 6.7 us and D
-// 4.0 -> 5.3 us of tile sums at batch 64.)
-
 // Phase stamps of a traced batched decode (100 MHz clock, thread 0 of each
 // block): MX_TRACE_STAMPS per block -- 0 entry, 1 exponents staged, 2 M
 // reduced, 3 tile sums formed, 4 A reduced, 5 epilogue done (stamped by the
@@ -129,8 +135,26 @@ __device__ __forceinline__ void mx_mark(unsigned long long *tr, int k) {
 }
 
 // LDS bytes mx_block<NC> needs beyond its caller's Ao / Mo: the block's
-// weight and input exponents, tile-major.
-__host__ __device__ constexpr int mx_lds_bytes(int nc, int nT) { return (nc + 1) * 16 * nT; }
+// weight exponents as 16-bit values, tile-major, and the input exponents as
+// pairs of one 16-bit value.
+__host__ __device__ constexpr int mx_lds_bytes(int nc, int nT) { return (nc * 32 + 64) * nT; }
+
+typedef short mx_s2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ mx_s2 mx_pair(int v) { return __builtin_bit_cast(mx_s2, v); }
+__device__ __forceinline__ int mx_bits(mx_s2 v) { return __builtin_bit_cast(int, v); }
+
+// The float64 rounding mode of the wave: toward minus infinity, or nearest.
+__device__ __forceinline__ void mx_round_down() {
+  asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 2\n\ts_nop 1");
+}
+__device__ __forceinline__ void mx_round_nearest() {
+  asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 0\n\ts_nop 1");
+}
+// acc = s * scale + acc under the mode set by mx_round_down (volatile: not
+// moved across the mode changes).
+__device__ __forceinline__ void mx_fma_down(double &acc, double s, double scale) {
+  asm volatile("v_fma_f64 %0, %1, %2, %0" : "+v"(acc) : "v"(s), "v"(scale));
+}
 
 // (A, M) of the (row, sequence) pairs of a block: the NC adjacent 16-row
 // chunks at pm / pe (device layout, nT tiles each; chunk c is rows
@@ -145,13 +169,15 @@ __device__ __forceinline__ void mx_block(const uint4 *__restrict__ pm, const int
   mx_mark(tr, 0);
   constexpr int G = 4;           // tiles whose loads are in flight together
   constexpr int RW = NC * 16;    // rows of the block
+  constexpr int EB = 128;        // bias of a stored exponent
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const int i = lane & 15, kg = lane >> 4, h = kg & 1;
   const bool first = kg < 2;     // first copy of the tile on the k axis
   const int sc = i < ns ? i : ns - 1;
   const uint4 *xr = reinterpret_cast<const uint4 *>(xm);
   const int wo = h * 16 + i, xo = sc * nT * 2 + h;   // + t*32 (+ c*nT*32), + t*2
-  int8_t *wex = ex, *xex = ex + RW * nT;             // [t*RW + row], [t*16 + sequence]
+  int16_t *wex = reinterpret_cast<int16_t *>(ex);    // [t*RW + row]
+  int *xex = reinterpret_cast<int *>(wex + RW * nT); // [t*16 + sequence]
   const int tpw = (nT + nw - 1) / nw;
   const int t0 = w * tpw, t1 = t0 + tpw < nT ? t0 + tpw : nT;
   // operand registers of G tiles, loaded together (the last valid tile
@@ -168,8 +194,9 @@ __device__ __forceinline__ void mx_block(const uint4 *__restrict__ pm, const int
       for (int c = 0; c < NC; ++c) wv[k][c] = pm[wo + c * nT * 32 + t * 32];
     }
   };
-  // exponents of the whole block into LDS: the weights' as 4-row words, the
-  // inputs' as bytes, every load of a thread issued before its stores
+  // exponents of the whole block into LDS, biased: the weights' as 4-row
+  // words of 16-bit values, the inputs' as pairs, every load of a thread
+  // issued before its stores
   {
     const int nw4 = NC * nT * 4, nx = MX_SEQ * nT, bs = blockDim.x;
     const int *pe4 = reinterpret_cast<const int *>(pe);
@@ -191,11 +218,14 @@ __device__ __forceinline__ void mx_block(const uint4 *__restrict__ pm, const int
       for (int k = 0; k < 4; ++k) {
         const int q = q0 + k * bs;
         if (q < nw4) {
-          // word q: chunk q / (4nT), tile (q / 4) % nT, rows 4*(q%4) .. +3
+          // word q: chunk q / (4nT), tile (q / 4) % nT, rows 4*(q%4) .. +3;
+          // a signed byte plus 128 is the byte with its sign bit flipped
           const int c = q / (4 * nT), t = (q >> 2) - c * nT;
-          *reinterpret_cast<int *>(wex + t * RW + c * 16 + 4 * (q & 3)) = v[k];
+          const unsigned u = (unsigned)v[k] ^ 0x80808080u;
+          *reinterpret_cast<int2 *>(wex + t * RW + c * 16 + 4 * (q & 3)) =
+              make_int2((int)__builtin_amdgcn_perm(0, u, 0x0c010c00u), (int)__builtin_amdgcn_perm(0, u, 0x0c030c02u));
         } else if (q < nw4 + nx) {
-          xex[q - nw4] = (int8_t)v[k];
+          xex[q - nw4] = (v[k] + EB) * 0x10001;
         }
       }
     }
@@ -206,87 +236,127 @@ __device__ __forceinline__ void mx_block(const uint4 *__restrict__ pm, const int
   }
   __syncthreads();
   mx_mark(tr, 1);
-  const mx_v4 zero = {0, 0, 0, 0};
-  // E = W_e + x_e of chunk c, tile t for this lane's outputs (rows 4 kg + v,
-  // sequence i): the four rows' exponents are one 4-byte word of wex
-  auto tile_E = [&](int c, int t, int (&E)[4]) {
-    const int ww = *reinterpret_cast<const int *>(wex + t * RW + c * 16 + 4 * kg);
-    const int xv = xex[t * 16 + i];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) E[v] = ((ww << (24 - 8 * v)) >> 24) + xv;
+  // (W_e + x_e, biased by 2 EB) of chunk c, tile t for this lane's outputs
+  // (rows 4 kg + v, sequence i), two rows a pair
+  auto tile_E = [&](int c, int t, mx_s2 (&E)[2]) {
+    const int2 ww = *reinterpret_cast<const int2 *>(wex + t * RW + c * 16 + 4 * kg);
+    const mx_s2 xp = mx_pair(xex[t * 16 + i]);
+    E[0] = mx_pair(ww.x) + xp;
+    E[1] = mx_pair(ww.y) + xp;
   };
-  // pass 1: M over all tiles, split across the waves, reduced in LDS
+  // pass 1: M over all tiles, split across the waves, reduced in LDS; and
+  // the smallest E of this wave's tiles
   int M[NC][4];
+  mx_s2 Emin[NC][2];
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) M[c][v] = -(1 << 29);
+    mx_s2 mx[2];
+    mx[0] = mx[1] = mx_s2{0, 0};
+    Emin[c][0] = Emin[c][1] = mx_s2{1024, 1024};
 #pragma unroll 4
     for (int t = t0; t < t1; ++t) {
-      int E[4];
+      mx_s2 E[2];
       tile_E(c, t, E);
 #pragma unroll
-      for (int v = 0; v < 4; ++v) M[c][v] = E[v] > M[c][v] ? E[v] : M[c][v];
+      for (int p = 0; p < 2; ++p) {
+        mx[p] = __builtin_elementwise_max(mx[p], E[p]);
+        Emin[c][p] = __builtin_elementwise_min(Emin[c][p], E[p]);
+      }
     }
     if (t0 < t1) {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) atomicMax(&Mo[(c * 16 + 4 * kg + v) * MX_SEQ + i], M[c][v]);
+      for (int v = 0; v < 4; ++v) atomicMax(&Mo[(c * 16 + 4 * kg + v) * MX_SEQ + i], (int)mx[v >> 1][v & 1] - 2 * EB);
     }
   }
   __syncthreads();
   mx_mark(tr, 2);
+  // accumulators at C = 1.5 * 2^(52 + M)
+  double A[NC][4];
+  bool far = false;   // a tile past the engine's 47-bit window
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) M[c][v] = Mo[(c * 16 + 4 * kg + v) * MX_SEQ + i];
-  // pass 2: aligned tile sums
-  long long A[NC][4];
+    for (int v = 0; v < 4; ++v) {
+      M[c][v] = Mo[(c * 16 + 4 * kg + v) * MX_SEQ + i];
+      A[c][v] = __hiloint2double(((1075 + M[c][v]) << 20) | 0x80000, 0);
+      far = far || M[c][v] + 2 * EB - (int)Emin[c][v >> 1][v & 1] > ALIGN_MAX;
+    }
+  // pass 2: aligned tile sums.  Byte selectors of v_perm_b32 over (second
+  // dword, first dword) of 4 int16: high bytes, low bytes, zeros
+  const unsigned HI = 0x07050301u, LO = 0x06040200u, ZR = 0x0c0c0c0cu;
+  const unsigned sA = first ? HI : LO, mA = first ? 0u : 0x80808080u;       // [Wh, Wl']
+  const unsigned sH = first ? HI : ZR;                                      // [xh, 0]
+  const unsigned sC = first ? LO : HI, mC = first ? 0x7f7f7f7fu : ~0u;      // [~xl', ~xh]
+  const unsigned sL = first ? ZR : LO, mL = first ? 0u : 0x7f7f7f7fu;       // [0, ~xl']
+  auto planes = [](const uint4 &v, unsigned sel, unsigned mask) {
+    const unsigned lo = __builtin_amdgcn_perm(v.y, v.x, sel) ^ mask, hi = __builtin_amdgcn_perm(v.w, v.z, sel) ^ mask;
+    return (long)(((unsigned long)hi << 32) | lo);
+  };
+  const long kC = first ? (long)0x8181818181818181ull : 0x0101010101010101L;   // [-127, 1]
+  const long kL = first ? 0L : (long)0x8181818181818181ull;                    // [0, -127]
+  const mx_v4 zero = {0, 0, 0, 0};
+  auto tiles = [&](auto window) {
+    constexpr bool WIN = decltype(window)::value;
+    for (int tb = t0; tb < t1; tb += G) {
+      load_group(tb);
 #pragma unroll
-  for (int c = 0; c < NC; ++c)
+      for (int k = 0; k < G; ++k) {
+        if (tb + k >= t1) break;
+        const long xh = planes(xv[k], sH, 0u), xc = planes(xv[k], sC, mC), xl = planes(xv[k], sL, mL);
+        // -128 sum x: this half's, then the tile's other half (k-group kg ^ 1)
+        int sx = 0;
+        const mx_s2 m128 = {-128, -128};
+        sx = __builtin_amdgcn_sdot2(mx_pair((int)xv[k].x), m128, sx, false);
+        sx = __builtin_amdgcn_sdot2(mx_pair((int)xv[k].y), m128, sx, false);
+        sx = __builtin_amdgcn_sdot2(mx_pair((int)xv[k].z), m128, sx, false);
+        sx = __builtin_amdgcn_sdot2(mx_pair((int)xv[k].w), m128, sx, false);
+        const auto sw = __builtin_amdgcn_permlane16_swap(sx, sx, false, false);
+        const int cx = (int)(sw[0] + sw[1]);
+        const mx_v4 cxv = {cx, cx, cx, cx};
+        const int xp = xex[(tb + k) * 16 + i];
+        // high word of 2^E is (1023 - 2 EB + W_e' + x_e') << 20 (a pair shifted
+        // left by 20 keeps its low value)
+        const int xs = (xp << 20) + ((1023 - 2 * EB) << 20);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) A[c][v] = 0;
-  const long k64 = 0x4040404040404040L;
-  for (int tb = t0; tb < t1; tb += G) {
-    load_group(tb);
+        for (int c = 0; c < NC; ++c) {
+          const long wa = planes(wv[k][c], sA, mA);
+          mx_v4 cr = mx_mfma(wa, kC, zero);
+          mx_v4 ll = mx_mfma(wa, kL, cxv);
+          const mx_v4 hh = mx_mfma(wa, xh, zero);
+          cr = mx_mfma(wa, xc, cr);
+          ll = mx_mfma(wa, xl, ll);
+          const int2 ww = *reinterpret_cast<const int2 *>(wex + (tb + k) * RW + c * 16 + 4 * kg);
 #pragma unroll
-    for (int k = 0; k < G; ++k) {
-      if (tb + k >= t1) break;
-      long xh, xl;
-      mx_split(xv[k], xh, xl);
-      int sx = mx_sum8(xv[k]);
-      sx += peer<16>(sx);   // the tile's other half (k-group l/16 ^ 1)
-      const int cx = 128 * sx;
-      // 128 sum x, one value per sequence, starts the low-byte product sum
-      const mx_v4 cxv = {cx, cx, cx, cx};
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        long wh, wl;
-        mx_split(wv[k][c], wh, wl);
-        const mx_v4 hh = mx_mfma(first ? wh : 0, xh, zero);
-        mx_v4 ll = mx_mfma(first ? wl : 0, xl, cxv);
-        mx_v4 cr = mx_mfma(first ? wh : wl, first ? xl : xh, zero);
-        cr = mx_mfma(wh, k64, cr);
-        ll = mx_mfma(wl, k64, ll);
-        int E[4];
-        tile_E(c, tb + k, E);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int d = M[c][v] - E[v];
-          const int lo = (cr[v] << 8) + ll[v];
-          const long long S = ((long long)hh[v] << 16) + lo;
-          if (d <= ALIGN_MAX) A[c][v] += S >> d;
+          for (int v = 0; v < 4; ++v) {
+            const int wp = v < 2 ? ww.x : ww.y;
+            int se = (v & 1) ? (int)((unsigned)wp >> 16 << 20) + xs : (wp << 20) + xs;
+            if constexpr (WIN) {
+              const int E = (int)((unsigned)se >> 20) - 1023;
+              se = M[c][v] - E > ALIGN_MAX ? 0 : se;
+            }
+            const int lo = (cr[v] << 8) + ll[v];   // - (low part of S)
+            const double S = fma((double)hh[v], 65536.0, -(double)lo);
+            mx_fma_down(A[c][v], S, __hiloint2double(se, 0));
+          }
         }
       }
     }
-  }
+  };
+  mx_round_down();
+  if (__builtin_expect(__any(far), 0)) tiles(std::true_type{});
+  else tiles(std::false_type{});
+  mx_round_nearest();
   mx_mark(tr, 3);
   if (t0 < t1) {
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
-      for (int v = 0; v < 4; ++v)
+      for (int v = 0; v < 4; ++v) {
+        const long long a = __double_as_longlong(A[c][v]) -
+                            ((long long)(((1075 + M[c][v]) << 20) | 0x80000) << 32);
         atomicAdd(reinterpret_cast<unsigned long long *>(&Ao[(c * 16 + 4 * kg + v) * MX_SEQ + i]),
-                  (unsigned long long)A[c][v]);
+                  (unsigned long long)a);
+      }
   }
   __syncthreads();
   mx_mark(tr, 4);
