@@ -138,3 +138,36 @@ def test_argmax(gpu):
     for b in range(2):
         assert got[b] == ort.rtl_argmax(m[b], e[b])
     assert rtl.argmax(np.full(64, 7, np.int16), np.zeros(64, np.int8))[0] == 0
+
+
+@pytest.mark.parametrize("n", [16, 48, 16 * 64, 16 * 65, 16 * 1025])
+def test_argmax_replacement_order(gpu, n):
+    """The chunk fold by blocks of 64: every chunk a replacement (rising
+    logits), none (falling), and values that truncation makes incomparable."""
+    from bfp import rtl
+    rng = np.random.default_rng(n)
+    up = np.linspace(-30000, 30000, n).astype(np.int16)
+    e0 = np.zeros(n, np.int8)
+    near = rng.integers(16380, 16388, n).astype(np.int16), rng.integers(0, 3, n).astype(np.int8)
+    low = np.full(n, -32768, np.int16), np.full(n, -128, np.int8)    # nothing beats the seed
+    for m, e in ((up, e0), (up[::-1].copy(), e0), near, low):
+        assert rtl.argmax(m[None], e[None])[0] == ort.rtl_argmax(m, e)
+
+
+@pytest.mark.parametrize("D", [16, 80, 576, 1024, 1040, 1728])
+def test_rmsnorm_exponent_rises(gpu, D):
+    """The norm's fold over 1 to 64 tiles by a wave's scan, and past 64 tiles
+    in order, with exponents that rise and fall by up to 60."""
+    from bfp import rtl
+    rng = np.random.default_rng(D)
+    for order in ("random", "rising", "falling"):
+        xe = rng.integers(-30, 31, D // 16)
+        xe = xe if order == "random" else np.sort(xe)[:: 1 if order == "rising" else -1]
+        xm = rng.integers(-32768, 32768, D).astype(np.int16)
+        gm = rng.integers(8000, 24000, D).astype(np.int16)
+        ge = rng.integers(0, 3, D // 16).astype(np.int8)
+        xe = np.ascontiguousarray(xe).astype(np.int8)
+        got = rtl.golden_rmsnorm(xm, xe, gm, ge)
+        want = ort.rtl_rmsnorm(xm, xe, gm, ge)
+        for a, b in zip(got, want):
+            assert np.array_equal(np.asarray(a).reshape(-1), np.asarray(b).reshape(-1)), order

@@ -106,7 +106,7 @@ struct RtlHeadArgs {
   int16_t *xn_m; int8_t *xn_e;               // normed hidden
   const uint4 *emb_m; const int8_t *emb_e;   // tile-quantised tied embedding, device layout
   int16_t *lg_m; int8_t *lg_e;               // per-row logits (VOCAB of each)
-  int *work;                                 // 3 * VOCAB / 16 ints
+  int *work;                                 // VOCAB / 16 words: each chunk's best
   int *token;                                // argmax out (device)
 };
 

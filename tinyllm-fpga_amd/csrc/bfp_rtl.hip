@@ -38,11 +38,10 @@ __device__ __forceinline__ int norm16(long long v, int lead, int &shift) {
 __device__ __forceinline__ int clamp8(int e) { return e < -128 ? -128 : (e > 127 ? 127 : e); }
 
 __device__ __forceinline__ int max16_lanes(int v) {
-  for (int o = 1; o < 16; o <<= 1) {
-    int w = __shfl_xor(v, o, 64);
-    v = w > v ? w : v;
-  }
-  return v;
+  v = pmax<8>(v);
+  v = pmax<4>(v);
+  v = pmax<2>(v);
+  return pmax<1>(v);
 }
 
 // ------------------------------------------------------------------ matvec
@@ -109,92 +108,180 @@ __constant__ int c_rms_seed[32] = {
     428079, 302698, 214040, 151349, 107020, 75674, 53510, 37837,
     26755, 18919, 13377, 9459, 6689, 4730, 3344, 2365};
 
-// One 64-thread wave normalises the D-vector x: writes ym (D) and ye (D/16).
-// sums: D/16 int64 of LDS; s_inv / s_einv: LDS scalars.
-__device__ void rmsnorm_wave(const int16_t *__restrict__ x, const int8_t *__restrict__ xex,
-                             const int16_t *gm, const int8_t *ge, int D, int16_t *ym, int8_t *ye,
-                             long long *sums, long long *s_inv, int *s_einv) {
-  const int tid = threadIdx.x, nt = D / 16;
-  for (int t = tid; t < nt; t += 64) {
-    long long s = 0;
-    for (int k = 0; k < 16; ++k) s += (long long)x[t * 16 + k] * x[t * 16 + k];
-    sums[t] = s;
+// One step of the engine's ordered fold over tiles (gen_matvec_bfp_golden.py
+// :53-108): the side with the smaller exponent is shifted right (zeroed past
+// 47), then added.  The engine's 48-bit saturation cannot be reached: a tile
+// sum is at most 2^34, so fewer than 2^13 of them stay below 2^47 (the
+// callers have at most 4096 tiles).  acc_e is the running maximum of the
+// exponents whatever the sums are, so the shift amounts do not wait for acc
+// and only a shift and an add chain from step to step.
+__device__ __forceinline__ void tile_fold(long long &acc, int &acc_e, long long s, int te) {
+  const int d = te - acc_e;
+  const int up = d > 0 ? d : 0, dn = d < 0 ? -d : 0;
+  const long long s2 = dn > ACC_W - 1 ? 0 : (s >> dn);
+  acc = (up > ACC_W - 1 ? 0 : (acc >> up)) + s2;
+  acc_e = d > 0 ? te : acc_e;
+}
+
+// The same fold over nt <= 64 tiles (LDS) by a wave, tile t in lane t: the
+// running maximum of the exponents is a scan, each sum's shift follows from
+// it, and the sums between two rises of the maximum add in any order; acc is
+// shifted once a rise (a few for 36 tiles).  Every lane returns the result.
+__device__ __forceinline__ void fold_wave(const long long *S, const int *E, int nt, long long &acc, int &acc_e) {
+  const int l = threadIdx.x & 63, lc = l < nt ? l : nt - 1;
+  constexpr int NONE = -100000;
+  const int e = l < nt ? E[lc] : NONE;
+  const long long sv = S[lc];
+  int p = e;
+  auto scan = [&](int o) { p = o > p ? o : p; };
+  scan(__builtin_amdgcn_update_dpp(NONE, p, 0x111, 0xf, 0xf, false));   // row_shr 1, 2, 4, 8
+  scan(__builtin_amdgcn_update_dpp(NONE, p, 0x112, 0xf, 0xf, false));
+  scan(__builtin_amdgcn_update_dpp(NONE, p, 0x114, 0xf, 0xf, false));
+  scan(__builtin_amdgcn_update_dpp(NONE, p, 0x118, 0xf, 0xf, false));
+  // the rows' maxima into the rows after them
+  const int r0 = __builtin_amdgcn_readlane(p, 15), r1 = __builtin_amdgcn_readlane(p, 31);
+  const int r2 = __builtin_amdgcn_readlane(p, 47);
+  const int r01 = r0 > r1 ? r0 : r1, r012 = r01 > r2 ? r01 : r2;
+  scan(l < 16 ? NONE : (l < 32 ? r0 : (l < 48 ? r01 : r012)));
+  int before = __shfl_up(p, 1, 64);
+  before = l == 0 ? e : before;
+  const int dn = p - e;
+  const long long s = l >= nt || dn > ACC_W - 1 ? 0 : (sv >> dn);
+  unsigned long long rises = __ballot(l < nt && e > before);
+  acc = 0;
+  for (int from = 0;;) {   // uniform
+    const int to = rises ? __builtin_ctzll(rises) : 64;
+    long long seg = l >= from && l < to ? s : 0;
+    seg = psum<8>(seg);
+    seg = psum<4>(seg);
+    seg = psum<2>(seg);
+    seg = psum<1>(seg);
+    seg = psum<16>(seg);
+    seg = psum<32>(seg);
+    acc += seg;
+    if (to == 64) break;
+    const int up = __builtin_amdgcn_readlane(e, to) - __builtin_amdgcn_readlane(before, to);
+    acc = up > ACC_W - 1 ? 0 : (acc >> up);
+    rises &= rises - 1;
+    from = to;
   }
-  __syncthreads();
-  if (tid == 0) {
-    long long acc = sums[0];
-    int acc_e = 2 * xex[0];
-    for (int t = 1; t < nt; ++t) {
-      const int te = 2 * xex[t];
-      const int d = te - acc_e;
-      if (d > 0) {
-        acc = d > ACC_W - 1 ? 0 : (acc >> d);
-        acc_e = te;
-        acc += sums[t];
-      } else if (d < 0) {
-        acc += (-d <= ACC_W - 1) ? (sums[t] >> (-d)) : 0;
-      } else {
-        acc += sums[t];
+  acc_e = __builtin_amdgcn_readlane(p, 63);
+}
+
+// The RMSNorm engine on the D-vector (x, xex) by a whole workgroup (any
+// multiple of 64 threads): gamma(i, m, e) gives gamma element i (called by
+// whole waves, 16-lane groups on one tile), out(i, m, e) takes the result
+// (i < D; lanes of a tile together).  sums: D/16 int64 of LDS, sexp: D/16
+// ints.  Thread tid keeps its first RMS_KE elements in registers from one
+// batch of loads.  Every thread folds the tile sums and runs the
+// Newton-Raphson steps itself (the same values in every lane), so one
+// barrier is enough.  (As one wave's chain of loads the norm of 576 elements
+// was a launch of 17 us; the head's, in this form, takes 6.)
+constexpr int RMS_KE = 3;
+template <class Gamma, class Out>
+__device__ __forceinline__ void rms_block(const int16_t *__restrict__ x, const int8_t *__restrict__ xex, Gamma gamma,
+                                          int D, long long *sums, int *sexp, Out out) {
+  const int tid = threadIdx.x, bs = blockDim.x, nt = D / 16;
+  int xv[RMS_KE], xe[RMS_KE], gm[RMS_KE], ge[RMS_KE];
+  auto load = [&](int base) {
+#pragma unroll
+    for (int k = 0; k < RMS_KE; ++k) {
+      const int i = base + tid + k * bs, ic = i < D ? i : D - 1;
+      xv[k] = x[ic];
+      xe[k] = xex[ic >> 4];
+    }
+#pragma unroll
+    for (int k = 0; k < RMS_KE; ++k) {
+      const int i = base + tid + k * bs;
+      gamma(i < D ? i : (D - 16) + (i & 15), gm[k], ge[k]);
+    }
+  };
+  for (int base = 0; base < D; base += RMS_KE * bs) {   // uniform
+    load(base);
+#pragma unroll
+    for (int k = 0; k < RMS_KE; ++k) {
+      const int i = base + tid + k * bs;
+      long long s = (long long)(xv[k] * xv[k]);   // at most 2^30
+      s = psum<1>(s);
+      s = psum<2>(s);
+      s = psum<4>(s);
+      s = psum<8>(s);
+      if (i < D && (i & 15) == 0) {
+        sums[i >> 4] = s;
+        sexp[i >> 4] = 2 * xe[k];
       }
     }
-    const unsigned long long inv_d = (1ULL << 32) / (unsigned)D;
-    // mean = (acc * inv_d) >> 32, acc >= 0
-    const unsigned __int128 prod = (unsigned __int128)(unsigned long long)acc * inv_d;
-    const unsigned long long mean = (unsigned long long)(prod >> 32);
-    int lead = mean ? 63 - __clzll(mean) : 0;
-    if ((acc_e + lead) & 1) lead -= 1;
-    long long v = lead >= 30 ? (long long)(mean >> (lead - 30))
-                             : (long long)(mean << (30 - lead));
-    v += 10737;                                       // EPS_Q30
-    const int vmsb = v ? 63 - __clzll((unsigned long long)v) : 0;
-    long long inv = vmsb < 32 ? c_rms_seed[vmsb] : 16777215;
-    const long long C = (3LL << 30) / 2;
-    for (int it = 0; it < 3; ++it) {
-      const __int128 vy2 = ((__int128)v * inv * inv) >> 24;
-      long long corr;
-      if (vy2 >= ((__int128)1 << 32)) {
-        corr = 0;
-      } else {
-        corr = C - ((long long)vy2 >> 1);
-        corr = corr < 0 ? 0 : corr;
-      }
-      long long ni = (inv * corr + (1LL << 29)) >> 30;
-      inv = ni < 16777215 ? ni : 16777215;
-    }
-    *s_inv = inv;
-    *s_einv = (30 - acc_e - lead) >> 1;
   }
-  __syncthreads();
-  const long long inv = *s_inv;
-  const int einv = *s_einv;
-  for (int base = 0; base < D; base += 64) {
-    const int i = base + tid;                         // D % 64 == 0 not required: D % 16 == 0
-    const bool ok = i < D;
-    const long long p = ok ? (long long)x[i] * gm[i] * inv : 0;
-    const int ml = max16_lanes(p ? lead64(p) : 0);
-    if (ok) {
+  lds_barrier();
+  long long acc;
+  int acc_e;
+  if (nt <= 64) {   // uniform
+    fold_wave(sums, sexp, nt, acc, acc_e);
+  } else {
+    acc = sums[0];
+    acc_e = sexp[0];
+#pragma unroll 4
+    for (int t = 1; t < nt; ++t) tile_fold(acc, acc_e, sums[t], sexp[t]);
+  }
+  const unsigned long long inv_d = (1ULL << 32) / (unsigned)D;
+  // mean = (acc * inv_d) >> 32, acc >= 0
+  const unsigned __int128 prod = (unsigned __int128)(unsigned long long)acc * inv_d;
+  const unsigned long long mean = (unsigned long long)(prod >> 32);
+  int lead = mean ? 63 - __clzll(mean) : 0;
+  if ((acc_e + lead) & 1) lead -= 1;
+  long long v = lead >= 30 ? (long long)(mean >> (lead - 30)) : (long long)(mean << (30 - lead));
+  v += 10737;                                       // EPS_Q30
+  const int vmsb = v ? 63 - __clzll((unsigned long long)v) : 0;
+  long long inv = vmsb < 32 ? c_rms_seed[vmsb] : 16777215;
+  const long long C = (3LL << 30) / 2;
+  for (int it = 0; it < 3; ++it) {
+    const __int128 vy2 = ((__int128)v * inv * inv) >> 24;
+    long long corr;
+    if (vy2 >= ((__int128)1 << 32)) {
+      corr = 0;
+    } else {
+      corr = C - ((long long)vy2 >> 1);
+      corr = corr < 0 ? 0 : corr;
+    }
+    const long long ni = (inv * corr + (1LL << 29)) >> 30;
+    inv = ni < 16777215 ? ni : 16777215;
+  }
+  const int einv = (30 - acc_e - lead) >> 1;
+  for (int base = 0; base < D; base += RMS_KE * bs) {   // uniform
+    if (D > RMS_KE * bs) load(base);
+#pragma unroll
+    for (int k = 0; k < RMS_KE; ++k) {
+      const int i = base + tid + k * bs;
+      const long long p = i < D ? (long long)xv[k] * gm[k] * inv : 0;
+      const int ml = max16_lanes(p ? lead64(p) : 0);
       int sh;
-      ym[i] = (int16_t)norm16(p, ml, sh);
-      if ((i & 15) == 0)
-        ye[i >> 4] = (int8_t)clamp8((int)xex[i >> 4] + (int)ge[i >> 4] + einv + sh - 27);
+      const int m = norm16(p, ml, sh);
+      out(i, m, clamp8(xe[k] + ge[k] + einv + sh - 27));
     }
   }
 }
 
-// gen_rmsnorm_bfp_golden.py:42-142: one workgroup (64 threads) per vector;
-// tile sums in parallel, the cross-tile fold and Newton-Raphson in lane 0,
-// the per-tile output normalisation one element per lane.
-__global__ __launch_bounds__(64) void k_rtl_rmsnorm(const int16_t *__restrict__ xm,
-                                                    const int8_t *__restrict__ xe,
-                                                    const int16_t *__restrict__ gm,
-                                                    const int8_t *__restrict__ ge, int D,
-                                                    int16_t *ym, int8_t *ye) {
-  extern __shared__ long long sums[];   // nt tile sums
-  __shared__ long long s_inv;
-  __shared__ int s_einv;
+// gen_rmsnorm_bfp_golden.py:42-142: one workgroup per vector.
+constexpr int RMS_T = 256;
+__global__ __launch_bounds__(RMS_T) void k_rtl_rmsnorm(const int16_t *__restrict__ xm, const int8_t *__restrict__ xe,
+                                                       const int16_t *__restrict__ gm, const int8_t *__restrict__ ge,
+                                                       int D, int16_t *__restrict__ ym, int8_t *__restrict__ ye) {
+  extern __shared__ long long sums[];   // nt tile sums, nt exponents
   const int b = blockIdx.x, nt = D / 16;
-  rmsnorm_wave(xm + (long long)b * D, xe + (long long)b * nt, gm, ge, D, ym + (long long)b * D,
-               ye + (long long)b * nt, sums, &s_inv, &s_einv);
+  ym += (long long)b * D;
+  ye += (long long)b * nt;
+  rms_block(
+      xm + (long long)b * D, xe + (long long)b * nt,
+      [&](int i, int &m, int &e) {
+        m = gm[i];
+        e = ge[i >> 4];
+      },
+      D, sums, reinterpret_cast<int *>(sums + nt),
+      [&](int i, int m, int e) {
+        if (i >= D) return;
+        ym[i] = (int16_t)m;
+        if ((i & 15) == 0) ye[i >> 4] = (int8_t)e;
+      });
 }
 
 // -------------------------------------------------------------------- rope
@@ -386,46 +473,102 @@ __device__ __forceinline__ bool bfp_gt(int ma, int ea, int mb, int eb) {
   return (-de >= 16 ? 0 : (ma >> (-de))) > mb;
 }
 
+// A chunk's best as one word: mantissa, exponent byte, lane.
+__device__ __forceinline__ int arg_word(int m, int e, int k) {
+  return (int)((unsigned)m << 16 | ((unsigned)e & 0xffu) << 8 | (unsigned)k);
+}
+__device__ __forceinline__ int arg_m(int w) { return w >> 16; }
+__device__ __forceinline__ int arg_e(int w) { return (int)(signed char)((w >> 8) & 0xff); }
+
+// The running argmax over chunk words w[0 .. nc) by one wave, in order
+// (bfp_gt is not transitive under truncation, so the order counts): every
+// lane compares one of 64 chunks with the best so far; the first lane whose
+// chunk is greater is the next replacement -- the chunks before it were
+// compared with the very best they would have met -- and the lanes after it
+// compare again.  A block without a replacement costs one comparison, and a
+// sequence's best is replaced about ln(nc) times: 3072 chunks take 11 us,
+// against 485 as one lane's fold.  Returns the best's index (16 chunk + lane) in every lane.
+__device__ __forceinline__ int argmax_fold(const int *__restrict__ w, int nc) {
+  const int l = threadIdx.x & 63;
+  constexpr int U = 16;   // blocks of 64 chunks loaded together
+  int bm = -32768, be = -128, bi = 0;
+  for (int c0 = 0; c0 < nc; c0 += 64 * U) {   // uniform
+    int v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int c = c0 + 64 * u + l;
+      v[u] = w[c < nc ? c : nc - 1];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int cb = c0 + 64 * u;
+      const int m = arg_m(v[u]), e = arg_e(v[u]);
+      unsigned long long rest = cb + 64 <= nc ? ~0ull : (cb < nc ? (1ull << (nc - cb)) - 1 : 0ull);
+      for (;;) {
+        const unsigned long long gt = __ballot(bfp_gt(m, e, bm, be)) & rest;
+        if (!gt) break;
+        const int j = __builtin_ctzll(gt);
+        const int wj = __builtin_amdgcn_readlane(v[u], j);
+        bm = arg_m(wj);
+        be = arg_e(wj);
+        bi = (cb + j) * 16 + (wj & 15);
+        rest &= j == 63 ? 0ull : ~0ull << (j + 1);
+      }
+    }
+  }
+  return bi;
+}
+
 // The decode head's running argmax (smollm_decode_head_bfp.sv:322-324,
-// 399-430): chunk-local bests in parallel, then the ordered fold over chunks
-// (bfp_gt is not transitive under truncation, so the fold order is kept).
-__global__ __launch_bounds__(256) void k_rtl_argmax(const int16_t *__restrict__ m,
-                                                    const int8_t *__restrict__ e, int n,
-                                                    int *lm, int *le, int *li, int *out) {
+// 399-430): chunk-local bests in parallel (lane 0 of a chunk seeds, the
+// others replace only when greater), then the ordered fold over chunks.
+// work: one word per chunk.
+constexpr int ARGMAX_T = 1024;
+__global__ __launch_bounds__(ARGMAX_T) void k_rtl_argmax(const int16_t *__restrict__ m, const int8_t *__restrict__ e,
+                                                         int n, int *work, int *out) {
   const int b = blockIdx.x, tid = threadIdx.x, nc = n / 16;
   const int16_t *mb = m + (long long)b * n;
   const int8_t *eb = e + (long long)b * n;
-  int *LM = lm + (long long)b * nc, *LE = le + (long long)b * nc, *LI = li + (long long)b * nc;
-  for (int c = tid; c < nc; c += blockDim.x) {
-    int bm = mb[c * 16], be_ = eb[c * 16], bi = 0;
-    for (int k = 1; k < 16; ++k)
-      if (bfp_gt(mb[c * 16 + k], eb[c * 16 + k], bm, be_)) {
-        bm = mb[c * 16 + k];
-        be_ = eb[c * 16 + k];
-        bi = k;
-      }
-    LM[c] = bm;
-    LE[c] = be_;
-    LI[c] = c * 16 + bi;
+  int *W = work + (long long)b * nc;
+  for (int c = tid; c < nc; c += ARGMAX_T) {
+    int mm[16], ee[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      mm[k] = mb[c * 16 + k];
+      ee[k] = eb[c * 16 + k];
+    }
+    int bm = mm[0], be = ee[0], bi = 0;
+#pragma unroll
+    for (int k = 1; k < 16; ++k) {
+      const bool g = bfp_gt(mm[k], ee[k], bm, be);
+      bm = g ? mm[k] : bm;
+      be = g ? ee[k] : be;
+      bi = g ? k : bi;
+    }
+    W[c] = arg_word(bm, be, bi);
   }
   __syncthreads();
-  if (tid == 0) {
-    int bm = -32768, be_ = -128, bi = 0;
-    for (int c = 0; c < nc; ++c)
-      if (bfp_gt(LM[c], LE[c], bm, be_)) {
-        bm = LM[c];
-        be_ = LE[c];
-        bi = LI[c];
-      }
-    out[b] = bi;
+  if (tid < 64) {
+    const int bi = argmax_fold(W, nc);
+    if (tid == 0) out[b] = bi;
   }
+}
+
+// The fold alone, over words that the head's matvec wrote.
+__global__ __launch_bounds__(64) void k_rl_argmax_fold(const int *__restrict__ w, int nc, int *out) {
+  const int bi = argmax_fold(w, nc);
+  if (threadIdx.x == 0) *out = bi;
 }
 
 // ===================================================== composed RTL layer
 // smollm_layer_bfp.sv:1603-2600 on one sequence: the engines above wired in
 // the FSM's order, with the matvec engine's sequential tile fold over the
-// device-layout weights.  Eight launches: NORM1, Q/K/V, RoPE + KV write,
-// attention, O + residual 1, NORM2, G/U + SwiGLU, D + residual 2.
+// device-layout weights.  Five launches: NORM1 + Q/K/V, RoPE + KV write +
+// attention, O + residual 1, NORM2 + G/U + SwiGLU, D + residual 2.  Each launch
+// is a chain of a few microseconds whatever its size, so the norm is
+// recomputed by every chunk's workgroup, and RoPE by every head's: the layer
+// of 576/1536 takes 37 us in a replayed step (7.8, 8.2, 5.2, 9.7 and 6.5),
+// against 92 as eight launches with one-wave norms and in-order folds.
 
 __device__ __forceinline__ void st_put(const StageDump *sd, int s, int i, int m) {
   if (sd && sd->m[s]) sd->m[s][i] = (int16_t)m;
@@ -461,52 +604,6 @@ __device__ __forceinline__ void swiglu16(int gm, int ge, int um, int ue,
   int s;
   ym = norm16(p, ml, s);
   ye = clamp8(ue + s - 10);
-}
-
-// One step of the engine's fold (gen_matvec_bfp_golden.py:53-108): the side
-// with the smaller exponent is shifted right (zeroed past 47), then the
-// 48-bit saturating add.
-__device__ __forceinline__ void engine_fold(long long &acc, int &acc_e, long long s, int te) {
-  const long long HI = (1LL << (ACC_W - 1)) - 1, LO = -(1LL << (ACC_W - 1));
-  const int d = te - acc_e;
-  if (d > 0) {
-    acc = d > ACC_W - 1 ? 0 : (acc >> d);
-    acc_e = te;
-  } else if (d < 0) {
-    s = -d > ACC_W - 1 ? 0 : (s >> (-d));
-  }
-  acc += s;
-  acc = acc > HI ? HI : (acc < LO ? LO : acc);
-}
-
-// NORM1 (second == 0: h, G1) or NORM2 (h1, G2) -> xn.  The gamma ROM holds
-// tile_quantize of the float gamma; it is formed here.
-__global__ __launch_bounds__(64) void k_rl_norm(RtlArgs a, int second) {
-  extern __shared__ long long rl_lds[];
-  __shared__ long long s_inv;
-  __shared__ int s_einv;
-  const LayerArgs &L = a.L;
-  const int D = L.D, nt = D / 16, tid = threadIdx.x;
-  long long *sums = rl_lds;
-  int16_t *gm = reinterpret_cast<int16_t *>(rl_lds + nt);
-  int8_t *ge = reinterpret_cast<int8_t *>(gm + D);
-  const double *g = second ? L.g2 : L.g1;
-  for (int base = 0; base < D; base += 64) {   // D % 64 == 0: whole 16-lane tiles
-    const int i = base + tid;
-    int e;
-    const int m = quantize16_lanes(g[i], e);
-    gm[i] = (int16_t)m;
-    if ((i & 15) == 0) ge[i >> 4] = (int8_t)e;
-  }
-  __syncthreads();
-  rmsnorm_wave(second ? L.h1_m : L.h_m, second ? L.h1_e : L.h_e, gm, ge, D, L.xn_m, L.xn_e, sums,
-               &s_inv, &s_einv);
-  if (L.dump) {
-    __syncthreads();
-    const int st = second ? ST_N2 : ST_N1;
-    for (int i = tid; i < D; i += 64) st_put(L.dump, st, i, L.xn_m[i]);
-    for (int t = tid; t < nt; t += 64) st_pute(L.dump, st, t, L.xn_e[t]);
-  }
 }
 
 // Exact tile sums S = sum_k x[t,k] W[r,t,k] and exponents E = x_e[t] + W_e[r,t]
@@ -550,87 +647,137 @@ __device__ __forceinline__ void tile_sums_to_lds(const ChunkRegs<TPT> &R, const 
 #undef RL_DOT2
 }
 
-// One 16-row chunk on the engine: sets, in every lane of wave 0, row
-// (lane & 15)'s per-lane output (m, e) (the engine's out_mant / out_exp).
-// All threads call it; it synchronises.
-template <int NW, int TPT>
-__device__ void rl_chunk_me(const uint4 *__restrict__ pm, const int8_t *__restrict__ pe, int nT,
-                            const int *xs, const int *xes, long long *Sl, int *El, int &m, int &e) {
-  ChunkRegs<TPT> R;
-  load_chunk_nb<NW, TPT>(R, pm, pe, nT);
-  tile_sums_to_lds<NW, TPT>(R, xs, xes, nT, Sl, El);
-  __syncthreads();
+// NC <= 2 16-row chunks (weights in R) on the engine: sets, in lane 16 c + r
+// of wave 0 (c < NC), row r of chunk c's per-lane output (m, e) (the engine's
+// out_mant / out_exp).  All threads call it; it synchronises.
+template <int NW, int TPT, int NC>
+__device__ __forceinline__ void rl_chunk_me(const ChunkRegs<TPT> (&R)[NC], int nT, const int *xs, const int *xes,
+                                            long long *Sl, int *El, int &m, int &e) {
+#pragma unroll
+  for (int c = 0; c < NC; ++c) tile_sums_to_lds<NW, TPT>(R[c], xs, xes, nT, Sl + c * nT * 16, El + c * nT * 16);
+  lds_barrier();
   m = 0;
   e = 0;
   if (threadIdx.x < 64) {
-    const int r = threadIdx.x & 15;
-    long long acc = Sl[r];
-    int acc_e = El[r];
-    for (int t = 1; t < nT; ++t) engine_fold(acc, acc_e, Sl[t * 16 + r], El[t * 16 + r]);
+    // PQ lanes a row, each a run of tiles.  A run maps acc to (acc + B) >> T
+    // with T the rise of the exponent's maximum over it and B its aligned
+    // sums shifted up by the rise so far (floors of floors), so the runs
+    // fold side by side and combine in order.  Rises past 20 in a run (B
+    // might leave 64 bits, or a step drop acc) take the sequential form.
+    constexpr int PQ = 4 / NC, NONE = -100000;
+    const int grp = threadIdx.x >> 4, lc = NC == 2 ? grp & 1 : 0, q = NC == 2 ? grp >> 1 : grp;
+    const long long *S = Sl + lc * nT * 16 + (threadIdx.x & 15);
+    const int *E = El + lc * nT * 16 + (threadIdx.x & 15);
+    const int run = (nT + PQ - 1) / PQ, t0 = q * run, t1 = t0 + run < nT ? t0 + run : nT;
+    int mxq = NONE;
+#pragma unroll 8
+    for (int t = t0; t < t1; ++t) mxq = E[t * 16] > mxq ? E[t * 16] : mxq;
+    // the maximum before this run (its own first exponent for the first)
+    int p0 = E[0];
+    if constexpr (NC == 1) {
+      const int a = peer<16>(mxq), b = peer<32>(mxq), c = peer<32>(a);
+      // rows of 16: q 1 has a = run 0; q 2 has b, c = runs 0, 1; q 3 a, b, c = runs 2, 1, 0
+      const int bc = b > c ? b : c, abc = a > bc ? a : bc;
+      p0 = q == 0 ? p0 : (q == 1 ? a : (q == 2 ? bc : abc));
+    } else {
+      const int b = peer<32>(mxq);
+      p0 = q == 0 ? p0 : b;
+    }
+    int p = p0;
+    long long B = 0;
+#pragma unroll 4
+    for (int t = t0; t < t1; ++t) {
+      const int te = E[t * 16];
+      p = te > p ? te : p;
+      const int dn = p - te, up = p - p0;
+      B += (dn > ACC_W - 1 ? 0 : (S[t * 16] >> dn)) << (up < 20 ? up : 20);
+    }
+    const int T = p - p0;
+    long long acc;
+    int acc_e;
+    if (!__any(T > 20)) {
+      acc = (B >> T);
+      acc_e = p;
+      if constexpr (NC == 1) {
+        const long long B1 = peer<16>(B), B2 = peer<32>(B), B3 = peer<32>(B1);
+        const int T1 = peer<16>(T), T2 = peer<32>(T), T3 = peer<32>(T1), e3 = peer<32>(peer<16>(p));
+        acc = (((acc + B1) >> T1) + B2) >> T2;
+        acc = (acc + B3) >> T3;
+        acc_e = e3;
+      } else {
+        const long long B1 = peer<32>(B);
+        const int T1 = peer<32>(T);
+        acc = (acc + B1) >> T1;
+        acc_e = peer<32>(p);
+      }
+    } else {
+      acc = S[0];
+      acc_e = E[0];
+#pragma unroll 4
+      for (int t = 1; t < nT; ++t) tile_fold(acc, acc_e, S[t * 16], E[t * 16]);
+    }
     int sh;
     m = norm16(acc, lead64(acc), sh);
     e = clamp8(acc_e + sh - 15);
   }
-  __syncthreads();   // Sl / El free for the next chunk
 }
 
-// The same chunk, then the chunk re-tile (S_xMV_DRAIN/REQ): returns, in
-// every lane of wave 0, row (lane & 15)'s re-tiled mantissa and sets emax
-// to the chunk exponent.
-template <int NW, int TPT>
-__device__ int rl_chunk(const uint4 *__restrict__ pm, const int8_t *__restrict__ pe, int nT,
-                        const int *xs, const int *xes, long long *Sl, int *El, int &emax) {
-  int m, e;
-  rl_chunk_me<NW, TPT>(pm, pe, nT, xs, xes, Sl, El, m, e);
-  int mq = 0;
-  emax = 0;
-  if (threadIdx.x < 64) {
-    emax = max16_lanes(e);
-    mq = shr8(m, emax, e);
-  }
-  return mq;
-}
+// Gamma element i as the gamma ROM holds it: tile_quantize of the float
+// gamma (whole waves, 16-lane groups on one tile).
+struct RomGamma {
+  const double *g;
+  __device__ __forceinline__ void operator()(int i, int &m, int &e) const { m = quantize16_lanes(g[i], e); }
+};
 
-// The layer's matvecs, one 16-row output chunk per workgroup.
-//   op 0: Q|K|V from xn            (chunks of qkv, re-tiled per chunk)
-//   op 1: O from att, then residual 1 with h -> h1
-//   op 2: G chunk c and U chunk c from xn, then SwiGLU -> mlp
-//   op 3: D from mlp, then residual 2 with h1 -> h
-template <int NW>
-__global__ __launch_bounds__(64 * NW) void k_rl_mv(RtlArgs a, int op) {
-  constexpr int TPT = 3;
+// The layer's matvecs, one 16-row output chunk per workgroup, every weight
+// load issued before the input is staged.
+//   OP 0: Q|K|V from NORM1(h, G1)  (chunks of qkv, re-tiled per chunk)
+//   OP 1: O from att, then residual 1 with h -> h1
+//   OP 2: G chunk c and U chunk c from NORM2(h1, G2), then SwiGLU -> mlp
+//   OP 3: D from mlp, then residual 2 with h1 -> h
+template <int NW, int op>
+__global__ __launch_bounds__(64 * NW) void k_rl_mv(RtlArgs a) {
+  constexpr int TPT = 3, NC = op == 2 ? 2 : 1;
   extern __shared__ long long rl_lds[];
   const LayerArgs &L = a.L;
   const int c = blockIdx.x;
   const int nT = (op == 3 ? L.FFN : L.D) / 16;
-  long long *Sl = rl_lds;
-  int *El = reinterpret_cast<int *>(Sl + nT * 16);
-  int *xs = El + nT * 16;
-  int *xes = xs + nT * 16;
-  const int16_t *xm = op == 1 ? L.att_m : (op == 3 ? L.mlp_m : L.xn_m);
-  const int8_t *xe = op == 1 ? L.att_e : (op == 3 ? L.mlp_e : L.xn_e);
-  stage_x_bfp(xs, xes, xm, xe, nT);
-  __syncthreads();
-  const uint4 *wm;
-  const int8_t *we;
-  int chunk = c;
-  if (op == 0) {
-    wm = L.w_qkv_m, we = L.w_qkv_e;
-  } else if (op == 1) {
-    wm = L.w_o_m, we = L.w_o_e;
-  } else if (op == 2) {
-    wm = L.w_gu_m, we = L.w_gu_e, chunk = 2 * c;
+  long long *Sl = rl_lds;                                  // NC x nT x 16
+  long long *sums = Sl + NC * nT * 16;                     // nT
+  int *El = reinterpret_cast<int *>(sums + nT);            // NC x nT x 16
+  int *xs = El + NC * nT * 16;                             // nT x 16
+  int *xes = xs + nT * 16;                                 // nT
+  int *sexp = xes + nT;                                    // nT
+  const uint4 *wm = op == 0 ? L.w_qkv_m : (op == 1 ? L.w_o_m : (op == 2 ? L.w_gu_m : L.w_d_m));
+  const int8_t *we = op == 0 ? L.w_qkv_e : (op == 1 ? L.w_o_e : (op == 2 ? L.w_gu_e : L.w_d_e));
+  ChunkRegs<TPT> R[NC];
+#pragma unroll
+  for (int k = 0; k < NC; ++k)
+    load_chunk_nb<NW, TPT>(R[k], wm + (size_t)(NC * c + k) * nT * 32, we + (size_t)(NC * c + k) * nT * 16, nT);
+  if constexpr (op == 0 || op == 2) {
+    const StageDump *sd = c == 0 ? L.dump : nullptr;
+    constexpr int st = op == 0 ? ST_N1 : ST_N2;
+    rms_block(op == 0 ? L.h_m : L.h1_m, op == 0 ? L.h_e : L.h1_e, RomGamma{op == 0 ? L.g1 : L.g2}, L.D, sums, sexp,
+              [&](int i, int m, int e) {
+                // the even lane writes the pair into the matvec's input form
+                const int odd = __builtin_amdgcn_mov_dpp(m, 0xB1, 0xf, 0xf, false);   // quad_perm 1,0,3,2
+                if (i >= L.D) return;
+                if ((i & 1) == 0) put_x_pair(xs, i >> 4, (i >> 1) & 7, m, odd);
+                if ((i & 15) == 0) xes[i >> 4] = e;
+                st_put(sd, st, i, m);
+                if ((i & 15) == 0) st_pute(sd, st, i >> 4, e);
+              });
   } else {
-    wm = L.w_d_m, we = L.w_d_e;
+    stage_x_bfp(xs, xes, op == 1 ? L.att_m : L.mlp_m, op == 1 ? L.att_e : L.mlp_e, nT);
   }
-  int emax;
-  const int mq = rl_chunk<NW, TPT>(wm + (size_t)chunk * nT * 32, we + (size_t)chunk * nT * 16, nT,
-                                   xs, xes, Sl, El, emax);
-  int mu = 0, eu = 0;
-  if (op == 2)
-    mu = rl_chunk<NW, TPT>(wm + (size_t)(chunk + 1) * nT * 32, we + (size_t)(chunk + 1) * nT * 16,
-                           nT, xs, xes, Sl, El, eu);
+  lds_barrier();
+  int m, e;
+  rl_chunk_me<NW, TPT, NC>(R, nT, xs, xes, Sl, El, m, e);
   if (threadIdx.x >= 64) return;
+  // the chunk re-tile (S_xMV_DRAIN/REQ): lanes 0-15 chunk 0, 16-31 chunk 1
+  const int em = max16_lanes(e), mt = shr8(m, em, e);
+  const int mq = mt, emax = em;
+  const int mu = __shfl(mt, (threadIdx.x & 15) + 16, 64), eu = __shfl(em, (threadIdx.x & 15) + 16, 64);
   const int r = threadIdx.x & 15, i = c * 16 + r;
   const bool w = threadIdx.x < 16;
   const StageDump *sd = L.dump;
@@ -676,149 +823,181 @@ __global__ __launch_bounds__(64 * NW) void k_rl_mv(RtlArgs a, int op) {
   }
 }
 
-// RoPE of Q head h (h < H_Q) or K head h - H_Q, then the re-tile of its four
-// tiles (S_ROPEx_RQ_A/B); K heads also write the KV slot kv_pos with the
-// rotated K and the V head (S_KVWR_M/E).  One 64-thread workgroup per head.
 // The step of the RTL layer: a.pos / a.kv_pos, or the device step counter.
 __device__ __forceinline__ int rl_pos(const RtlArgs &a) { return a.pos_ptr ? *a.pos_ptr : a.pos; }
 __device__ __forceinline__ int rl_kv_pos(const RtlArgs &a) { return a.pos_ptr ? *a.pos_ptr : a.kv_pos; }
 
-__global__ __launch_bounds__(64) void k_rl_rope_kv(RtlArgs a) {
-  const LayerArgs &L = a.L;
-  const int h = blockIdx.x, j = threadIdx.x & 31, HD = 64;
-  const bool is_k = h >= L.H_Q;
-  const int kh = h - L.H_Q;
-  const int off = is_k ? L.D + kh * HD : h * HD;   // element offset in qkv
-  const int16_t *x = L.qkv_m + off;
-  const int8_t *e = L.qkv_e + off / 16;
-  const long long ang = wrap31((wrap31((long long)rl_pos(a) * a.freq[j]) * PI_OVER_8_Q29) >> 29);
-  int cs, sn;
-  cordic(ang, cs, sn);
+// RoPE of one head (x: 64 mantissas, e: 4 exponents) by the first 32 lanes
+// of a wave (lanes 32-63 repeat them), then the re-tile of its four tiles
+// (S_ROPEx_RQ_A/B): elements j and j + 32 in (qlo, elo), (qhi, ehi).
+__device__ __forceinline__ void rl_rope(const int16_t *x, const int8_t *e, int pos, const unsigned *freq, int &qlo,
+                                        int &elo, int &qhi, int &ehi) {
+  const int j = threadIdx.x & 31;
+  const long long ang = wrap31((wrap31((long long)pos * freq[j]) * PI_OVER_8_Q29) >> 29);
   const int xa = x[j], xb = x[j + 32];
   const int ea = e[j >> 4], eb = e[(j + 32) >> 4];
+  int cs, sn;
+  cordic(ang, cs, sn);
   const int em = ea > eb ? ea : eb;
   const long long aa = em - ea < 16 ? (xa >> (em - ea)) : 0;
   const long long ba = em - eb < 16 ? (xb >> (em - eb)) : 0;
   const long long lo = aa * cs - ba * sn, hi = ba * cs + aa * sn;
   int sh;
   const int mlo = norm16(lo, lead64(lo), sh);
-  const int elo = clamp8(em + sh - 15);
+  const int e0 = clamp8(em + sh - 15);
   const int mhi = norm16(hi, lead64(hi), sh);
-  const int ehi = clamp8(em + sh - 15);
+  const int e1 = clamp8(em + sh - 15);
   // lanes 0-15 hold tiles 0 (lo) and 2 (hi), lanes 16-31 tiles 1 and 3
-  const int emlo = max16_lanes(elo), emhi = max16_lanes(ehi);
-  const int qlo = shr8(mlo, emlo, elo), qhi = shr8(mhi, emhi, ehi);
-  if (threadIdx.x >= 32) return;
-  const StageDump *sd = L.dump;
-  int16_t *ym = L.qkv_m + off;
-  int8_t *ye = L.qkv_e + off / 16;
-  ym[j] = (int16_t)qlo;
-  ym[j + 32] = (int16_t)qhi;
-  if ((j & 15) == 0) {
-    ye[j >> 4] = (int8_t)emlo;
-    ye[(j + 32) >> 4] = (int8_t)emhi;
-  }
-  const int st = is_k ? ST_K : ST_Q, so = is_k ? kh * HD : h * HD;
-  st_put(sd, st, so + j, qlo);
-  st_put(sd, st, so + j + 32, qhi);
-  if ((j & 15) == 0) {
-    st_pute(sd, st, so / 16 + (j >> 4), emlo);
-    st_pute(sd, st, so / 16 + ((j + 32) >> 4), emhi);
-  }
-  if (!is_k) return;
-  const size_t slot = (size_t)rl_kv_pos(a) * L.H_KV + kh;   // sequence 0
-  int16_t *km = L.k_m + slot * HD;
-  int8_t *ke = L.k_e + slot * (HD / 16);
-  km[j] = (int16_t)qlo;
-  km[j + 32] = (int16_t)qhi;
-  if ((j & 15) == 0) {
-    ke[j >> 4] = (int8_t)emlo;
-    ke[(j + 32) >> 4] = (int8_t)emhi;
-  }
-  const int voff = L.D + L.KV + kh * HD;
-  int16_t *vm = L.v_m + slot * HD;
-  int8_t *ve = L.v_e + slot * (HD / 16);
-  const int v0 = L.qkv_m[voff + j], v1 = L.qkv_m[voff + j + 32];
-  vm[j] = (int16_t)v0;
-  vm[j + 32] = (int16_t)v1;
-  st_put(sd, ST_V, kh * HD + j, v0);
-  st_put(sd, ST_V, kh * HD + j + 32, v1);
-  if (j < 4) {
-    const int vt = L.qkv_e[voff / 16 + j];
-    ve[j] = (int8_t)vt;
-    st_pute(sd, ST_V, kh * 4 + j, vt);
-  }
+  elo = max16_lanes(e0);
+  ehi = max16_lanes(e1);
+  qlo = shr8(mlo, elo, e0);
+  qhi = shr8(mhi, ehi, e1);
 }
 
 constexpr int RL_ATT_T = 256;
 
-__device__ __forceinline__ int block_max_i(int v, int *red) {
-  for (int o = 1; o < 64; o <<= 1) {
-    const int w = __shfl_xor(v, o, 64);
-    v = w > v ? w : v;
-  }
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  v = red[0];
-  for (int i = 1; i < RL_ATT_T / 64; ++i) v = red[i] > v ? red[i] : v;
-  return v;
+__device__ __forceinline__ int wave_max_i(int v) {
+  v = max16_lanes(v);
+  v = pmax<16>(v);
+  return pmax<32>(v);
 }
 
-__device__ __forceinline__ long long block_sum_ll(long long v, long long *red) {
-  for (int o = 1; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  v = 0;
-  for (int i = 0; i < RL_ATT_T / 64; ++i) v += red[i];
-  return v;
-}
-
-// Attention of query head h (S_QK_* .. S_AV_*): scores of t = 0..kv_pos on
-// the engine's lane 0 (Q head as x, K[t] as the weight row), pre-align to the
-// shared max exponent, softmax with exponent - 3 (1/sqrt(64)), then per
-// 16-dim chunk the engine over one 16-input tile of probabilities (t <= 15)
-// with V pre-shifted to its largest exponent over t <= kv_pos.
+// RoPE and attention of query head h (S_ROPE*, S_KVWR_*, S_QK_* .. S_AV_*):
+// wave 0 rotates the head's Q, wave 1 its K head, wave 2 takes its V; the
+// first head of a KV group writes the slot kv_pos (rotated K, V), and row
+// kv_pos is used from LDS.  Then scores of t = 0..kv_pos on the engine's lane
+// 0 (Q head as x, K[t] as the weight row), pre-align to the shared max
+// exponent, softmax with exponent - 3 (1/sqrt(64)), then per 16-dim chunk the
+// engine over one 16-input tile of probabilities (t <= 15) with V pre-shifted
+// to its largest exponent over t <= kv_pos.
 __global__ __launch_bounds__(RL_ATT_T) void k_rl_attn(RtlArgs a) {
   extern __shared__ long long rl_lds[];
-  __shared__ int qs[64], qe[4], red_i[RL_ATT_T / 64], s_pe, s_vmax[4];
-  __shared__ long long red_l[RL_ATT_T / 64], s_inv;
+  constexpr int NW = RL_ATT_T / 64;
+  __shared__ int qs[64], qe[4], red_e[NW], red_x[NW], red_s[NW], red_v[4 * NW];
+  __shared__ __align__(16) int16_t kc[64], vc[64];
+  __shared__ int kce[4], vce[4];
   __shared__ int pm[16];
   const LayerArgs &L = a.L;
-  const int h = blockIdx.x, tid = threadIdx.x, HD = 64;
+  const int h = blockIdx.x, tid = threadIdx.x, HD = 64, wv = tid >> 6, ln = tid & 63;
   const int g = (h * L.H_KV) / L.H_Q;
-  const int n = rl_kv_pos(a) + 1;
+  const bool writer = h == 0 || ((h - 1) * L.H_KV) / L.H_Q != g;
+  const int kv = rl_kv_pos(a), n = kv + 1;
   int *xs = reinterpret_cast<int *>(rl_lds);   // n aligned scores, then LUT values
   int *se = xs + n;                             // n score exponents
-  if (tid < 64) qs[tid] = L.qkv_m[h * HD + tid];
-  if (tid < 4) qe[tid] = L.qkv_e[h * 4 + tid];
-  __syncthreads();
+  const size_t slot0 = (size_t)kv * L.H_KV + g;   // sequence 0
+  const StageDump *sd = L.dump;
+  if (wv < 2) {
+    const int off = wv == 0 ? h * HD : L.D + g * HD, j = ln & 31;
+    int qlo, elo, qhi, ehi;
+    rl_rope(L.qkv_m + off, L.qkv_e + off / 16, rl_pos(a), a.freq, qlo, elo, qhi, ehi);
+    if (ln < 32) {
+      if (wv == 0) {
+        qs[j] = qlo;
+        qs[j + 32] = qhi;
+        if ((j & 15) == 0) {
+          qe[j >> 4] = elo;
+          qe[(j + 32) >> 4] = ehi;
+        }
+      } else {
+        kc[j] = (int16_t)qlo;
+        kc[j + 32] = (int16_t)qhi;
+        if ((j & 15) == 0) {
+          kce[j >> 4] = elo;
+          kce[(j + 32) >> 4] = ehi;
+        }
+        if (writer) {
+          int16_t *km = L.k_m + slot0 * HD;
+          int8_t *ke = L.k_e + slot0 * (HD / 16);
+          km[j] = (int16_t)qlo;
+          km[j + 32] = (int16_t)qhi;
+          if ((j & 15) == 0) {
+            ke[j >> 4] = (int8_t)elo;
+            ke[(j + 32) >> 4] = (int8_t)ehi;
+          }
+        }
+      }
+      const int st = wv == 0 ? ST_Q : ST_K, so = wv == 0 ? h * HD : g * HD;
+      if (wv == 0 || writer) {
+        st_put(sd, st, so + j, qlo);
+        st_put(sd, st, so + j + 32, qhi);
+        if ((j & 15) == 0) {
+          st_pute(sd, st, so / 16 + (j >> 4), elo);
+          st_pute(sd, st, so / 16 + ((j + 32) >> 4), ehi);
+        }
+      }
+    }
+  } else if (wv == 2) {
+    const int off = L.D + L.KV + g * HD;
+    const int v = L.qkv_m[off + ln], vt = L.qkv_e[off / 16 + (ln & 3)];
+    vc[ln] = (int16_t)v;
+    if (ln < 4) vce[ln] = vt;
+    if (writer) {
+      L.v_m[slot0 * HD + ln] = (int16_t)v;
+      st_put(sd, ST_V, g * HD + ln, v);
+      if (ln < 4) {
+        L.v_e[slot0 * (HD / 16) + ln] = (int8_t)vt;
+        st_pute(sd, ST_V, g * 4 + ln, vt);
+      }
+    }
+  }
+  lds_barrier();
   for (int t = tid; t < n; t += RL_ATT_T) {
-    const size_t slot = (size_t)t * L.H_KV + g;
-    const int16_t *k = L.k_m + slot * HD;
-    const int8_t *ke = L.k_e + slot * 4;
+    const size_t slot = (size_t)(t < kv ? t : 0) * L.H_KV + g;
+    const uint4 *kp = reinterpret_cast<const uint4 *>(t < kv ? L.k_m + slot * HD : kc);
+    const int ke4 = *reinterpret_cast<const int *>(L.k_e + slot * 4);
+    uint4 kr[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) kr[q] = kp[q];
     long long acc = 0;
     int acc_e = 0;
+#pragma unroll
     for (int c = 0; c < 4; ++c) {
       long long s = 0;
-      for (int kk = 0; kk < 16; ++kk) s += (long long)qs[c * 16 + kk] * k[c * 16 + kk];
-      const int te = qe[c] + ke[c];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const unsigned wd[4] = {kr[2 * c + q].x, kr[2 * c + q].y, kr[2 * c + q].z, kr[2 * c + q].w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int *x = qs + c * 16 + 8 * q + 2 * k;
+          s += (long long)(x[0] * (int)(short)(wd[k] & 0xffff)) + (long long)(x[1] * ((int)wd[k] >> 16));
+        }
+      }
+      const int te = qe[c] + (t < kv ? (int)(signed char)((ke4 >> (8 * c)) & 0xff) : kce[c]);
       if (c == 0) {
         acc = s;
         acc_e = te;
       } else {
-        engine_fold(acc, acc_e, s, te);
+        tile_fold(acc, acc_e, s, te);
       }
     }
     int sh;
     xs[t] = norm16(acc, lead64(acc), sh);
     se[t] = clamp8(acc_e + sh - 15);
   }
-  __syncthreads();
-  int lmax = -128;
-  for (int t = tid; t < n; t += RL_ATT_T) lmax = se[t] > lmax ? se[t] : lmax;
-  const int es = block_max_i(lmax, red_i);
+  // (each thread reads back only the scores it wrote until the last barrier)
+  // the largest score exponent, and V's per 16-dim chunk over t <= kv_pos
+  int lmax = -128, vm4[4] = {-128, -128, -128, -128};
+  for (int t = tid; t < n; t += RL_ATT_T) {
+    lmax = se[t] > lmax ? se[t] : lmax;
+    const int ve4 = *reinterpret_cast<const int *>(L.v_e + ((size_t)(t < kv ? t : 0) * L.H_KV + g) * 4);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int ve = t < kv ? (int)(signed char)((ve4 >> (8 * c)) & 0xff) : vce[c];
+      vm4[c] = ve > vm4[c] ? ve : vm4[c];
+    }
+  }
+  lmax = wave_max_i(lmax);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) vm4[c] = wave_max_i(vm4[c]);
+  if (ln == 0) {
+    red_e[wv] = lmax;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) red_v[4 * wv + c] = vm4[c];
+  }
+  lds_barrier();
+  int es = red_e[0];
+#pragma unroll
+  for (int i = 1; i < NW; ++i) es = red_e[i] > es ? red_e[i] : es;
   int xmax = -32768;
   for (int t = tid; t < n; t += RL_ATT_T) {
     const int d = es - se[t];               // 9-bit in the FSM: no wrap
@@ -826,10 +1005,15 @@ __global__ __launch_bounds__(RL_ATT_T) void k_rl_attn(RtlArgs a) {
     xs[t] = v;
     xmax = v > xmax ? v : xmax;
   }
-  const int mx = block_max_i(xmax, red_i);
+  xmax = wave_max_i(xmax);
+  if (ln == 0) red_x[wv] = xmax;
+  lds_barrier();
+  int mx = red_x[0];
+#pragma unroll
+  for (int i = 1; i < NW; ++i) mx = red_x[i] > mx ? red_x[i] : mx;
   const int xe = (int)(signed char)(es - 3);
   const int sh = xe - 8;
-  long long part = 0;
+  int part = 0;                              // at most 4096 * 65535
   for (int t = tid; t < n; t += RL_ATT_T) {
     const long long d = (long long)xs[t] - mx;
     const long long ds = sh >= 0 ? d * (1LL << (sh > 40 ? 40 : sh)) : (d >> (-sh > 62 ? 62 : -sh));
@@ -838,47 +1022,51 @@ __global__ __launch_bounds__(RL_ATT_T) void k_rl_attn(RtlArgs a) {
     xs[t] = v;
     part += v;
   }
-  const long long tot = block_sum_ll(part, red_l);
-  if (tid == 0) {
-    const int msb = tot ? 63 - __clzll((unsigned long long)tot) : 0;
-    __int128 y = (__int128)1 << (31 - msb);
-    for (int it = 0; it < 4; ++it) y = (y * (((__int128)1 << 33) - (__int128)tot * y)) >> 32;
-    s_inv = (long long)y;
+  part = psum<8>(part);
+  part = psum<4>(part);
+  part = psum<2>(part);
+  part = psum<1>(part);
+  part = psum<16>(part);
+  part = psum<32>(part);
+  if (ln == 0) red_s[wv] = part;
+  lds_barrier();
+  if (tid >= 64) return;
+  const int c = tid >> 4, l = tid & 15;
+  // 16 rows, every load issued before the first is used; p is 0 past kv_pos
+  int vr[16], vt[16];
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    const size_t slot = (size_t)(t < kv ? t : 0) * L.H_KV + g;
+    vr[t] = L.v_m[slot * HD + c * 16 + l];
+    vt[t] = L.v_e[slot * 4 + c];
   }
-  __syncthreads();
-  const long long inv = s_inv;
-  int ml = 0;
-  for (int t = tid; t < n; t += RL_ATT_T) {
-    const long long p = (long long)xs[t] * inv;
-    const int l = p ? lead64(p) : 0;
-    ml = l > ml ? l : ml;
-  }
-  ml = block_max_i(ml, red_i);
+  long long tot = 0;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) tot += red_s[i];
+  const int msb = tot ? 63 - __clzll((unsigned long long)tot) : 0;
+  __int128 y = (__int128)1 << (31 - msb);
+  for (int it = 0; it < 4; ++it) y = (y * (((__int128)1 << 33) - (__int128)tot * y)) >> 32;
+  const long long inv = (long long)y;
+  // the largest product's leading bit: the table rises, and the largest score
+  // (difference 0) takes its last entry
+  const long long pmax_ = (long long)a.exp_lut[1023] * inv;
+  const int ml = pmax_ ? lead64(pmax_) : 0;
   if (tid < 16) {
     int s2;
     pm[tid] = tid < n ? norm16((long long)xs[tid] * inv, ml, s2) : 0;
   }
-  if (tid == 0) s_pe = clamp8(ml - 14 - 17);
-  // V exponent max per 16-dim chunk over t <= kv_pos
-  int vm4[4] = {-128, -128, -128, -128};
-  for (int t = tid; t < n; t += RL_ATT_T) {
-    const int8_t *ve = L.v_e + ((size_t)t * L.H_KV + g) * 4;
-    for (int c = 0; c < 4; ++c) vm4[c] = ve[c] > vm4[c] ? ve[c] : vm4[c];
-  }
-  for (int c = 0; c < 4; ++c) {
-    const int v = block_max_i(vm4[c], red_i);
-    if (tid == 0) s_vmax[c] = v;
-  }
-  __syncthreads();
-  if (tid >= 64) return;
-  const int c = tid >> 4, l = tid & 15;
-  const int vmax = s_vmax[c];
-  const int nav = n < 16 ? n : 16;
+  const int s_pe = clamp8(ml - 14 - 17);
+  int vmax = red_v[c];
+#pragma unroll
+  for (int i = 1; i < NW; ++i) vmax = red_v[4 * i + c] > vmax ? red_v[4 * i + c] : vmax;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
   long long s = 0;
-  for (int t = 0; t < nav; ++t) {
-    const size_t slot = (size_t)t * L.H_KV + g;
-    const int vt = L.v_e[slot * 4 + c];
-    s += (long long)pm[t] * shr8(L.v_m[slot * HD + c * 16 + l], vmax, vt);
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    const int v = t < kv ? vr[t] : vc[c * 16 + l], ve = t < kv ? vt[t] : vce[c];
+    s += (long long)(pm[t] * shr8(v, vmax, ve));
   }
   int sh2;
   const int m = norm16(s, lead64(s), sh2);
@@ -897,27 +1085,20 @@ __global__ __launch_bounds__(RL_ATT_T) void k_rl_attn(RtlArgs a) {
 // gamma from its ROM, i.e. tile_quantize'd), then per 16-row chunk of the
 // tied embedding the matvec engine (S_MV_*), whose per-lane (m, e) feed the
 // bfp_gt running argmax (S_MV_LANE_CMP / S_MV_MERGE, k_rtl_argmax).
-__global__ __launch_bounds__(64) void k_rl_head_norm(RtlHeadArgs a) {
+__global__ __launch_bounds__(RMS_T) void k_rl_head_norm(RtlHeadArgs a) {
   extern __shared__ long long rl_lds[];
-  __shared__ long long s_inv;
-  __shared__ int s_einv;
-  const int D = a.D, nt = D / 16, tid = threadIdx.x;
-  long long *sums = rl_lds;
-  int16_t *gm = reinterpret_cast<int16_t *>(rl_lds + nt);
-  int8_t *ge = reinterpret_cast<int8_t *>(gm + D);
-  for (int base = 0; base < D; base += 64) {   // D % 64 == 0: whole 16-lane tiles
-    const int i = base + tid;
-    int e;
-    const int m = quantize16_lanes(a.norm_w[i], e);
-    gm[i] = (int16_t)m;
-    if ((i & 15) == 0) ge[i >> 4] = (int8_t)e;
-  }
-  __syncthreads();
-  rmsnorm_wave(a.h_m, a.h_e, gm, ge, D, a.xn_m, a.xn_e, sums, &s_inv, &s_einv);
+  const int nt = a.D / 16;
+  rms_block(a.h_m, a.h_e, RomGamma{a.norm_w}, a.D, rl_lds, reinterpret_cast<int *>(rl_lds + nt),
+            [&](int i, int m, int e) {
+              if (i >= a.D) return;
+              a.xn_m[i] = (int16_t)m;
+              if ((i & 15) == 0) a.xn_e[i >> 4] = (int8_t)e;
+            });
 }
 
 // One 16-row chunk of the embedding per workgroup: the engine's per-row
-// (m, e) into lg_m / lg_e.
+// (m, e) into lg_m / lg_e, and the chunk's best (lane 0 seeds, the next
+// lane that is greater replaces) into work[chunk].
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_rl_head_mv(RtlHeadArgs a) {
   constexpr int TPT = 3;
@@ -927,15 +1108,28 @@ __global__ __launch_bounds__(64 * NW) void k_rl_head_mv(RtlHeadArgs a) {
   int *El = reinterpret_cast<int *>(Sl + nT * 16);
   int *xs = El + nT * 16;
   int *xes = xs + nT * 16;
+  ChunkRegs<TPT> R[1];
+  load_chunk_nb<NW, TPT>(R[0], a.emb_m + (size_t)c * nT * 32, a.emb_e + (size_t)c * nT * 16, nT);
   stage_x_bfp(xs, xes, a.xn_m, a.xn_e, nT);
-  __syncthreads();
+  lds_barrier();
   int m, e;
-  rl_chunk_me<NW, TPT>(a.emb_m + (size_t)c * nT * 32, a.emb_e + (size_t)c * nT * 16, nT, xs, xes,
-                       Sl, El, m, e);
+  rl_chunk_me<NW, TPT, 1>(R, nT, xs, xes, Sl, El, m, e);
+  if (threadIdx.x >= 64) return;
   if (threadIdx.x < 16) {
     a.lg_m[c * 16 + threadIdx.x] = (int16_t)m;
     a.lg_e[c * 16 + threadIdx.x] = (int8_t)e;
   }
+  int bm = __builtin_amdgcn_readlane(m, 0), be = __builtin_amdgcn_readlane(e, 0), bk = 0;
+  unsigned rest = 0xfffeu;
+  for (;;) {
+    const unsigned gt = (unsigned)__ballot(bfp_gt(m, e, bm, be)) & rest;
+    if (!gt) break;
+    bk = __builtin_ctz(gt);
+    bm = __builtin_amdgcn_readlane(m, bk);
+    be = __builtin_amdgcn_readlane(e, bk);
+    rest &= ~0u << (bk + 1);
+  }
+  if (threadIdx.x == 0) a.work[c] = arg_word(bm, be, bk);
 }
 
 // One step of the FPGA driver's token loop on the device
@@ -1053,7 +1247,7 @@ int bfp_rtl_rmsnorm_d(const int16_t *x_m, const int8_t *x_e, const int16_t *g_m,
                       int D, int batch, int16_t *y_m, int8_t *y_e, void *stream) {
   if (D <= 0 || D % 16 || D > 65536 || batch <= 0)
     return set_err(BFP_EINVAL, "rtl_rmsnorm: D=%d batch=%d", D, batch);
-  hipLaunchKernelGGL(rtl::k_rtl_rmsnorm, dim3(batch), dim3(64), (size_t)(D / 16) * 8,
+  hipLaunchKernelGGL(rtl::k_rtl_rmsnorm, dim3(batch), dim3(rtl::RMS_T), (size_t)(D / 16) * 12,
                      (hipStream_t)stream, x_m, x_e, g_m, g_e, D, y_m, y_e);
   return launch_status("rtl_rmsnorm");
 }
@@ -1107,8 +1301,7 @@ int bfp_rtl_argmax_static_d(const int16_t *m, const int8_t *e, int n, int batch,
                    nc, bfp::ARGMAX_STATIC_CHUNKS);
   int *w = nullptr;
   BFP_TRY(bfp::argmax_scratch(&w));
-  hipLaunchKernelGGL(rtl::k_rtl_argmax, dim3(batch), dim3(256), 0, (hipStream_t)stream, m, e, n, w,
-                     w + nc, w + 2 * nc, idx);
+  hipLaunchKernelGGL(rtl::k_rtl_argmax, dim3(batch), dim3(rtl::ARGMAX_T), 0, (hipStream_t)stream, m, e, n, w, idx);
   return launch_status("rtl_argmax_static");
 }
 
@@ -1116,9 +1309,8 @@ int bfp_rtl_argmax_static_d(const int16_t *m, const int8_t *e, int n, int batch,
 int bfp_rtl_argmax_d(const int16_t *m, const int8_t *e, int n, int batch, int32_t *work,
                      int32_t *idx, void *stream) {
   if (n <= 0 || n % 16 || batch <= 0 || !work) return set_err(BFP_EINVAL, "rtl_argmax: n=%d", n);
-  const long long nc = (long long)batch * (n / 16);
-  hipLaunchKernelGGL(rtl::k_rtl_argmax, dim3(batch), dim3(256), 0, (hipStream_t)stream, m, e, n,
-                     work, work + nc, work + 2 * nc, idx);
+  hipLaunchKernelGGL(rtl::k_rtl_argmax, dim3(batch), dim3(rtl::ARGMAX_T), 0, (hipStream_t)stream, m, e, n,
+                     work, idx);
   return launch_status("rtl_argmax");
 }
 
@@ -1127,20 +1319,22 @@ int bfp_rtl_argmax_d(const int16_t *m, const int8_t *e, int n, int batch, int32_
 namespace bfp {
 
 namespace {
-typedef void (*rl_mv_fn)(RtlArgs, int);
+typedef void (*rl_mv_fn)(RtlArgs);
+template <int OP>
 rl_mv_fn rl_mv_kernel(int nw) {
-  static const rl_mv_fn k[9] = {rtl::k_rl_mv<1>, rtl::k_rl_mv<2>, rtl::k_rl_mv<3>,
-                                rtl::k_rl_mv<4>, rtl::k_rl_mv<5>, rtl::k_rl_mv<6>,
-                                rtl::k_rl_mv<7>, rtl::k_rl_mv<8>, rtl::k_rl_mv<9>};
+  static const rl_mv_fn k[9] = {rtl::k_rl_mv<1, OP>, rtl::k_rl_mv<2, OP>, rtl::k_rl_mv<3, OP>,
+                                rtl::k_rl_mv<4, OP>, rtl::k_rl_mv<5, OP>, rtl::k_rl_mv<6, OP>,
+                                rtl::k_rl_mv<7, OP>, rtl::k_rl_mv<8, OP>, rtl::k_rl_mv<9, OP>};
   return nw >= 1 && nw <= 9 ? k[nw - 1] : nullptr;
 }
 
 // One matvec op of the layer: nT input tiles, n_wg output chunks.
-int rl_mv(const RtlArgs &a, int op, int nT, int n_wg, hipStream_t s) {
+template <int OP>
+int rl_mv(const RtlArgs &a, int nT, int n_wg, hipStream_t s) {
   const int nw = (nT + 11) / 12;   // 3 tiles per lane, 4 tile lanes per wave
-  rl_mv_fn f = rl_mv_kernel(nw);
+  rl_mv_fn f = rl_mv_kernel<OP>(nw);
   if (!f) return set_err(BFP_EINVAL, "rtl layer: %d input tiles unsupported", nT);
-  hipLaunchKernelGGL(f, dim3(n_wg), dim3(64 * nw), (size_t)nT * 260, s, a, op);
+  hipLaunchKernelGGL(f, dim3(n_wg), dim3(64 * nw), (size_t)nT * ((OP == 2 ? 2 : 1) * 192 + 80), s, a);
   return launch_status("rtl layer matvec");
 }
 }  // namespace
@@ -1154,19 +1348,12 @@ int launch_rtl_layer(const RtlArgs &a, hipStream_t s) {
     return set_err(BFP_EINVAL, "rtl layer: batch %d, HD %d, pos %d, kv_pos %d (capacity %d)",
                    L.batch, L.HD, a.pos, a.kv_pos, L.max_ctx);
   const int n_att = a.pos_ptr ? L.max_ctx : a.kv_pos + 1;   // positions the attention's LDS holds
-  const size_t lds_norm = (size_t)ntD * 9 + (size_t)L.D * 2;
-  hipLaunchKernelGGL(rtl::k_rl_norm, dim3(1), dim3(64), lds_norm, s, a, 0);
-  BFP_TRY(launch_status("rtl layer norm1"));
-  BFP_TRY(rl_mv(a, 0, ntD, (L.D + 2 * L.KV) / 16, s));
-  hipLaunchKernelGGL(rtl::k_rl_rope_kv, dim3(L.H_Q + L.H_KV), dim3(64), 0, s, a);
-  BFP_TRY(launch_status("rtl layer rope"));
+  BFP_TRY(rl_mv<0>(a, ntD, (L.D + 2 * L.KV) / 16, s));
   hipLaunchKernelGGL(rtl::k_rl_attn, dim3(L.H_Q), dim3(rtl::RL_ATT_T), (size_t)n_att * 8, s, a);
   BFP_TRY(launch_status("rtl layer attention"));
-  BFP_TRY(rl_mv(a, 1, ntD, ntD, s));
-  hipLaunchKernelGGL(rtl::k_rl_norm, dim3(1), dim3(64), lds_norm, s, a, 1);
-  BFP_TRY(launch_status("rtl layer norm2"));
-  BFP_TRY(rl_mv(a, 2, ntD, ntF, s));
-  return rl_mv(a, 3, ntF, ntD, s);
+  BFP_TRY(rl_mv<1>(a, ntD, ntD, s));
+  BFP_TRY(rl_mv<2>(a, ntD, ntF, s));
+  return rl_mv<3>(a, ntF, ntD, s);
 }
 
 int launch_rtl_ctl(const RtlCtlArgs &a, hipStream_t s) {
@@ -1185,13 +1372,11 @@ int launch_rtl_head(const RtlHeadArgs &a, hipStream_t s) {
                              rtl::k_rl_head_mv<7>, rtl::k_rl_head_mv<8>, rtl::k_rl_head_mv<9>};
   const int nw = (nT + 11) / 12;   // 3 tiles per lane, 4 tile lanes per wave
   if (nw > 9) return set_err(BFP_EINVAL, "rtl head: %d input tiles unsupported", nT);
-  hipLaunchKernelGGL(rtl::k_rl_head_norm, dim3(1), dim3(64), (size_t)nT * 9 + (size_t)a.D * 2, s, a);
+  hipLaunchKernelGGL(rtl::k_rl_head_norm, dim3(1), dim3(rtl::RMS_T), (size_t)nT * 12, s, a);
   BFP_TRY(launch_status("rtl head norm"));
   hipLaunchKernelGGL(k[nw - 1], dim3(a.VOCAB / 16), dim3(64 * nw), (size_t)nT * 260, s, a);
   BFP_TRY(launch_status("rtl head matvec"));
-  const long long nc = a.VOCAB / 16;
-  hipLaunchKernelGGL(rtl::k_rtl_argmax, dim3(1), dim3(256), 0, s, a.lg_m, a.lg_e, a.VOCAB, a.work,
-                     a.work + nc, a.work + 2 * nc, a.token);
+  hipLaunchKernelGGL(rtl::k_rl_argmax_fold, dim3(1), dim3(64), 0, s, a.work, a.VOCAB / 16, a.token);
   return launch_status("rtl head argmax");
 }
 
