@@ -335,8 +335,8 @@ int bfp_rtl_decode(bfp_ctx *ctx, const int32_t *prompt, int n_prompt, int n_gen,
                    int16_t *hist_m, int8_t *hist_e);
 
 /* Decode head (full.py:438-440): final norm, float64 logits over the raw
- * embedding, first-index argmax.  logits may be NULL: then, from 32
- * sequences on (contexts made with max_batch >= 32), the argmax comes from
+ * embedding, first-index argmax.  logits may be NULL: then, from 2
+ * sequences on (D at most 576), the argmax comes from
  * the bounded head, which forms float64 logits only for the rows that can
  * hold the largest (an exact int16 dot product brackets every logit) and
  * returns the same index; the environment variable BFP_HEAD_BOUNDED=0
@@ -400,8 +400,7 @@ int bfp_decode(bfp_ctx *ctx, const int32_t *prompt, int n_prompt, int n_gen, int
 int bfp_decode_path(const bfp_ctx *ctx);
 /* The launch form of the last bfp_decode's layers (no reference
  * counterpart; for tests and tuning): BFP_FORM_SINGLE (per-sequence stage
- * kernels, batches below 4), BFP_FORM_MULTI (multi-sequence kernels on the
- * vector unit), or BFP_FORM_MX (int8 matrix-core matvecs) with
+ * kernels, batches below 16), or BFP_FORM_MX (int8 matrix-core matvecs) with
  * BFP_FORM_QKV_ATTN when Q|K|V and attention ran as one launch (with
  * BFP_FORM_ATT_GROUP when its attention workgroups each took a whole KV
  * group's query heads: contexts of at most 256, the default; the environment
@@ -410,7 +409,7 @@ int bfp_decode_path(const bfp_ctx *ctx);
  * BFP_FORM_PERSIST for the persistent batch-1 decode, BFP_FORM_PIPE for the
  * pipelined batched step; -1 before any decode. */
 #define BFP_FORM_SINGLE 0
-#define BFP_FORM_MULTI 1
+#define BFP_FORM_MULTI 1 /* no longer taken */
 #define BFP_FORM_MX 2
 #define BFP_FORM_QKV_ATTN 4
 #define BFP_FORM_NORM_FUSED 8

@@ -403,3 +403,50 @@ def test_batched_trace(gpu):
         assert len(st) == chunks[k] * groups, (k, len(st))
         assert (np.diff(st, axis=1) >= 0).all(), k
     gm.close()
+
+
+@pytest.mark.parametrize("batch", [2, 15, 16, 17, 31])
+def test_head_bounded_small_batches(gpu, batch):
+    """The bounded head below 32 sequences (one sequence group up to 16, four
+    above) against the full head's logits, with ties within and across
+    blocks, a zero block, an all-zero hidden state and a short last block of
+    workgroups."""
+    from bfp import Dims, synth
+    from bfp.model import BfpModel
+    d = Dims(D=192, H_Q=3, H_KV=1, HD=64, FFN=256, NL=1, MAX_CTX=8, VOCAB=1040)
+    fm = synth.make_model(d, seed=batch)
+    E = fm.embed
+    E[5] = E[9] = E[7] * np.float32(60.0)
+    E[40] = -E[5]
+    E[200:216] = 0.0
+    E[101] = np.nextafter(E[100], np.float32(np.inf))
+    gm = BfpModel(d, max_batch=batch)
+    gm.load_fp32(fm)
+    rng = np.random.default_rng(batch)
+    hs = [rng.standard_normal(d.D) * (0.3 + 0.1 * b) for b in range(batch)]
+    hs[0] = np.zeros(d.D)
+    hs[-1] = E[100].astype(np.float64) * 40.0
+    q = [sim.tile_quantize(h) for h in hs]
+    hm, he = np.stack([x[0].reshape(-1) for x in q]), np.stack([x[1] for x in q])
+    full, lg = gm.head(hm, he, logits=True)
+    am, _ = gm.head(hm, he)
+    assert list(full) == [int(np.argmax(r)) for r in lg]
+    assert list(am) == list(full) and am[0] == 0
+    gm.close()
+
+
+@pytest.mark.parametrize("batch", [2, 7, 15, 16])
+def test_decode_small_batches(gpu, batch):
+    """Batches on the per-sequence kernels (below 16) and the first on the
+    matrix cores: layer outputs at every step and tokens of the first and
+    last sequences equal the oracle's."""
+    d, om, gm = _setup(dict(TINY, D=192, H_Q=3, FFN=272), seed=batch, max_batch=batch)
+    from bfp import synth
+    prompts = np.stack([synth.make_prompt(d, 3, seed=800 + b) for b in range(batch)])
+    toks, (hm, he) = gm.decode(prompts, 6, hist=True)
+    assert gm.decode_form() == "single" if batch < 16 else gm.decode_form().startswith("mx")
+    for b in (0, batch - 1):
+        want, whm, whe = _oracle_decode(om, prompts[b], 6)
+        assert list(toks[b]) == list(want)
+        assert np.array_equal(hm[b], whm) and np.array_equal(he[b], whe)
+    gm.close()

@@ -307,7 +307,7 @@ class BfpModel:
 
     def decode_form(self):
         """How the last decode's layers were launched: 'persist', 'pipe' (the
-        pipelined batched step), 'single', 'multi', or 'mx' followed by
+        pipelined batched step), 'single' (batches below 16), or 'mx' followed by
         '+qkv_attn' (Q|K|V and attention in one launch), '+attn_group' (its
         attention a KV group per workgroup) and '+norm_fused' (RMSNorms
         inside the O and D launches)."""

@@ -58,7 +58,7 @@ struct bfp_ctx {
   float *embed = nullptr;
   float *embedp = nullptr;     // the embedding permuted per row for the batched head
                                // (made when max_batch >= HEAD_SEQ_MIN)
-  // the bounded head (made with embedp): the embedding as split int16 with
+  // the bounded head (made when max_batch >= HEADQ_MIN): the embedding as split int16 with
   // per-row meta, and per step the quantised hidden, its per-sequence
   // record and the per-block bounds
   uint4 *embq = nullptr, *hq_x = nullptr;
@@ -68,7 +68,7 @@ struct bfp_ctx {
   // activations (max_batch sequences)
   int16_t *h_m = nullptr, *h1_m = nullptr, *qkv_am = nullptr, *att_m = nullptr, *mlp_m = nullptr;
   int8_t *h_e = nullptr, *h1_e = nullptr, *qkv_ae = nullptr, *att_e = nullptr, *mlp_e = nullptr;
-  int16_t *xn_m = nullptr;   // RMSNorm output, multi-sequence layer path
+  int16_t *xn_m = nullptr;   // RMSNorm output, matrix-core layer path
   int8_t *xn_e = nullptr;
   double *hn = nullptr;      // normed final hidden, batch > 1 head
   // KV cache: NL x max_batch x max_ctx x KV
@@ -221,12 +221,14 @@ int head_part_max(const bfp_ctx *c) {
   return m;
 }
 
-// The bounded head (argmax only) where its copy exists, no logits are asked
-// for and the batch takes the float64 matrix-core form; BFP_HEAD_BOUNDED=0
-// keeps k_head_mx.
+// The bounded head (argmax only) where its copy exists and no logits are
+// asked for, from HEADQ_MIN sequences; BFP_HEAD_BOUNDED=0 keeps the full
+// head.  (Below HEAD_SEQ_MIN sequences a vocabulary too large for the pick's
+// candidate list takes the full head too.)
 bool head_bounded(const bfp_ctx *c, int batch, const double *logits) {
   const char *v = getenv("BFP_HEAD_BOUNDED");
-  return c->embq && !logits && head_seq_form(c->d.D, batch, c->embedp != nullptr) && !(v && atoi(v) == 0);
+  return c->embq && !logits && batch >= HEADQ_MIN && !(v && atoi(v) == 0) &&
+         (batch >= HEAD_SEQ_MIN || headq_pick_lds(c->d.D, c->d.VOCAB) <= 64 * 1024);
 }
 
 HeadArgs head_args(bfp_ctx *c, int batch, double *logits) {
@@ -666,8 +668,9 @@ bfp_ctx *bfp_create(const bfp_dims *dims, int device, int max_batch) {
       (rc = c->alloc((void **)&c->rope_row, sizeof(double) * d.HD)) ||
       (rc = c->alloc((void **)&c->embed, sizeof(float) * (size_t)d.VOCAB * d.D)) ||
       (max_batch >= HEAD_SEQ_MIN && d.D % 64 == 0 && d.D <= 576 &&
-       ((rc = c->alloc((void **)&c->embedp, sizeof(float) * (size_t)d.VOCAB * d.D)) ||
-        (rc = c->alloc((void **)&c->embq, (size_t)d.VOCAB * d.D * 2)) ||
+       (rc = c->alloc((void **)&c->embedp, sizeof(float) * (size_t)d.VOCAB * d.D))) ||
+      (max_batch >= HEADQ_MIN && d.D % 64 == 0 && d.D <= 576 &&
+       ((rc = c->alloc((void **)&c->embq, (size_t)d.VOCAB * d.D * 2)) ||
         (rc = c->alloc((void **)&c->embq_meta, sizeof(HeadQRow) * (size_t)d.VOCAB)) ||
         (rc = c->alloc((void **)&c->hq_x, (size_t)(B + 15) / 16 * (d.D / 64) * 64 * 32)) ||
         (rc = c->alloc((void **)&c->hq_seq, sizeof(HeadQSeq) * B)) ||
@@ -858,9 +861,9 @@ int bfp_load_weights(bfp_ctx *c, int which, int layer, const float *fp32, const 
         hipLaunchKernelGGL(permute_embed_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                            s, c->embed, n, d.D, c->embedp);
         BFP_TRY(launch_status("embed permute"));
-        BFP_TRY(launch_embq_build(c->embed, d.VOCAB, d.D, c->embq, c->embq_meta, s));
-        HIP_TRY(hipStreamSynchronize(s));
       }
+      if (c->embq) BFP_TRY(launch_embq_build(c->embed, d.VOCAB, d.D, c->embq, c->embq_meta, s));
+      if (c->embedp || c->embq) HIP_TRY(hipStreamSynchronize(s));
       return BFP_OK;
     }
     default:

@@ -43,7 +43,7 @@ struct LayerArgs {
   int16_t *qkv_m; int8_t *qkv_e;   // D + 2KV, pre-rope
   int16_t *att_m; int8_t *att_e;   // D
   int16_t *mlp_m; int8_t *mlp_e;   // FFN
-  int16_t *xn_m;  int8_t *xn_e;    // D, RMSNorm output (multi-sequence path)
+  int16_t *xn_m;  int8_t *xn_e;    // D, RMSNorm output (matrix-core path)
   // this layer's KV cache: sequence b, position t, kv head g at
   // ((b*max_ctx + t)*H_KV + g)*HD mantissas and /16 exponents
   int16_t *k_m; int8_t *k_e;
@@ -144,9 +144,13 @@ struct HeadArgs {
   double2 *hq_blk;                         // (batch, VOCAB / 16) per 16-row block: max lower, max upper bound
 };
 
-// The bounded head runs from HEAD_SEQ_MIN sequences (with the permuted
-// copy's conditions, D % 64 == 0 and D <= 576) unless logits are asked for.
-constexpr int HEADQ_SEQ = 64;   // sequences per k_headq_mx workgroup
+// The bounded head runs from HEADQ_MIN sequences (D % 64 == 0 and D <= 576)
+// unless logits are asked for.  Against the full head over all rows, 30 layers
+// and 23 + 25 tokens: 2 sequences 23.6 / 24.1 ms, 5 26.1 / 27.2, 16 44.6 / 45.9,
+// 24 48.5 / 50.0.
+constexpr int HEADQ_MIN = 2;
+constexpr int HEADQ_SEQ = 64;   // most sequences per k_headq_mx workgroup
+inline size_t headq_pick_lds(int D, int VOCAB) { return (size_t)D * 8 + (size_t)(VOCAB / 16) * 4; }
 
 // Batches from HEAD_SEQ_MIN sequences on run the head on the float64 matrix
 // cores (k_head_mx), when the embedding's permuted copy exists and

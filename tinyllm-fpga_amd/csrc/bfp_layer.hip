@@ -29,14 +29,43 @@
 
 namespace bfp {
 
+// The RMSNorm prologue of k_qkv and k_gu: n = tile_quantize(rmsnorm_fp(x, g))
+// into the matvec's LDS input form (and the stage dump dm / de).  PAIRS:
+// thread t on elements 2t, 2t + 1 (rmsnorm_pairs; D <= 128 NW), the squares'
+// sum formed by each wave alone; else one thread per up to 4 elements
+// (rmsnorm_to_x) with the block-wide sum.  dsm: norm_prologue_doubles
+// doubles of LDS.
+__host__ __device__ inline int norm_prologue_doubles(bool pairs, int D) {
+  return (pairs ? D : 3 * D) + PW_MAX_LEAVES;
+}
+template <bool PAIRS>
+__device__ __forceinline__ void norm_prologue(const int16_t *hm, const int8_t *he, const double *g, int D, int *xs,
+                                              int *xes, double *dsm, int16_t *dm, int8_t *de) {
+  if constexpr (PAIRS) {
+    const int i0 = 2 * (int)threadIdx.x;
+    const double2 gg = *reinterpret_cast<const double2 *>(g + (i0 < D ? i0 : 0));
+    int m0, m1, e;
+    rmsnorm_pairs(hm, he, gg.x, gg.y, D, dsm, dsm + D, m0, m1, e);
+    if (i0 < D) {
+      put_x_pair(xs, i0 >> 4, (i0 >> 1) & 7, m0, m1);
+      if ((i0 & 15) == 0) xes[i0 >> 4] = e;
+      if (dm) {
+        dm[i0] = (int16_t)m0;
+        dm[i0 + 1] = (int16_t)m1;
+        if ((i0 & 15) == 0) de[i0 >> 4] = (int8_t)e;
+      }
+    }
+  } else {
+    rmsnorm_to_x(hm, he, g, D, xs, xes, dsm, dsm + 3 * D, dm, de);
+  }
+}
+
 // ------------------------------------------------------------------- qkv
-template <int NW, int TPT>
+template <int NW, int TPT, bool PAIRS>
 __global__ __launch_bounds__(64 * NW) void k_qkv(LayerArgs a) {
   extern __shared__ double dsm[];
   const int nT = a.D / 16;
-  double *dbuf = dsm;                                   // 3*D
-  double *leaf = dsm + 3 * a.D;                         // PW_MAX_LEAVES
-  int *xs = reinterpret_cast<int *>(leaf + PW_MAX_LEAVES);   // nT*16
+  int *xs = reinterpret_cast<int *>(dsm + norm_prologue_doubles(PAIRS, a.D));   // nT*16
   int *xes = xs + nT * 16;                              // nT
   __shared__ int redM[NW * 16];
   __shared__ long long redA[NW * 16];
@@ -50,8 +79,8 @@ __global__ __launch_bounds__(64 * NW) void k_qkv(LayerArgs a) {
     dm = a.dump->m[ST_N1] + b * a.dump->mstride[ST_N1];
     de = a.dump->e[ST_N1] + b * (a.dump->mstride[ST_N1] / 16);
   }
-  rmsnorm_to_x(a.h_m + b * a.D, a.h_e + b * (a.D / 16), a.g1, a.D, xs, xes, dbuf, leaf, dm, de);
-  __syncthreads();
+  norm_prologue<PAIRS>(a.h_m + b * a.D, a.h_e + b * (a.D / 16), a.g1, a.D, xs, xes, dsm, dm, de);
+  lds_barrier();
   long long A;
   int M;
   chunk_AM<NW, TPT>(R, xs, xes, nT, redM, redA, A, M);
@@ -98,13 +127,11 @@ __global__ __launch_bounds__(64 * NW) void k_o_res(LayerArgs a) {
 }
 
 // -------------------------------------------------------------------- gu
-template <int NW, int TPT>
+template <int NW, int TPT, bool PAIRS>
 __global__ __launch_bounds__(64 * NW) void k_gu(LayerArgs a) {
   extern __shared__ double dsm[];
   const int nT = a.D / 16;
-  double *dbuf = dsm;             // 3*D
-  double *leaf = dsm + 3 * a.D;
-  int *xs = reinterpret_cast<int *>(leaf + PW_MAX_LEAVES);
+  int *xs = reinterpret_cast<int *>(dsm + norm_prologue_doubles(PAIRS, a.D));
   int *xes = xs + nT * 16;
   __shared__ int redM[2 * NW * 16];
   __shared__ long long redA[2 * NW * 16];
@@ -120,8 +147,8 @@ __global__ __launch_bounds__(64 * NW) void k_gu(LayerArgs a) {
     dm = a.dump->m[ST_N2] + b * a.dump->mstride[ST_N2];
     de = a.dump->e[ST_N2] + b * (a.dump->mstride[ST_N2] / 16);
   }
-  rmsnorm_to_x(a.h1_m + b * a.D, a.h1_e + b * (a.D / 16), a.g2, a.D, xs, xes, dbuf, leaf, dm, de);
-  __syncthreads();
+  norm_prologue<PAIRS>(a.h1_m + b * a.D, a.h1_e + b * (a.D / 16), a.g2, a.D, xs, xes, dsm, dm, de);
+  lds_barrier();
   long long Ag, Au;
   int Mg, Mu;
   chunk_AM2<NW, TPT>(RG, RU, xs, xes, nT, redM, redA, Ag, Mg, Au, Mu);   // G and U in one pass
@@ -152,12 +179,11 @@ __global__ __launch_bounds__(64 * NW) void k_d_res(LayerArgs a) {
 
 
 // ------------------------------------------------- multi-sequence kernels
-// For batch >= MULTI_MIN_BATCH the layer runs as norm -> matvec kernels in
-// which a workgroup keeps its weight chunk in registers and loops over S
-// sequences (grid.y = sequence groups), so weights are fetched once per
-// group rather than once per sequence, and each RMSNorm is computed once per
-// sequence rather than once per chunk.  Same arithmetic as the fused
-// kernels: the outputs are bit-identical.
+// For batches on the matrix cores and the rows of a prompt pass the layer
+// runs as norm -> matvec kernels: each RMSNorm is computed once per sequence
+// rather than once per chunk, and weights are fetched once per group of
+// sequences.  Same arithmetic as the fused kernels: the outputs are
+// bit-identical.
 
 // n = tile_quantize(rmsnorm_fp(x, gamma)) of sequence blockIdx.x into xn
 // (which = 1: h with g1 -> N1; which = 2: h1 with g2 -> N2).
@@ -233,108 +259,9 @@ static void launch_norm_seq(const LayerArgs &a, int which, hipStream_t s) {
   }
 }
 
-constexpr int MSEQ = 8;   // sequences per workgroup of the multi-sequence matvecs
-
-// The epilogue of a multi-sequence chunk: wave 0, four sequences per pass
-// (one per 16-lane group).
-#define BFP_MULTI_EPI(CALL)                                                       \
-  if (threadIdx.x < 64) {                                                         \
-    const int r_ = threadIdx.x & 15;                                              \
-    for (int p_ = 0; p_ < ns; p_ += 4) {                                          \
-      const int s_ = p_ + (threadIdx.x >> 4);                                     \
-      const bool wr_ = s_ < ns;                                                   \
-      const int sc_ = wr_ ? s_ : 0;                                               \
-      const int b = b0 + sc_;                                                     \
-      CALL;                                                                       \
-    }                                                                             \
-  }
-
-template <int NW, int TPT>
-__global__ __launch_bounds__(64 * NW) void k_qkv_m(LayerArgs a) {
-  extern __shared__ int ism[];
-  const int nT = a.D / 16;
-  int *xs = ism;
-  int *xes = ism + MSEQ * nT * 16;
-  __shared__ int redM[NW * 16 * MSEQ];
-  __shared__ long long redA[NW * 16 * MSEQ];
-  __shared__ long long Ao[16 * MSEQ];
-  __shared__ int Mo[16 * MSEQ];
-  const int c = blockIdx.x, b0 = blockIdx.y * MSEQ, ns = min(MSEQ, a.batch - b0);
-  ChunkRegs<TPT> R;
-  load_chunk<NW, TPT>(R, a.w_qkv_m + (long long)c * nT * 32, a.w_qkv_e + (long long)c * nT * 16, nT);
-  stage_x_bfp(xs, xes, a.xn_m + b0 * a.D, a.xn_e + b0 * (a.D / 16), ns * nT);
-  __syncthreads();
-  chunk_AM_multi<NW, TPT, MSEQ>(R, xs, xes, nT, ns, redM, redA, Ao, Mo);
-  BFP_MULTI_EPI(epi_qkv(a, b, c, Ao[r_ * MSEQ + sc_], Mo[r_ * MSEQ + sc_], wr_))
-}
-
-template <int NW, int TPT>
-__global__ __launch_bounds__(64 * NW) void k_o_res_m(LayerArgs a) {
-  extern __shared__ int ism[];
-  const int nT = a.D / 16;
-  int *xs = ism;
-  int *xes = ism + MSEQ * nT * 16;
-  __shared__ int redM[NW * 16 * MSEQ];
-  __shared__ long long redA[NW * 16 * MSEQ];
-  __shared__ long long Ao[16 * MSEQ];
-  __shared__ int Mo[16 * MSEQ];
-  const int c = blockIdx.x, b0 = blockIdx.y * MSEQ, ns = min(MSEQ, a.batch - b0);
-  ChunkRegs<TPT> R;
-  load_chunk<NW, TPT>(R, a.w_o_m + (long long)c * nT * 32, a.w_o_e + (long long)c * nT * 16, nT);
-  stage_x_bfp(xs, xes, a.att_m + b0 * a.D, a.att_e + b0 * (a.D / 16), ns * nT);
-  __syncthreads();
-  chunk_AM_multi<NW, TPT, MSEQ>(R, xs, xes, nT, ns, redM, redA, Ao, Mo);
-  BFP_MULTI_EPI(epi_ores(a, b, c, Ao[r_ * MSEQ + sc_], Mo[r_ * MSEQ + sc_], wr_,
-                         a.h_m[b * a.D + c * 16 + r_], a.h_e[b * (a.D / 16) + c]))
-}
-
-template <int NW, int TPT>
-__global__ __launch_bounds__(64 * NW) void k_gu_m(LayerArgs a) {
-  extern __shared__ int ism[];
-  const int nT = a.D / 16;
-  int *xs = ism;
-  int *xes = ism + MSEQ * nT * 16;
-  __shared__ int redM[NW * 16 * MSEQ];
-  __shared__ long long redA[NW * 16 * MSEQ];
-  __shared__ long long Aog[16 * MSEQ], Aou[16 * MSEQ];
-  __shared__ int Mog[16 * MSEQ], Mou[16 * MSEQ];
-  const int c = blockIdx.x, b0 = blockIdx.y * MSEQ, ns = min(MSEQ, a.batch - b0);
-  ChunkRegs<TPT> RG, RU;
-  load_chunk<NW, TPT>(RG, a.w_gu_m + (long long)(2 * c) * nT * 32,
-                      a.w_gu_e + (long long)(2 * c) * nT * 16, nT);
-  load_chunk<NW, TPT>(RU, a.w_gu_m + (long long)(2 * c + 1) * nT * 32,
-                      a.w_gu_e + (long long)(2 * c + 1) * nT * 16, nT);
-  stage_x_bfp(xs, xes, a.xn_m + b0 * a.D, a.xn_e + b0 * (a.D / 16), ns * nT);
-  __syncthreads();
-  chunk_AM_multi<NW, TPT, MSEQ>(RG, xs, xes, nT, ns, redM, redA, Aog, Mog);
-  chunk_AM_multi<NW, TPT, MSEQ>(RU, xs, xes, nT, ns, redM, redA, Aou, Mou);
-  BFP_MULTI_EPI(epi_gu(a, b, c, Aog[r_ * MSEQ + sc_], Mog[r_ * MSEQ + sc_], Aou[r_ * MSEQ + sc_],
-                       Mou[r_ * MSEQ + sc_], wr_))
-}
-
-template <int NW, int TPT>
-__global__ __launch_bounds__(64 * NW) void k_d_res_m(LayerArgs a) {
-  extern __shared__ int ism[];
-  const int nT = a.FFN / 16;
-  int *xs = ism;
-  int *xes = ism + MSEQ * nT * 16;
-  __shared__ int redM[NW * 16 * MSEQ];
-  __shared__ long long redA[NW * 16 * MSEQ];
-  __shared__ long long Ao[16 * MSEQ];
-  __shared__ int Mo[16 * MSEQ];
-  const int c = blockIdx.x, b0 = blockIdx.y * MSEQ, ns = min(MSEQ, a.batch - b0);
-  ChunkRegs<TPT> R;
-  load_chunk<NW, TPT>(R, a.w_d_m + (long long)c * nT * 32, a.w_d_e + (long long)c * nT * 16, nT);
-  stage_x_bfp(xs, xes, a.mlp_m + b0 * a.FFN, a.mlp_e + b0 * (a.FFN / 16), ns * nT);
-  __syncthreads();
-  chunk_AM_multi<NW, TPT, MSEQ>(R, xs, xes, nT, ns, redM, redA, Ao, Mo);
-  BFP_MULTI_EPI(epi_dres(a, b, c, Ao[r_ * MSEQ + sc_], Mo[r_ * MSEQ + sc_], wr_,
-                         a.h1_m[b * a.D + c * 16 + r_], a.h1_e[b * (a.D / 16) + c]))
-}
-
 // ------------------------------------------ matrix-core multi-sequence path
 // The four matvecs of a layer for 16 sequences per workgroup on the int8
-// MFMA (bfp_mx.h); the epilogues are the multi-sequence path's.  blockIdx.x
+// MFMA (bfp_mx.h); the epilogues are the per-sequence kernels'.  blockIdx.x
 // is a block of NC chunks, blockIdx.y a group of 16 sequences.  Each
 // 16-lane group runs the epilogue of one (chunk, sequence) pair per pass.
 // The phase stamps of a traced batched decode (MX_TRACE_KERNELS x
@@ -1071,13 +998,18 @@ __global__ __launch_bounds__(256) void k_ctl_embed(CtlArgs a, EmbedArgs e) {
 // --------------------------------------------------------------- launchers
 typedef void (*lk_fn)(LayerArgs);
 
-// Batches from this size on use the multi-sequence kernels, and from
-// MX_MIN_BATCH on their matrix-core form (measured crossover: the MFMA form
-// is ahead from 8 sequences; env BFP_MX_MIN_BATCH overrides).
-constexpr int MULTI_MIN_BATCH = 4;
+// Batches from this size on (a whole group of 16 sequences) run the matvecs
+// on the matrix cores with the RMSNorms once per sequence; below, every
+// (chunk, sequence) is a workgroup of the per-sequence kernels.  At SmolLM2's
+// 30 layers, 23 + 25 tokens, per-sequence against matrix-core launches: 5
+// sequences 26.8 / 38.2 ms, 8 31.0 / 41.1, 12 35.9 / 43.0, 16 41.0 / 45.9, 20
+// 46.4 / 47.6, 24 51.6 / 50.6 -- the crossing is near 22, where the rows are
+// ragged; 16 keeps whole groups on the matrix cores.  (A vector form with 8
+// sequences per workgroup, weights read once for them, took 46.5 ms at 5.)
+// env BFP_MX_MIN_BATCH overrides.
 static int MX_MIN_BATCH = [] {
   const char *v = getenv("BFP_MX_MIN_BATCH");
-  return v ? atoi(v) : 8;
+  return v ? atoi(v) : 16;
 }();
 
 // The (waves, tiles per lane) pairs default_waves() produces for
@@ -1088,16 +1020,35 @@ static int MX_MIN_BATCH = [] {
 #define BFP_CASE(KER, NW, TPT) \
   if (nw == NW && tpt == TPT) return KER<NW, TPT>;
 
-static lk_fn pick_qkv(int nw, int tpt) { BFP_LAYER_SHAPES(BFP_CASE, k_qkv) return nullptr; }
-static lk_fn pick_ores(int nw, int tpt) { BFP_LAYER_SHAPES(BFP_CASE, k_o_res) return nullptr; }
-static lk_fn pick_gu(int nw, int tpt) { BFP_LAYER_SHAPES(BFP_CASE, k_gu) return nullptr; }
-static lk_fn pick_dres(int nw, int tpt) { BFP_LAYER_SHAPES(BFP_CASE, k_d_res) return nullptr; }
+// k_qkv and k_gu: up to D = 1024 a thread per pair of elements (D / 128 waves,
+// at most two tiles a lane), so the RMSNorm prologue is one division pair and
+// one quantisation a thread and every wave sums the squares itself; above, the
+// matvec's own shape with the block-wide norm.
+static bool norm_pairs_shape(int D, int &nw, int &tpt) {
+  if (D > 1024) return false;
+  nw = (D + 127) / 128;
+  tpt = (D / 16 + 4 * nw - 1) / (4 * nw);
+  return true;
+}
+#define BFP_NORM_CASES(KER)                                                                          \
+  int nw, tpt;                                                                                        \
+  if (norm_pairs_shape(D, nw, tpt)) {                                                                 \
+    static const lk_fn k1[8] = {KER<1, 1, true>, KER<2, 1, true>, KER<3, 1, true>, KER<4, 1, true>,   \
+                                KER<5, 1, true>, KER<6, 1, true>, KER<7, 1, true>, KER<8, 1, true>};  \
+    static const lk_fn k2[8] = {KER<1, 2, true>, KER<2, 2, true>, KER<3, 2, true>, KER<4, 2, true>,   \
+                                KER<5, 2, true>, KER<6, 2, true>, KER<7, 2, true>, KER<8, 2, true>};  \
+    threads = 64 * nw;                                                                                \
+    lds = (size_t)norm_prologue_doubles(true, D) * 8 + (size_t)(D / 16) * 17 * 4;                     \
+    return (tpt == 1 ? k1 : k2)[nw - 1];                                                              \
+  }                                                                                                   \
+  threads = 64 * 9;                                                                                   \
+  lds = (size_t)norm_prologue_doubles(false, D) * 8 + (size_t)(D / 16) * 17 * 4;                      \
+  return KER<9, 3, false>;
+static lk_fn pick_qkv(int D, int &threads, size_t &lds) { BFP_NORM_CASES(k_qkv) }
+static lk_fn pick_gu(int D, int &threads, size_t &lds) { BFP_NORM_CASES(k_gu) }
 
-typedef void (*lkm_fn)(LayerArgs);
-static lkm_fn pick_qkv_m(int nw, int tpt) { BFP_LAYER_SHAPES(BFP_CASE, k_qkv_m) return nullptr; }
-static lkm_fn pick_ores_m(int nw, int tpt) { BFP_LAYER_SHAPES(BFP_CASE, k_o_res_m) return nullptr; }
-static lkm_fn pick_gu_m(int nw, int tpt) { BFP_LAYER_SHAPES(BFP_CASE, k_gu_m) return nullptr; }
-static lkm_fn pick_dres_m(int nw, int tpt) { BFP_LAYER_SHAPES(BFP_CASE, k_d_res_m) return nullptr; }
+static lk_fn pick_ores(int nw, int tpt) { BFP_LAYER_SHAPES(BFP_CASE, k_o_res) return nullptr; }
+static lk_fn pick_dres(int nw, int tpt) { BFP_LAYER_SHAPES(BFP_CASE, k_d_res) return nullptr; }
 
 // Waves and tiles per lane of a matvec over nT input tiles.
 static void shape_for(int nT, int &nw, int &tpt) {
@@ -1128,7 +1079,7 @@ int raise_lds_limit(const void *f, int bytes) {
 }
 
 // Per device, before the first launch (outside any stream capture): allow
-// the dynamic LDS the attention and multi-sequence kernels take.
+// the dynamic LDS the attention kernels take.
 int prepare_layer_kernels(int max_ctx, int D, int FFN) {
   const int ppw = attn_ppw(max_ctx);
   BFP_TRY(raise_lds_limit(reinterpret_cast<const void *>(attn_kernel(ppw)),
@@ -1149,17 +1100,6 @@ int prepare_layer_kernels(int max_ctx, int D, int FFN) {
     for (bool tr : {false, true})
       BFP_TRY(raise_lds_limit(reinterpret_cast<const void *>(qkv_attng_kernel(ppw, tr)), (int)qkv_attng_lds(la)));
   }
-  int nw, tpt, nwf, tptf;
-  shape_for(D / 16, nw, tpt);
-  shape_for(FFN / 16, nwf, tptf);
-  const int shD = MSEQ * (D / 16) * 17 * 4, shF = MSEQ * (FFN / 16) * 17 * 4;
-  const void *fs[4] = {reinterpret_cast<const void *>(pick_qkv_m(nw, tpt)),
-                       reinterpret_cast<const void *>(pick_ores_m(nw, tpt)),
-                       reinterpret_cast<const void *>(pick_gu_m(nw, tpt)),
-                       reinterpret_cast<const void *>(pick_dres_m(nwf, tptf))};
-  const int sh[4] = {shD, shD, shD, shF};
-  for (int i = 0; i < 4; ++i)
-    if (fs[i]) BFP_TRY(raise_lds_limit(fs[i], sh[i]));
   return BFP_OK;
 }
 
@@ -1210,9 +1150,11 @@ static bool mx_joined_qkv_attn(const LayerArgs &a) {
          mx_waves(a.D / 16, bq * G) == ATT_WAVES;
 }
 
+// The matrix-core path (its norm buffer is the context's).
+static bool mx_path(const LayerArgs &a) { return a.batch >= MX_MIN_BATCH && a.batch > 1 && a.xn_m; }
+
 int layer_form(const LayerArgs &a) {
-  if (!(a.batch >= MULTI_MIN_BATCH && a.xn_m)) return BFP_FORM_SINGLE;
-  if (a.batch < MX_MIN_BATCH) return BFP_FORM_MULTI;
+  if (!mx_path(a)) return BFP_FORM_SINGLE;
   return BFP_FORM_MX | (mx_joined_qkv_attn(a) ? BFP_FORM_QKV_ATTN : 0) |
          (mx_joined_qkv_attn(a) && mx_attn_grouped(a) ? BFP_FORM_ATT_GROUP : 0) |
          (mx_fused_norms(a) ? BFP_FORM_NORM_FUSED : 0);
@@ -1264,42 +1206,21 @@ static int launch_layer_mx(const LayerArgs &a, hipStream_t s, bool mx_traced) {
   return launch_status("layer");
 }
 
-static int launch_layer_multi(const LayerArgs &a, hipStream_t s, bool mx_traced) {
-  if (a.batch >= MX_MIN_BATCH) return launch_layer_mx(a, s, mx_traced);
-  const int nTD = a.D / 16, nTF = a.FFN / 16;
-  int nw, tpt, nwf, tptf;
-  shape_for(nTD, nw, tpt);
-  shape_for(nTF, nwf, tptf);
-  lkm_fn fq = pick_qkv_m(nw, tpt), fo = pick_ores_m(nw, tpt), fg = pick_gu_m(nw, tpt);
-  lkm_fn fd = pick_dres_m(nwf, tptf);
-  if (!fq || !fo || !fg || !fd) return set_err(BFP_EINVAL, "no layer kernel for D=%d FFN=%d", a.D, a.FFN);
-  const int nq = a.D + 2 * a.KV;
-  const int G = (a.batch + MSEQ - 1) / MSEQ;
-  const size_t shD = (size_t)MSEQ * nTD * 17 * 4, shF = (size_t)MSEQ * nTF * 17 * 4;
-  launch_norm_seq(a, 1, s);
-  hipLaunchKernelGGL(fq, dim3(nq / 16, G), dim3(64 * nw), shD, s, a);
-  BFP_TRY(launch_attn(a, s));
-  hipLaunchKernelGGL(fo, dim3(a.D / 16, G), dim3(64 * nw), shD, s, a);
-  launch_norm_seq(a, 2, s);
-  hipLaunchKernelGGL(fg, dim3(a.FFN / 16, G), dim3(64 * nw), shD, s, a);
-  hipLaunchKernelGGL(fd, dim3(a.D / 16, G), dim3(64 * nwf), shF, s, a);
-  return launch_status("layer");
-}
-
 int launch_layer(const LayerArgs &a, hipStream_t s, bool mx_traced) {
-  if (a.batch >= MULTI_MIN_BATCH && a.xn_m) return launch_layer_multi(a, s, mx_traced);
+  if (mx_path(a)) return launch_layer_mx(a, s, mx_traced);
   const int nTD = a.D / 16, nTF = a.FFN / 16;
   int nw, tpt;
   shape_for(nTD, nw, tpt);
   const int nq = a.D + 2 * a.KV;
-  const size_t sh_norm = (size_t)(3 * a.D + PW_MAX_LEAVES) * 8 + (size_t)nTD * 17 * 4;
-  lk_fn f = pick_qkv(nw, tpt);
-  lk_fn fo = pick_ores(nw, tpt), fg = pick_gu(nw, tpt);
-  if (!f || !fo || !fg) return set_err(BFP_EINVAL, "no layer kernel for D=%d", a.D);
-  hipLaunchKernelGGL(f, dim3(nq / 16, a.batch), dim3(64 * nw), sh_norm, s, a);
+  int tq, tg;
+  size_t sq, sg;
+  lk_fn f = pick_qkv(a.D, tq, sq);
+  lk_fn fo = pick_ores(nw, tpt), fg = pick_gu(a.D, tg, sg);
+  if (!fo) return set_err(BFP_EINVAL, "no layer kernel for D=%d", a.D);
+  hipLaunchKernelGGL(f, dim3(nq / 16, a.batch), dim3(tq), sq, s, a);
   BFP_TRY(launch_attn(a, s));
   hipLaunchKernelGGL(fo, dim3(a.D / 16, a.batch), dim3(64 * nw), (size_t)nTD * 17 * 4, s, a);
-  hipLaunchKernelGGL(fg, dim3(a.FFN / 16, a.batch), dim3(64 * nw), sh_norm, s, a);
+  hipLaunchKernelGGL(fg, dim3(a.FFN / 16, a.batch), dim3(tg), sg, s, a);
   int nwf, tptf;
   shape_for(nTF, nwf, tptf);
   f = pick_dres(nwf, tptf);
@@ -1568,14 +1489,17 @@ __global__ __launch_bounds__(256) void k_embq_build(const float *__restrict__ E,
 // group; the block's maxima over its rows go to hq_blk[s][block].
 typedef int headq_v4 __attribute__((ext_vector_type(4)));
 constexpr int HEADQ_PD = 4;   // weight groups in flight ahead of the one in use
-template <int G>
+// NQ: sequence groups of the workgroup, 4 (64 sequences), or 1 for at most
+// 16 sequences (a quarter of the LDS reads and products: 12.1 against 18.9 us
+// at 5 sequences and 64).
+template <int G, int NQ>
 __global__ __launch_bounds__(512, 4) void k_headq_mx(HeadArgs a) {
-  extern __shared__ uint4 xq[];   // [4 groups][G][2 planes][64 lanes]
+  extern __shared__ uint4 xq[];   // [NQ groups][G][2 planes][64 lanes]
   __shared__ HeadQSeq sq[HEADQ_SEQ];
   __shared__ HeadQRow rq[8 * 16];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, kg = lane >> 4, i = lane & 15;
-  const int b0 = blockIdx.y * HEADQ_SEQ;
-  const int nq = min(4, (a.batch - b0 + 15) / 16);
+  const int b0 = blockIdx.y * (16 * NQ);
+  const int nq = min(NQ, (a.batch - b0 + 15) / 16);
   const int nch = a.VOCAB / 16;
   const int c = min(blockIdx.x * 8 + w, nch - 1);   // past the end: block nch-1 again, not stored
   // the first weight groups of this wave's block, then the stage: the
@@ -1591,7 +1515,7 @@ __global__ __launch_bounds__(512, 4) void k_headq_mx(HeadArgs a) {
   {
     // every staging load of a thread before its stores (one after another,
     // load then store, the stage took 6 us)
-    constexpr int SPT = (4 * G * 128 + 511) / 512;
+    constexpr int SPT = (NQ * G * 128 + 511) / 512;
     const int lim = nq * G * 128;
     const uint4 *src = a.hq_x + (long long)(b0 / 16) * G * 128;
     uint4 st[SPT];
@@ -1613,11 +1537,11 @@ __global__ __launch_bounds__(512, 4) void k_headq_mx(HeadArgs a) {
     if (tid < HEADQ_SEQ) sq[tid] = ss;
   }
   __syncthreads();
-  // the four sequence groups' products side by side: 16 independent
+  // the sequence groups' products side by side: 4 NQ independent
   // accumulators, one group of 64 columns at a time
-  headq_v4 acc[4][4];
+  headq_v4 acc[NQ][4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
+  for (int q = 0; q < NQ; ++q)
 #pragma unroll
     for (int k = 0; k < 4; ++k) acc[q][k] = headq_v4{0, 0, 0, 0};
 #pragma unroll
@@ -1630,7 +1554,7 @@ __global__ __launch_bounds__(512, 4) void k_headq_mx(HeadArgs a) {
     const headq_v4 wh = {(int)wh4.x, (int)wh4.y, (int)wh4.z, (int)wh4.w};
     const headq_v4 wl = {(int)wl4.x, (int)wl4.y, (int)wl4.z, (int)wl4.w};
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < NQ; ++q) {
       const uint4 xh4 = xq[(q * G + g) * 128 + lane], xl4 = xq[(q * G + g) * 128 + 64 + lane];
       const headq_v4 xh = {(int)xh4.x, (int)xh4.y, (int)xh4.z, (int)xh4.w};
       const headq_v4 xl = {(int)xl4.x, (int)xl4.y, (int)xl4.z, (int)xl4.w};
@@ -1642,7 +1566,7 @@ __global__ __launch_bounds__(512, 4) void k_headq_mx(HeadArgs a) {
   }
   const bool store = blockIdx.x * 8 + w < nch;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int s = b0 + 16 * q + i;
     const HeadQSeq Q = sq[(16 * q + i) < HEADQ_SEQ ? 16 * q + i : 0];
     const long long sx = 128LL * Q.sumx - 16384LL * a.D;
@@ -1767,23 +1691,17 @@ __global__ __launch_bounds__(HEADQ_PICK_T) void k_headq_pick(HeadArgs a) {
     a.part_i[b] = besti;
   }
 }
-inline size_t headq_pick_lds(int D, int VOCAB) { return (size_t)D * 8 + (size_t)(VOCAB / 16) * 4; }
-
 typedef void (*headq_mx_fn)(HeadArgs);
-static headq_mx_fn headq_mx_kernel(int G) {
-  switch (G) {
-    case 1: return k_headq_mx<1>;
-    case 2: return k_headq_mx<2>;
-    case 3: return k_headq_mx<3>;
-    case 4: return k_headq_mx<4>;
-    case 5: return k_headq_mx<5>;
-    case 6: return k_headq_mx<6>;
-    case 7: return k_headq_mx<7>;
-    case 8: return k_headq_mx<8>;
-    default: return k_headq_mx<9>;
-  }
+template <int NQ>
+static headq_mx_fn headq_mx_pick(int G) {
+  static const headq_mx_fn k[9] = {k_headq_mx<1, NQ>, k_headq_mx<2, NQ>, k_headq_mx<3, NQ>,
+                                   k_headq_mx<4, NQ>, k_headq_mx<5, NQ>, k_headq_mx<6, NQ>,
+                                   k_headq_mx<7, NQ>, k_headq_mx<8, NQ>, k_headq_mx<9, NQ>};
+  return k[G - 1];
 }
-inline int headq_mx_lds(int D) { return 4 * (D / 64) * 64 * 32; }
+inline int headq_nq(int batch) { return batch <= 16 ? 1 : 4; }
+static headq_mx_fn headq_mx_kernel(int G, int nq) { return nq == 1 ? headq_mx_pick<1>(G) : headq_mx_pick<4>(G); }
+inline int headq_mx_lds(int D, int nq) { return nq * (D / 64) * 64 * 32; }
 
 int launch_embq_build(const float *embed, int VOCAB, int D, uint4 *q, HeadQRow *meta, hipStream_t s) {
   hipLaunchKernelGGL(k_embq_build, dim3(VOCAB / 16), dim3(256), 0, s, embed, D, q, meta);
@@ -1822,7 +1740,8 @@ int prepare_head_kernels(int D) {
   BFP_TRY(raise_lds_limit(reinterpret_cast<const void *>(k_head_gemv<27, 1, false>), sh));
   if (D % 64 == 0 && D <= 576) {
     BFP_TRY(raise_lds_limit(reinterpret_cast<const void *>(head_mx_kernel(D / 64)), head_mx_lds(D)));
-    BFP_TRY(raise_lds_limit(reinterpret_cast<const void *>(headq_mx_kernel(D / 64)), headq_mx_lds(D)));
+    for (int nq : {1, 4})
+      BFP_TRY(raise_lds_limit(reinterpret_cast<const void *>(headq_mx_kernel(D / 64, nq)), headq_mx_lds(D, nq)));
   }
   return BFP_OK;
 }
@@ -1842,11 +1761,12 @@ int launch_head(const HeadArgs &a, hipStream_t s) {
   const bool seqf = head_seq_form(a.D, a.batch, a.embedp != nullptr);
   if (a.hq_blk) {
     // the bounded head: one (value, index) a sequence
-    if (!seqf || a.logits || !a.embq || !a.embq_meta || !a.hq_x || !a.hq_seq || a.n_wg != 1)
+    if (a.D % 64 || a.D > 576 || a.logits || !a.embq || !a.embq_meta || !a.hq_x || !a.hq_seq || a.n_wg != 1)
       return set_err(BFP_EINVAL, "head: bounded form without its buffers");
+    const int nq = headq_nq(a.batch);
     hipLaunchKernelGGL(k_head_norm, dim3(a.batch), dim3(256), sh, s, a);
-    hipLaunchKernelGGL(headq_mx_kernel(a.D / 64), dim3((a.VOCAB / 16 + 7) / 8, (a.batch + HEADQ_SEQ - 1) / HEADQ_SEQ),
-                       dim3(512), headq_mx_lds(a.D), s, a);
+    hipLaunchKernelGGL(headq_mx_kernel(a.D / 64, nq), dim3((a.VOCAB / 16 + 7) / 8, (a.batch + 16 * nq - 1) / (16 * nq)),
+                       dim3(512), headq_mx_lds(a.D, nq), s, a);
     const size_t shp = headq_pick_lds(a.D, a.VOCAB);
     if (shp > 64 * 1024) return set_err(BFP_EINVAL, "head: vocabulary %d too large for the bounded form", a.VOCAB);
     if (a.D == 576)
