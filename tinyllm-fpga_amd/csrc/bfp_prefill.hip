@@ -23,6 +23,7 @@
 #include "bfp_internal.h"
 #include "bfp_prefill.h"
 
+#include "bfp_attn_rows.h"
 #include "bfp_layer_dev.h"
 
 namespace bfp {
@@ -82,23 +83,28 @@ __global__ __launch_bounds__(64 * PF_ROPE_WAVES) void k_pf_rope(PrefillArgs a) {
 // heads of one KV group: NP = QT * GH (position, head) pairs over the same K
 // and V rows.
 //   scores   a block of 256 K rows goes through LDS (coalesced 16-byte
-//            loads); lane t of a wave decodes K row t once and forms that
-//            row's SkylakeX ddot with half of the pairs' q, whose elements
-//            are the same for every lane and come through scalar loads;
+//            loads, the next block's in flight); lane t of a wave decodes K
+//            row t once and forms that row's SkylakeX ddot with half of the
+//            pairs' q (ddot64_rows);
 //   softmax  one wave per pair, the whole row of scores in LDS, numpy's
 //            pairwise sum on the wave (pairwise_sum_wave);
-//   AV       V blocks of 32 rows decoded to float64 in LDS (two buffers);
-//            waves 0-3 run the chains, one dimension a lane, NP / 4 pairs
-//            each, p taken from a lane register by readlane; waves 4-7
-//            decode the next block meanwhile.
+//   AV       V blocks of 32 rows decoded to float64 in LDS (two buffers) by
+//            waves 4-7; waves 0-3 run the chains, one dimension a lane, NP / 4
+//            pairs each (av_block).
 // The LDS holds NP rows of scores, so NP is chosen by the longest context of
-// the pass (pf_attn_shape).
+// the pass (pf_attn_shape).  What bounds it at long contexts is the vector
+// unit: per pair and position two float64 products with their zeroed
+// accumulators and the adds of ddot64_rows on a 64-lane wave, and three
+// instructions of the chain.  1000 positions at SmolLM2's width: 153 us a layer
+// (223 with q by scalar loads, p by lane reads and one V block in flight), of
+// which the chains take 57, the scores 40 and the softmax 26; 64 sequences of
+// 8: 30 (46), 5 of 23: 16 (27).
 constexpr int PF_KB = 256;             // K rows per staged block
 constexpr int PF_KS = 72;              // K row stride in LDS (int16), bank-spread
-constexpr int PF_VB = 32;              // V rows per decoded block
 constexpr int PF_NP = 12;              // most pairs of a workgroup
 constexpr int PF_SC_BYTES = 98304;     // most LDS for the scores
 constexpr int PF_T = 512;
+constexpr int PF_WORK = PF_KB * (PF_KS * 2 + 4) > 2 * ROWS_VB * 64 * 8 ? PF_KB * (PF_KS * 2 + 4) : 2 * ROWS_VB * 64 * 8;
 
 struct PfAttnShape {
   int gh, ngh, qt, scl;   // heads a workgroup, workgroups a KV group, positions, score row length
@@ -112,33 +118,8 @@ inline PfAttnShape pf_attn_shape(int H_Q, int H_KV, int n, int ctx) {
   s.scl = (ctx + 1) & ~1;
   const int np = std::min(PF_NP, std::max(s.gh, PF_SC_BYTES / (s.scl * 8)));
   s.qt = std::max(1, std::min(np / s.gh, n));
-  const size_t kst = (size_t)PF_KB * (PF_KS * 2 + 4), vst = (size_t)2 * PF_VB * 64 * 8;
-  s.lds = (size_t)s.qt * s.gh * s.scl * 8 + std::max(kst, vst) + 8 * PW_MAX_LEAVES * 8;
+  s.lds = (size_t)s.qt * s.gh * s.scl * 8 + PF_WORK + 8 * PW_MAX_LEAVES * 8;
   return s;
-}
-
-typedef const __attribute__((address_space(4))) double *pf_cdouble;
-__device__ __forceinline__ pf_cdouble pf_const(const double *p) {
-  return (pf_cdouble)(uintptr_t)p;
-}
-
-// np.dot(q, K[t]) in the SkylakeX ddot order (ddot64_skx) with q through the
-// constant address space and K decoded in registers.
-__device__ __forceinline__ double pf_ddot(pf_cdouble x, const double (&y)[64]) {
-  double s[4];
-#pragma unroll
-  for (int l = 0; l < 4; ++l) {
-    double f[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = 8 * r + l;
-      const double a0 = fma(x[32 + i], y[32 + i], fma(x[i], y[i], 0.0));
-      const double a1 = fma(x[36 + i], y[36 + i], fma(x[4 + i], y[4 + i], 0.0));
-      f[r] = a0 + a1;
-    }
-    s[l] = ((f[0] + f[1]) + f[2]) + f[3];
-  }
-  return (s[0] + s[2]) + (s[1] + s[3]);
 }
 
 // numpy's add-reduce of a[0..n) (1 <= n <= 4096, LDS) by one wave:
@@ -191,48 +172,13 @@ __device__ __forceinline__ double pairwise_sum_wave(const double *a, int n, doub
   return 0.0 + pw_combine_wave(n, leaf);
 }
 
-__device__ __forceinline__ double pf_readlane(double v, int lane) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), lane);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
-}
-
-// The chains of NC pairs of one wave over the rows t0 .. t0 + PF_VB - 1:
-// pair i has n[i] positions (rows from n[i] on are left out).
-template <int NC>
-__device__ __forceinline__ void pf_av_block(const double *vb, const double *const (&p)[3], const int (&n)[3],
-                                            int t0, double (&acc)[3]) {
-  const int l = threadIdx.x & 63;
-  double pv[NC];
-#pragma unroll
-  for (int i = 0; i < NC; ++i) pv[i] = l < PF_VB && t0 + l < n[i] ? p[i][t0 + l] : 0.0;
-  // a position past n[i] has p = 0 here: its product is +-0, and adding it
-  // leaves acc unchanged (acc starts at +0.0 and is never -0)
-  int end = t0;
-#pragma unroll
-  for (int i = 0; i < NC; ++i) end = n[i] > end ? n[i] : end;
-  end = (end < t0 + PF_VB ? end : t0 + PF_VB) - t0;
-  for (int u0 = 0; u0 < end; u0 += 8) {   // uniform
-    double v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = vb[(u0 + u) * 64 + l];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-#pragma unroll
-      for (int i = 0; i < NC; ++i) acc[i] = acc[i] + pf_readlane(pv[i], u0 + u) * v[u];
-    }
-  }
-}
-
 __global__ __launch_bounds__(PF_T, 2) void k_pf_attn(PrefillArgs a, int gh, int ngh, int qt, int scl) {
   extern __shared__ double dsm[];
   const LayerArgs &L = a.L;
   const int np = qt * gh;
   double *sc = dsm;                                         // np x scl
   double *work = sc + np * scl;                             // K stage / V blocks
-  const int kbytes = PF_KB * (PF_KS * 2 + 4), vbytes = 2 * PF_VB * 64 * 8;
-  double *leaf = work + (kbytes > vbytes ? kbytes : vbytes) / 8;   // 8 x PW_MAX_LEAVES
+  double *leaf = work + PF_WORK / 8;                        // 8 x PW_MAX_LEAVES
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
   const int grp = L.H_Q / L.H_KV;
   // blockIdx.x: (KV group, head part); y: position tiles, the longest first; z: sequence
@@ -253,38 +199,44 @@ __global__ __launch_bounds__(PF_T, 2) void k_pf_attn(PrefillArgs a, int gh, int 
   // scores[t] = float(np.dot(q, K[t])) / sqrt(HD)   (full.py:277-278)
   int16_t *kst = reinterpret_cast<int16_t *>(work);
   int8_t *kex = reinterpret_cast<int8_t *>(kst + PF_KB * PF_KS);
-  for (int k0 = 0; k0 < nk; k0 += PF_KB) {   // uniform
-    uint4 kr[PF_KB * 8 / PF_T];
+  constexpr int KL = PF_KB * 8 / PF_T;
+  uint4 kr[KL];
+  int ke;
+  auto load_k = [&](int k0) {
 #pragma unroll
-    for (int j = 0; j < PF_KB * 8 / PF_T; ++j) {
+    for (int j = 0; j < KL; ++j) {
       int t = k0 + (tid >> 3) + (PF_T / 8) * j;
       t = t < nk ? t : nk - 1;
       kr[j] = *reinterpret_cast<const uint4 *>(Km + t * kv_tok + 8 * (tid & 7));
     }
     const int te = min(k0 + (tid & (PF_KB - 1)), nk - 1);
-    const int ke = *reinterpret_cast<const int *>(Ke + te * (kv_tok / 16));
+    ke = *reinterpret_cast<const int *>(Ke + te * (kv_tok / 16));
+  };
+  auto q_ptr = [&](int i) {   // pair i's q
+    const int qi = i / nh;
+    return qb + (long long)qi * L.D + (i - qi * nh) * 64;
+  };
+  load_k(0);
+  for (int k0 = 0; k0 < nk; k0 += PF_KB) {   // uniform
     if (k0) lds_barrier();   // the block before is read
 #pragma unroll
-    for (int j = 0; j < PF_KB * 8 / PF_T; ++j)
+    for (int j = 0; j < KL; ++j)
       *reinterpret_cast<uint4 *>(kst + ((tid >> 3) + (PF_T / 8) * j) * PF_KS + 8 * (tid & 7)) = kr[j];
     if (tid < PF_KB) *reinterpret_cast<int *>(kex + 4 * tid) = ke;
+    load_k(k0 + PF_KB);      // past the end: the last row again
     lds_barrier();
     const int tl = 64 * (w & 3) + l, t = k0 + tl;
-    if (k0 + 64 * (w & 3) < nk) {   // uniform per wave
+    const int i0 = w >> 2;
+    if (k0 + 64 * (w & 3) < nk && i0 < npl) {   // uniform per wave
+      RowVec q;
+      q.load(q_ptr(i0));
       double y[64];
-      const int ke4 = *reinterpret_cast<const int *>(kex + 4 * tl);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const uint4 u = *reinterpret_cast<const uint4 *>(kst + tl * PF_KS + 8 * j);
-        const double s = ldexp(1.0, (int)(signed char)((ke4 >> (8 * (j >> 1))) & 0xff) - 15);
-        const unsigned wd[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-        for (int i = 0; i < 8; ++i) y[8 * j + i] = (double)(int)(short)((wd[i >> 1] >> (16 * (i & 1))) & 0xffff) * s;
-      }
-      for (int i = w >> 2; i < npl; i += 2) {
-        const int qi = i / nh, hi = i - qi * nh;
-        const double s = pf_ddot(pf_const(qb + (long long)qi * L.D + hi * 64), y) * L.score_mul;
-        if (t <= pos0 + qi) sc[i * scl + t] = s;
+      decode_row64(kst + tl * PF_KS, *reinterpret_cast<const int *>(kex + 4 * tl), y);
+      for (int i = i0; i < npl; i += 2) {
+        const RowVec qc = q;
+        q.load(q_ptr(i + 2 < npl ? i + 2 : i));   // in flight during this pair's products
+        const double s = ddot64_rows(qc, y) * L.score_mul;
+        if (t <= pos0 + i / nh) sc[i * scl + t] = s;
       }
     }
   }
@@ -312,22 +264,36 @@ __global__ __launch_bounds__(PF_T, 2) void k_pf_attn(PrefillArgs a, int gh, int 
   lds_barrier();
 
   // attn = sum_t p[t] * V[t], ascending t from 0.0 (full.py:280-281)
-  const int nvb = (nk + PF_VB - 1) / PF_VB;
-  // decode V block k into its buffer: `part` of `parts` waves, lane = (row
-  // l / 8 of 8, 16-byte part l % 8)
-  auto decode_v = [&](int k, int part, int parts) {
-    double *vb = work + (k & 1) * (PF_VB * 64);
-    for (int rr = 8 * part; rr < PF_VB; rr += 8 * parts) {
-      const int r = rr + (l >> 3), t = min(k * PF_VB + r, nk - 1), q = l & 7;
-      const uint4 u = *reinterpret_cast<const uint4 *>(Vm + t * kv_tok + 8 * q);
-      const double s = ldexp(1.0, (int)Ve[t * (kv_tok / 16) + (q >> 1)] - 15);
-      const unsigned wd[4] = {u.x, u.y, u.z, u.w};
-      double2 *o = reinterpret_cast<double2 *>(vb + r * 64 + 8 * q);
+  const int nvb = (nk + ROWS_VB - 1) / ROWS_VB;
+  if (w >= 4) {
+    // producers: block k's 32 rows, wave part w - 4 of 8 rows
+    VRing R;
+    auto load_v = [&](int k, uint4 &m, int &e) {
+      const int t = min(k * ROWS_VB + 8 * (w - 4) + (l >> 3), nk - 1), q = l & 7;
+      m = *reinterpret_cast<const uint4 *>(Vm + t * kv_tok + 8 * q);
+      e = Ve[t * (kv_tok / 16) + (q >> 1)];
+    };
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        o[i] = make_double2((double)(int)(short)(wd[i] & 0xffff) * s, (double)((int)wd[i] >> 16) * s);
+    for (int d = 0; d < ROWS_DEPTH; ++d) load_v(d, R.m[d], R.e[d]);
+    for (int k0 = 0; k0 < nvb; k0 += ROWS_DEPTH) {   // uniform
+#pragma unroll
+      for (int d = 0; d < ROWS_DEPTH; ++d) {
+        const int k = k0 + d;
+        if (k < nvb) {
+          const uint4 u = R.m[d];
+          const double s = ldexp(1.0, R.e[d] - 15);
+          const unsigned wd[4] = {u.x, u.y, u.z, u.w};
+          double2 *o = reinterpret_cast<double2 *>(work + (k & 1) * (ROWS_VB * 64) + (8 * (w - 4) + (l >> 3)) * 64 + 8 * (l & 7));
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            o[i] = make_double2((double)(int)(short)(wd[i] & 0xffff) * s, (double)((int)wd[i] >> 16) * s);
+        }
+        load_v(k + ROWS_DEPTH, R.m[d], R.e[d]);
+        if (k < nvb) lds_barrier();   // block k is in place, block k - 1 used
+      }
     }
-  };
+    return;
+  }
   // wave w < 4 holds pairs w, w + 4, w + 8
   double acc[3] = {0.0, 0.0, 0.0};
   const double *pp[3];
@@ -336,25 +302,19 @@ __global__ __launch_bounds__(PF_T, 2) void k_pf_attn(PrefillArgs a, int gh, int 
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     const int pi = w + 4 * i;
-    const bool on = w < 4 && pi < npl;
+    const bool on = pi < npl;
     pp[i] = sc + (on ? pi : 0) * scl;
     pn[i] = on ? pos0 + pi / nh + 1 : 0;
     nc += on ? 1 : 0;
   }
-  decode_v(0, w, 8);
-  lds_barrier();
   for (int k = 0; k < nvb; ++k) {
-    if (w >= 4) {
-      if (k + 1 < nvb) decode_v(k + 1, w - 4, 4);
-    } else {
-      const double *vb = work + (k & 1) * (PF_VB * 64);
-      if (nc == 3) pf_av_block<3>(vb, pp, pn, k * PF_VB, acc);
-      else if (nc == 2) pf_av_block<2>(vb, pp, pn, k * PF_VB, acc);
-      else if (nc == 1) pf_av_block<1>(vb, pp, pn, k * PF_VB, acc);
-    }
-    lds_barrier();
+    lds_barrier();   // block k is in place
+    const double *vb = work + (k & 1) * (ROWS_VB * 64);
+    if (nc == 3) av_block<3>(vb, pp, pn, k * ROWS_VB, acc);
+    else if (nc == 2) av_block<2>(vb, pp, pn, k * ROWS_VB, acc);
+    else if (nc == 1) av_block<1>(vb, pp, pn, k * ROWS_VB, acc);
   }
-  if (w < 4) {
+  {
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       const int pi = w + 4 * i;
@@ -387,9 +347,7 @@ __global__ __launch_bounds__(256) void k_pf_hist(PrefillArgs a) {
 
 // --------------------------------------------------------------- launchers
 int prepare_prefill_kernels() {
-  return raise_lds_limit(reinterpret_cast<const void *>(k_pf_attn),
-                         (int)(PF_SC_BYTES + std::max((size_t)PF_KB * (PF_KS * 2 + 4), (size_t)2 * PF_VB * 64 * 8) +
-                               8 * PW_MAX_LEAVES * 8));
+  return raise_lds_limit(reinterpret_cast<const void *>(k_pf_attn), PF_SC_BYTES + PF_WORK + 8 * PW_MAX_LEAVES * 8);
 }
 
 int launch_prefill_embed(const PrefillArgs &a, hipStream_t s) {
