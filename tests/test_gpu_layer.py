@@ -172,3 +172,42 @@ def test_batched_matvecs_exponent_spreads(gpu, spread):
             assert np.array_equal(st[name][1][b], ws[name][1][0]), (b, name)
         assert np.array_equal(om[b], wm[0]) and np.array_equal(oe[b], we[0])
     gm.close()
+
+
+@pytest.mark.parametrize("cfg", [dict(D=576, H_Q=9, H_KV=3, FFN=256, MAX_CTX=2048),
+                                 dict(D=768, H_Q=12, H_KV=12, FFN=336, MAX_CTX=513),
+                                 dict(D=512, H_Q=8, H_KV=2, FFN=512, MAX_CTX=4096)],
+                         ids=["ctx2048", "ctx513", "ctx4096"])
+def test_long_attention_forms(gpu, cfg):
+    """Capacities past 512: one workgroup per head (past 512 / 4 heads a
+    launch, without a stage dump) against four per head (with one, and below
+    that), at the edges of the 32-row V blocks, the 64-row wave shares and the
+    512-row K blocks, peaked and flat scores, RoPE position and KV slot apart."""
+    from bfp import Dims, synth
+    from bfp.model import BfpModel
+    d = Dims(HD=64, NL=1, VOCAB=256, **cfg)
+    B = 128 // d.H_Q + 1
+    fm = synth.make_model(d, seed=5)
+    gm = BfpModel(d, max_batch=B)
+    gm.load_fp32(fm)
+    rng = np.random.default_rng(d.MAX_CTX)
+    n = d.MAX_CTX
+    for b in range(B):
+        km = rng.integers(-32768, 32768, size=(n, d.KV)).astype(np.int16)
+        ke = rng.integers(-3 if b else -12, 3 if b else 5, size=(n, d.KV // 16)).astype(np.int8)
+        gm.kv_io(0, b, 0, n, k=(km, ke), v=(km[::-1], ke[::-1]))
+    for pos in (0, 1, 31, 32, 33, 63, 64, 500, 511, 512, 513, 1023, 1024, 1100, n - 1):
+        if pos >= n:
+            continue
+        hm = rng.integers(-20000, 20000, size=(B, d.D)).astype(np.int16)
+        he = np.zeros((B, d.D // 16), np.int8)
+        want = gm.layer_step_bfp(0, pos + 3, hm, he, kv_pos=pos, dump=True)
+        k0 = [gm.kv_io(0, b, pos, 1) for b in range(B)]
+        got = gm.layer_step_bfp(0, pos + 3, hm, he, kv_pos=pos)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), pos
+        for b in range(B):
+            k1 = gm.kv_io(0, b, pos, 1)
+            assert all(np.array_equal(x, y) for p, q in zip(k0[b], k1) for x, y in zip(p, q)), pos
+        one = gm.layer_step_bfp(0, pos + 3, hm[0], he[0], kv_pos=pos)
+        assert np.array_equal(one[0][0], got[0][0]) and np.array_equal(one[1][0], got[1][0]), pos
+    gm.close()

@@ -81,6 +81,9 @@ int launch_rows_post(const LayerArgs &a, hipStream_t s);
 // The launch form launch_layer takes for a (BFP_FORM_* bits).
 int layer_form(const LayerArgs &a);
 int prepare_layer_kernels(int max_ctx, int D, int FFN);
+// One workgroup per (head, sequence) for capacities past 512 (bfp_attn_long.hip).
+int prepare_attn_long(int max_ctx);
+int launch_attn_long(const LayerArgs &a, hipStream_t s);
 int prepare_head_kernels(int D);
 // Raise a kernel's dynamic-LDS limit on the current device to at least
 // `bytes` (never lowering it: the limit is process-wide per device).

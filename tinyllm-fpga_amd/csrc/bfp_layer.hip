@@ -1084,6 +1084,7 @@ int prepare_layer_kernels(int max_ctx, int D, int FFN) {
   const int ppw = attn_ppw(max_ctx);
   BFP_TRY(raise_lds_limit(reinterpret_cast<const void *>(attn_kernel(ppw)),
                           (int)attn_lds_bytes(max_ctx, ppw, AttnPlainIO::kAvBlock)));
+  if (ppw == 8) BFP_TRY(prepare_attn_long(max_ctx));
   if (ppw <= 4) {
     LayerArgs la{};
     la.max_ctx = max_ctx;
@@ -1103,8 +1104,17 @@ int prepare_layer_kernels(int max_ctx, int D, int FFN) {
   return BFP_OK;
 }
 
+// Long contexts: four workgroups a head (k_attn<8>) while they all run at
+// once, two rounds of the 256 CUs at most, since their quarter of the AV chain
+// is the shorter one; one workgroup a head past that, which forms the scores
+// once and not four times.  Two layer calls, four / one, us: 1 sequence at
+// position 1500 118 / 172, 4 at 600 109 / 137, 16 at 100 185 / 168, 16 at 1500
+// 272 / 239, 64 at 600 392 / 328.
+constexpr int ATT_LONG_SPLIT_MAX = 512;
 static int launch_attn(const LayerArgs &a, hipStream_t s) {
   const int ppw = attn_ppw(a.max_ctx);
+  if (ppw == 8 && !a.dump && a.H_Q * ATT_DSPLIT * a.batch > ATT_LONG_SPLIT_MAX)
+    return launch_attn_long(a, s);
   // long contexts: ATT_DSPLIT workgroups per head, one 16-dimension tile each
   const int split = ppw == 8 ? ATT_DSPLIT : 1;
   hipLaunchKernelGGL(attn_kernel(ppw), dim3(a.H_Q * split, a.batch), dim3(64 * ATT_WAVES),
