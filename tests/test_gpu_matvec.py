@@ -264,3 +264,38 @@ def test_bad_shapes_raise(gpu):
         from bfp import _dev
         from bfp._lib import call
         call("bfp_matvec_d", 0, 0, 15, 16, 1, 0, 0, 0, 0, 0, 0, 0, 0, 0, _dev.stream())
+
+
+@pytest.mark.parametrize("n_out,n_in", [(16, 16), (16, 48), (48, 32), (80, 144), (176, 1536)])
+def test_quantize_pack_values(gpu, n_out, n_in):
+    """The packing quantizer against the tile quantizer of float64 values,
+    bit for bit: odd tile counts, partial wave units, zero tiles, denormals,
+    values at and beside powers of two, the largest floats, infinities; the
+    bytes behind both outputs are left alone."""
+    import torch
+    from bfp import _dev
+    from bfp._lib import call
+    rng = np.random.default_rng(n_out * n_in)
+    W = rng.standard_normal((n_out, n_in)).astype(np.float32)
+    W = np.ldexp(W, np.repeat(rng.integers(-148, 126, size=(n_out, n_in // 16)), 16, axis=1)).astype(np.float32)
+    t = W.reshape(-1, 16)
+    t[0] = 0
+    t[1::7, 3] = np.ldexp(np.float32(1), rng.integers(-149, 127, size=t[1::7, 3].shape)).astype(np.float32)
+    t[2::7, 5] = np.nextafter(np.float32(4), np.float32(0))
+    t[3::7] = np.float32(3.4e38) * np.sign(t[3::7])
+    t[4::7, :] *= np.float32(1e-40)
+    t[5::29, 15] = np.float32(-np.inf)
+    dW = _dev.to_dev(W)
+    nb = n_out * n_in
+    Pm = torch.full((nb + 8,), 0x5A5A, dtype=torch.int16, device="cuda")
+    Pe = torch.full((nb // 16 + 16,), 0x5A, dtype=torch.int8, device="cuda")
+    call("bfp_quantize_pack_f32_d", dW.data_ptr(), n_out, n_in, Pm.data_ptr(), Pe.data_ptr(), _dev.stream())
+    dV = _dev.to_dev(W.astype(np.float64))
+    m = torch.empty(nb, dtype=torch.int16, device="cuda")
+    e = torch.empty(nb // 16, dtype=torch.int8, device="cuda")
+    call("bfp_tile_quantize_f64_d", dV.data_ptr(), nb, m.data_ptr(), e.data_ptr(), _dev.stream())
+    nT = n_in // 16
+    m = m.view(-1, 16, nT, 2, 8).permute(0, 2, 3, 1, 4).flatten()
+    e = e.view(-1, 16, nT).permute(0, 2, 1).flatten()
+    assert torch.equal(Pm[:nb], m) and torch.equal(Pe[:nb // 16], e)
+    assert (Pm[nb:] == 0x5A5A).all() and (Pe[nb // 16:] == 0x5A).all()
