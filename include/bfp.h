@@ -348,7 +348,8 @@ int bfp_head(bfp_ctx *ctx, int batch, const int16_t *h_m, const int8_t *h_e, dou
  * independent sequences, including the reference's quirk that step
  * n_prompt re-feeds the last prompt token.  prompt: batch x n_prompt;
  * tokens_out: batch x n_gen.  hist_m/hist_e (optional): every layer's
- * output at every step, (batch, n_prompt + n_gen, NL, D) / (..., D/16).
+ * output at every step, (batch, n_prompt + n_gen, NL, D) / (..., D/16),
+ * written while the decode runs (after an error they hold some of it).
  * The KV cache is overwritten from position 0. */
 #define BFP_DECODE_NO_GRAPH 1
 #define BFP_DECODE_STEP_TIMES 2   /* record one HIP event per step */

@@ -450,3 +450,26 @@ def test_decode_small_batches(gpu, batch):
         assert list(toks[b]) == list(want)
         assert np.array_equal(hm[b], whm) and np.array_equal(he[b], whe)
     gm.close()
+
+
+@pytest.mark.parametrize("batch,n_prompt,n_gen", [(700, 3, 9), (40, 20, 41), (1, 1000, 9), (1, 9, 1010)])
+def test_history_pieces(gpu, batch, n_prompt, n_gen):
+    """The history's pieces on their way to the host: a step of more bytes
+    than a piece (700 sequences), several pieces and marks, a prompt pass of
+    several pieces, one piece after another behind the persistent launch --
+    against decodes of a few of the sequences, or step by step, whose pieces
+    lie elsewhere."""
+    from bfp import Dims, synth
+    from bfp.model import BfpModel
+    d = Dims(D=128, H_Q=2, H_KV=1, HD=64, FFN=256, NL=13, MAX_CTX=n_prompt + n_gen, VOCAB=512)
+    gm = BfpModel(d, max_batch=batch)
+    gm.load_fp32(synth.make_model(d, seed=3))
+    prompts = np.stack([synth.make_prompt(d, n_prompt, seed=b) for b in range(batch)])
+    toks, (hm, he) = gm.decode(prompts, n_gen, hist=True)
+    assert hm.any(axis=(2, 3)).all()   # every step of every sequence is there
+    for b0 in sorted({0, batch // 2, max(batch - 8, 0)}):
+        part = slice(b0, min(b0 + 8, batch))
+        want, (wm, we) = gm.decode(prompts[part], n_gen, hist=True, graph=False)
+        assert (toks[part] == want).all(), b0
+        assert (hm[part] == wm).all() and (he[part] == we).all(), b0
+    gm.close()
