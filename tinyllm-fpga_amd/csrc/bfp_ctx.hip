@@ -554,32 +554,50 @@ class HistOut {
   std::deque<Mark> marks_;
 };
 
+// The prompt pass's activations for `rows` rows, in one block made on the
+// first use for the most rows any call of this context takes.  False where
+// there is no memory for it: the decode then runs its prompt step by step.
+bool prefill_ready(bfp_ctx *c, int rows) {
+  if (rows <= c->pf_rows) return true;
+  const bfp_dims &d = c->d;
+  const size_t R = (size_t)std::min<long long>(PF_ROWS, (long long)c->max_batch * c->max_ctx);
+  const size_t D = d.D, nq = D + 2 * (size_t)d.H_KV * d.HD, F = d.FFN;
+  if ((size_t)rows > R || prepare_prefill_kernels()) return false;
+  struct Part {
+    void **p;
+    size_t bytes;
+  };
+  const Part parts[] = {
+      {(void **)&c->pf_q, sizeof(double) * R * D},
+      {(void **)&c->pf_h_m, 2 * R * D},     {(void **)&c->pf_h_e, R * D / 16},
+      {(void **)&c->pf_h1_m, 2 * R * D},    {(void **)&c->pf_h1_e, R * D / 16},
+      {(void **)&c->pf_qkv_m, 2 * R * nq},  {(void **)&c->pf_qkv_e, R * nq / 16},
+      {(void **)&c->pf_att_m, 2 * R * D},   {(void **)&c->pf_att_e, R * D / 16},
+      {(void **)&c->pf_mlp_m, 2 * R * F},   {(void **)&c->pf_mlp_e, R * F / 16},
+      {(void **)&c->pf_xn_m, 2 * R * D},    {(void **)&c->pf_xn_e, R * D / 16},
+  };
+  auto padded = [](size_t n) { return (n + 255) & ~(size_t)255; };
+  size_t total = 0;
+  for (const Part &q : parts) total += padded(q.bytes);
+  uint8_t *block = nullptr;
+  if (c->alloc((void **)&block, total)) {
+    (void)hipGetLastError();   // not the next launch's error
+    return false;
+  }
+  for (const Part &q : parts) {
+    *q.p = block;
+    block += padded(q.bytes);
+  }
+  c->pf_rows = (int)R;
+  return true;
+}
+
 // Steps 0 .. n_prompt-1 of a decode as passes over the prompt's positions
 // (bfp_prefill.hip): the cache rows and the history those steps leave.
 int prefill(bfp_ctx *c, const int *dprompt, int n_prompt, int batch, int16_t *dhm, int8_t *dhe, int steps) {
   const bfp_dims &d = c->d;
   hipStream_t s = c->stream;
   const int n = prefill_chunk(batch, n_prompt), rows = batch * n;
-  if (rows > c->pf_rows) {
-    // the most rows any call of this context takes, at once
-    const size_t R = (size_t)std::min<long long>(PF_ROWS, (long long)c->max_batch * c->max_ctx);
-    const size_t D = d.D, nq = D + 2 * (size_t)d.H_KV * d.HD, F = d.FFN;
-    BFP_TRY(prepare_prefill_kernels());
-    BFP_TRY(c->alloc((void **)&c->pf_h_m, 2 * R * D));
-    BFP_TRY(c->alloc((void **)&c->pf_h_e, R * D / 16));
-    BFP_TRY(c->alloc((void **)&c->pf_h1_m, 2 * R * D));
-    BFP_TRY(c->alloc((void **)&c->pf_h1_e, R * D / 16));
-    BFP_TRY(c->alloc((void **)&c->pf_qkv_m, 2 * R * nq));
-    BFP_TRY(c->alloc((void **)&c->pf_qkv_e, R * nq / 16));
-    BFP_TRY(c->alloc((void **)&c->pf_att_m, 2 * R * D));
-    BFP_TRY(c->alloc((void **)&c->pf_att_e, R * D / 16));
-    BFP_TRY(c->alloc((void **)&c->pf_mlp_m, 2 * R * F));
-    BFP_TRY(c->alloc((void **)&c->pf_mlp_e, R * F / 16));
-    BFP_TRY(c->alloc((void **)&c->pf_xn_m, 2 * R * D));
-    BFP_TRY(c->alloc((void **)&c->pf_xn_e, R * D / 16));
-    BFP_TRY(c->alloc((void **)&c->pf_q, sizeof(double) * R * D));
-    c->pf_rows = (int)R;
-  }
   if (rows > c->pf_rows) return set_err(BFP_EINVAL, "prefill: %d rows of %d", rows, c->pf_rows);
   PrefillArgs a{};
   a.batch = batch;
@@ -616,15 +634,15 @@ int prefill(bfp_ctx *c, const int *dprompt, int n_prompt, int batch, int16_t *dh
 }
 
 // The steps a decode runs as prompt passes: the prompt's, when it is long
-// enough to pay for a pass and nothing asks for each step on its own (the
-// FPGA loop records every step's prediction; direct launches, step times,
-// traces and the abort hook are per step).
-int prefill_steps(int batch, int n_prompt, int flags, bool persist) {
+// enough to pay for a pass, there is memory for its rows and nothing asks for
+// each step on its own (the FPGA loop records every step's prediction; direct
+// launches, step times, traces and the abort hook are per step).
+int prefill_steps(bfp_ctx *c, int batch, int n_prompt, int flags, bool persist) {
   const int per_step = BFP_DECODE_RTL_LOOP | BFP_DECODE_NO_GRAPH | BFP_DECODE_STEP_TIMES | BFP_DECODE_TRACE |
                        BFP_DECODE_ABORT_TEST;
   if (flags & per_step) return 0;
   const int n = prefill_chunk(batch, n_prompt);
-  return n >= (persist ? PF_MIN_PERSIST : PF_MIN) ? n_prompt : 0;
+  return n >= (persist ? PF_MIN_PERSIST : PF_MIN) && prefill_ready(c, batch * n) ? n_prompt : 0;
 }
 
 // The whole batch-1 decode as one persistent launch (bfp_persist.hip);
@@ -1524,7 +1542,7 @@ int bfp_decode(bfp_ctx *c, const int32_t *prompt, int n_prompt, int n_gen, int b
   int grid = 0;
   if (batch == 1 && !(flags & (BFP_DECODE_NO_GRAPH | BFP_DECODE_NO_PERSIST)) && persist_enabled() &&
       persist_plan(d, c->max_ctx, c->device, pa, grid)) {
-    const int step0 = prefill_steps(batch, n_prompt, flags, true);
+    const int step0 = prefill_steps(c, batch, n_prompt, flags, true);
     BFP_TRY(decode_persist(c, pa, grid, dprompt, n_prompt, n_gen, dout, dhm, dhe, rtl_loop,
                            (flags & BFP_DECODE_TRACE) != 0, (flags & BFP_DECODE_ABORT_TEST) != 0, step0,
                            prompt[step0 ? n_prompt - 1 : 0], hist));
@@ -1533,7 +1551,7 @@ int bfp_decode(bfp_ctx *c, const int32_t *prompt, int n_prompt, int n_gen, int b
   c->last_path = (flags & BFP_DECODE_NO_GRAPH) ? BFP_PATH_EAGER : BFP_PATH_GRAPH;
   // the first step0 steps as prompt passes; the step after them feeds the
   // last prompt token once more
-  const int step0 = prefill_steps(batch, n_prompt, flags, false);
+  const int step0 = prefill_steps(c, batch, n_prompt, flags, false);
   std::vector<int> st(batch + 2, 0);   // step, next inputs, k_ctl_embed's arrival count
   st[0] = step0;
   for (int b = 0; b < batch; ++b) st[1 + b] = prompt[b * n_prompt + (step0 ? n_prompt - 1 : 0)];
