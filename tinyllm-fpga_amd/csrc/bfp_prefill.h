@@ -26,11 +26,11 @@ struct PrefillArgs {
 // Most rows of one pass.
 constexpr int PF_ROWS = 1024;
 // Fewest positions a pass is made for, against the persistent batch-1 decode
-// and against a batch's steps.  Measured at SmolLM2's 30 layers, prompt part
-// of a decode, pass against steps: batch 1, 3 positions ~2.0 / 1.59 ms, 4
-// 1.99 / 2.10, 8 2.02 / 4.17; 2 positions at batch 2 1.72 / 1.82, batch 5
-// 1.76 / 3.17, batch 64 2.51 / 2.94.  (A pass of few rows is 8 launches a
-// layer, 66 us, whatever their number.)
+// and against a batch's steps.  Calls at SmolLM2's 30 layers with 4 tokens
+// generated, ms, pass / steps: batch 1, 3 positions about 3.98 / 3.86, 4 3.99 /
+// 4.38, 6 4.00 / 5.43; 2 positions at batch 2 4.99 / 5.16, 5 5.30 / 5.55, 15
+// 6.57 / 7.42, 16 7.21 / 8.41, 64 8.36 / 9.16.  (A pass of few rows is 8
+// launches a layer whatever their number.)
 constexpr int PF_MIN_PERSIST = 4;
 constexpr int PF_MIN = 2;
 

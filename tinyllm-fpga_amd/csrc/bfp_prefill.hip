@@ -11,8 +11,9 @@
 // SkylakeX ddot scores, numpy's softmax sum, the ascending-t AV chain -- is
 // the decode kernels', so the cache rows and outputs are bit-identical to
 // the step-by-step loop's.  A 1000-token prompt and 24 tokens at SmolLM2's
-// width and batch 1 take 42 ms so, against 829 step by step; 5 sequences of
-// 23 + 25 tokens 47 against 81.
+// width and batch 1 take 36 ms so, of which the pass is 12, against 828 step by
+// step; a layer of the 1000-row pass is 405 us: 151 of attention, 232 of
+// matvecs.
 #include <stdint.h>
 
 #include <algorithm>
