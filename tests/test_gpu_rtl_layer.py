@@ -97,3 +97,12 @@ def test_rtl_layer_exponent_rises(gpu, spread):
         for name in NAMES:
             assert (st[name][1] == want[name][1]).all() and (st[name][0] == want[name][0]).all(), (pos, name)
     gm.close()
+
+
+@pytest.mark.parametrize("ffn", [80, 176, 1712])
+def test_rtl_layer_odd_ffn_tiles(gpu, ffn):
+    """An odd number of input tiles for D (5, 11, 107): the matvec's LDS parts
+    behind one another at sizes that are no multiple of 16 bytes."""
+    d, om, gm = _setup(dict(TINY, FFN=ffn, NL=1), ffn)
+    _run(d, om, gm, 0, [(p, p) for p in range(2)], seed=ffn)
+    gm.close()

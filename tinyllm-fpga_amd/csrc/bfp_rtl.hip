@@ -729,6 +729,32 @@ struct RomGamma {
   __device__ __forceinline__ void operator()(int i, int &m, int &e) const { m = quantize16_lanes(g[i], e); }
 };
 
+// LDS of a k_rl_mv workgroup of NC chunks over nT input tiles, in bytes from
+// the start: the tile sums (at 0), their exponents, the input in the matvec's
+// form, and where the input is a norm's output (NORM) that norm's tile sums;
+// the exponents of both.  The input is read 16 bytes at a time and nT may be
+// odd (FFN is any multiple of 16), so the parts stand in the order of their
+// alignment.
+struct RlMvLds {
+  int El, xs, sums, xes, sexp, bytes;
+};
+template <int NC, bool NORM>
+__host__ __device__ constexpr RlMvLds rl_mv_lds(int nT) {
+  const int El = NC * nT * 128, xs = El + NC * nT * 64, sums = xs + nT * 64, xes = sums + (NORM ? nT * 8 : 0),
+            sexp = xes + nT * 4;
+  return {El, xs, sums, xes, sexp, sexp + (NORM ? nT * 4 : 0)};
+}
+template <int NC, bool NORM>
+constexpr bool rl_mv_lds_aligned() {
+  for (int nT = 1; nT <= 108; ++nT) {
+    const RlMvLds o = rl_mv_lds<NC, NORM>(nT);
+    if (o.xs % 16 || o.sums % 8 || o.El % 4 || o.xes % 4 || o.sexp % 4 || o.bytes > 65536) return false;
+  }
+  return true;
+}
+static_assert(rl_mv_lds_aligned<1, true>() && rl_mv_lds_aligned<1, false>() && rl_mv_lds_aligned<2, true>(),
+              "the parts of k_rl_mv's LDS are aligned and fit a workgroup's default limit");
+
 // The layer's matvecs, one 16-row output chunk per workgroup, every weight
 // load issued before the input is staged.
 //   OP 0: Q|K|V from NORM1(h, G1)  (chunks of qkv, re-tiled per chunk)
@@ -738,23 +764,26 @@ struct RomGamma {
 template <int NW, int op>
 __global__ __launch_bounds__(64 * NW) void k_rl_mv(RtlArgs a) {
   constexpr int TPT = 3, NC = op == 2 ? 2 : 1;
-  extern __shared__ long long rl_lds[];
+  constexpr bool NORM = op == 0 || op == 2;
+  extern __shared__ __align__(16) long long rl_lds[];
   const LayerArgs &L = a.L;
   const int c = blockIdx.x;
   const int nT = (op == 3 ? L.FFN : L.D) / 16;
-  long long *Sl = rl_lds;                                  // NC x nT x 16
-  long long *sums = Sl + NC * nT * 16;                     // nT
-  int *El = reinterpret_cast<int *>(sums + nT);            // NC x nT x 16
-  int *xs = El + NC * nT * 16;                             // nT x 16
-  int *xes = xs + nT * 16;                                 // nT
-  int *sexp = xes + nT;                                    // nT
+  const RlMvLds o = rl_mv_lds<NC, NORM>(nT);
+  char *lds = reinterpret_cast<char *>(rl_lds);
+  long long *Sl = rl_lds;                                       // NC x nT x 16
+  long long *sums = reinterpret_cast<long long *>(lds + o.sums);   // nT
+  int *El = reinterpret_cast<int *>(lds + o.El);                // NC x nT x 16
+  int *xs = reinterpret_cast<int *>(lds + o.xs);                // nT x 16
+  int *xes = reinterpret_cast<int *>(lds + o.xes);              // nT
+  int *sexp = reinterpret_cast<int *>(lds + o.sexp);            // nT
   const uint4 *wm = op == 0 ? L.w_qkv_m : (op == 1 ? L.w_o_m : (op == 2 ? L.w_gu_m : L.w_d_m));
   const int8_t *we = op == 0 ? L.w_qkv_e : (op == 1 ? L.w_o_e : (op == 2 ? L.w_gu_e : L.w_d_e));
   ChunkRegs<TPT> R[NC];
 #pragma unroll
   for (int k = 0; k < NC; ++k)
     load_chunk_nb<NW, TPT>(R[k], wm + (size_t)(NC * c + k) * nT * 32, we + (size_t)(NC * c + k) * nT * 16, nT);
-  if constexpr (op == 0 || op == 2) {
+  if constexpr (NORM) {
     const StageDump *sd = c == 0 ? L.dump : nullptr;
     constexpr int st = op == 0 ? ST_N1 : ST_N2;
     rms_block(op == 0 ? L.h_m : L.h1_m, op == 0 ? L.h_e : L.h1_e, RomGamma{op == 0 ? L.g1 : L.g2}, L.D, sums, sexp,
@@ -1334,7 +1363,8 @@ int rl_mv(const RtlArgs &a, int nT, int n_wg, hipStream_t s) {
   const int nw = (nT + 11) / 12;   // 3 tiles per lane, 4 tile lanes per wave
   rl_mv_fn f = rl_mv_kernel<OP>(nw);
   if (!f) return set_err(BFP_EINVAL, "rtl layer: %d input tiles unsupported", nT);
-  hipLaunchKernelGGL(f, dim3(n_wg), dim3(64 * nw), (size_t)nT * ((OP == 2 ? 2 : 1) * 192 + 80), s, a);
+  const size_t lds = rtl::rl_mv_lds<OP == 2 ? 2 : 1, OP == 0 || OP == 2>(nT).bytes;
+  hipLaunchKernelGGL(f, dim3(n_wg), dim3(64 * nw), lds, s, a);
   return launch_status("rtl layer matvec");
 }
 }  // namespace
