@@ -144,6 +144,10 @@ __device__ __forceinline__ mx_s2 mx_pair(int v) { return __builtin_bit_cast(mx_s
 __device__ __forceinline__ int mx_bits(mx_s2 v) { return __builtin_bit_cast(int, v); }
 
 // The float64 rounding mode of the wave: toward minus infinity, or nearest.
+// Volatile statements keep their order among themselves, but nothing orders
+// ordinary float64 operations against them: between the two only exact ones
+// may stand (the conversions and S below).  tests/test_mx_rounding_code.py
+// reads the built kernels for that.
 __device__ __forceinline__ void mx_round_down() {
   asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 2\n\ts_nop 1");
 }
