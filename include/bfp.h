@@ -227,6 +227,16 @@ typedef struct bfp_ctx bfp_ctx;
 bfp_ctx *bfp_create(const bfp_dims *dims, int device, int max_batch);
 void bfp_destroy(bfp_ctx *ctx);
 int bfp_get_dims(const bfp_ctx *ctx, bfp_dims *out);
+/* Memory that a context uses where it can have it and does without
+ * otherwise, with the same results: the bits of what it holds now (no
+ * reference counterpart; for tests and tuning).
+ *   BFP_MEM_HISTORY  the pinned pieces through which bfp_decode's history
+ *                    reaches the host while the decode runs (4.3 MB, made on
+ *                    first use); else one copy after it.
+ * With the environment variable BFP_OPTIONAL_MEMORY=0 when the context is
+ * made, it asks for none of it. */
+#define BFP_MEM_HISTORY 1
+int bfp_optional_memory(const bfp_ctx *ctx);
 
 /* Load one tensor (which = enum bfp_which).  Matrices (rows x cols as in
  * full.py:312-318) from float32 -- quantize_W on the device (full.py:110-119)

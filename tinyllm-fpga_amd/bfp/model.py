@@ -301,6 +301,13 @@ class BfpModel:
             lib().bfp_decode_step_times(self._h, _p(out), n)
         return out
 
+    def optional_memory(self):
+        """What this context holds of the memory it can do without
+        (include/bfp.h, bfp_optional_memory): a set of 'history'.  The
+        environment variable BFP_OPTIONAL_MEMORY=0 at construction: none."""
+        f = lib().bfp_optional_memory(self._h)
+        return {n for b, n in ((1, "history"),) if f & b}
+
     def decode_path(self):
         """'persist', 'graph' or 'eager': how the last decode ran."""
         return {0: "graph", 1: "persist", 2: "eager"}.get(lib().bfp_decode_path(self._h), None)

@@ -135,6 +135,7 @@ struct bfp_ctx {
   hipStream_t hist_stream = nullptr;
   hipEvent_t hist_ev[2] = {nullptr, nullptr};
   uint8_t *hist_pin = nullptr;
+  bool optional = true;   // BFP_OPTIONAL_MEMORY when the context was made
   size_t hist_slot = 0;
   int last_path = -1;   // BFP_PATH_* of the last decode
   int last_form = -1;   // BFP_FORM_* of the last decode
@@ -151,6 +152,17 @@ struct bfp_ctx {
     }
     allocs.push_back(*p);
     return BFP_OK;
+  }
+  // Pinned memory that the context can do without: null when there is none
+  // (or it is not to be asked for), with no error left behind.
+  uint8_t *pinned_optional(size_t bytes) {
+    void *p = nullptr;
+    if (!optional) return nullptr;
+    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();   // not the next launch's error
+      return nullptr;
+    }
+    return static_cast<uint8_t *>(p);
   }
   // Fine-grained device memory: device-coherent (SC1) accesses to it are
   // faster than to ordinary allocations (a cross-XCD hand-off measured
@@ -436,6 +448,7 @@ constexpr int HIST_LAG = 8;   // steps
 // the last step only the last marks' steps are left to copy.  64 sequences x
 // 32 steps x 30 layers x 576 (73 MB): the call's time past the decode's last
 // kernel 4.0 ms, 10.3 with one copy at the end; the decode itself takes the same.
+// Without pinned memory for the pieces it is that one copy.
 class HistOut {
  public:
   HistOut(bfp_ctx *c, int batch, int steps, const int16_t *dm, const int8_t *de, int16_t *m, int8_t *e)
@@ -448,8 +461,9 @@ class HistOut {
   bool on() const { return dm_ != nullptr; }
   // The steps below `upto` are complete once the decode's stream gets here.
   int mark(int upto) {
-    if (!on() || upto <= (marks_.empty() ? done_ : marks_.back().upto)) return BFP_OK;
-    if (!c_->hist_ev[1]) BFP_TRY(prepare());
+    if (!on() || whole_ || upto <= (marks_.empty() ? done_ : marks_.back().upto)) return BFP_OK;
+    BFP_TRY(prepare());
+    if (whole_) return BFP_OK;
     Mark k{upto, nullptr};
     HIP_TRY(hipEventCreateWithFlags(&k.ev, hipEventDisableTiming));
     marks_.push_back(k);
@@ -480,6 +494,11 @@ class HistOut {
   int finish() {
     if (!on()) return BFP_OK;
     BFP_TRY(mark(steps_));
+    if (whole_) {
+      HIP_TRY(hipMemcpy(m_, dm_, row_ * steps_ * batch_, hipMemcpyDeviceToHost));
+      HIP_TRY(hipMemcpy(e_, de_, row_ / 32 * steps_ * batch_, hipMemcpyDeviceToHost));
+      return BFP_OK;
+    }
     BFP_TRY(copy(steps_));
     for (int i = 0; i < 2; ++i) {
       BFP_TRY(store(next_));
@@ -499,15 +518,12 @@ class HistOut {
   static constexpr size_t PIECE = 2 << 20;
 
   int prepare() {
+    if (c_->hist_ev[1]) return BFP_OK;
     // mantissas, then exponents (a 32nd), of a piece
     c_->hist_slot = (std::max(PIECE, row_) * 33 / 32 + 255) & ~(size_t)255;
-    if (!c_->hist_pin) {
-      void *p = nullptr;
-      hipError_t e = hipHostMalloc(&p, 2 * c_->hist_slot, hipHostMallocDefault);
-      if (e != hipSuccess)
-        return set_err(BFP_ENOMEM, "hipHostMalloc(%zu): %s", 2 * c_->hist_slot, hipGetErrorString(e));
-      c_->hist_pin = static_cast<uint8_t *>(p);
-    }
+    if (!c_->hist_pin) c_->hist_pin = c_->pinned_optional(2 * c_->hist_slot);
+    whole_ = !c_->hist_pin;
+    if (whole_) return BFP_OK;
     for (hipEvent_t &ev : c_->hist_ev)
       if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     return BFP_OK;
@@ -549,6 +565,7 @@ class HistOut {
   int16_t *m_;
   int8_t *e_;
   const size_t row_;   // bytes of a step's mantissas, one sequence
+  bool whole_ = false;   // no pinned pieces: one copy at the end
   int done_ = 0, next_ = 0;
   Piece slot_[2] = {};
   std::deque<Mark> marks_;
@@ -784,6 +801,7 @@ bfp_ctx *bfp_create(const bfp_dims *dims, int device, int max_batch) {
   c->device = device;
   c->max_batch = max_batch;
   c->max_ctx = dims->MAX_CTX;
+  if (const char *v = getenv("BFP_OPTIONAL_MEMORY")) c->optional = atoi(v) != 0;
   const bfp_dims &d = c->d;
   const int KV = d.H_KV * d.HD;
   const size_t nq = (size_t)d.D + 2 * KV;
@@ -883,6 +901,10 @@ int bfp_get_dims(const bfp_ctx *c, bfp_dims *out) {
   if (!c || !out) return set_err(BFP_EINVAL, "null argument");
   *out = c->d;
   return BFP_OK;
+}
+
+int bfp_optional_memory(const bfp_ctx *c) {
+  return c ? (c->hist_pin ? BFP_MEM_HISTORY : 0) : 0;
 }
 
 // Load one weight tensor.  Matrices: from float32 (quantize_W on the device,
