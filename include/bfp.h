@@ -232,10 +232,14 @@ int bfp_get_dims(const bfp_ctx *ctx, bfp_dims *out);
  * reference counterpart; for tests and tuning).
  *   BFP_MEM_HISTORY  the pinned pieces through which bfp_decode's history
  *                    reaches the host while the decode runs (4.3 MB, made on
- *                    first use); else one copy after it.
+ *                    first use); else one copy after it;
+ *   BFP_MEM_HEAD     the bounded head's copy of the embedding and its
+ *                    buffers (2 bytes an element and 24 a row; contexts for
+ *                    2 sequences and more, D at most 576); else the full head.
  * With the environment variable BFP_OPTIONAL_MEMORY=0 when the context is
  * made, it asks for none of it. */
 #define BFP_MEM_HISTORY 1
+#define BFP_MEM_HEAD 2
 int bfp_optional_memory(const bfp_ctx *ctx);
 
 /* Load one tensor (which = enum bfp_which).  Matrices (rows x cols as in

@@ -497,3 +497,30 @@ def test_history_without_pinned_memory(gpu, monkeypatch, batch, n_prompt, n_gen)
     for toks, (hm, he) in got[1:]:
         assert np.array_equal(toks, got[0][0])
         assert np.array_equal(hm, got[0][1][0]) and np.array_equal(he, got[0][1][1])
+
+
+@pytest.mark.parametrize("max_batch", [1, 2, 15, 33])
+def test_head_without_bounded_buffers(gpu, monkeypatch, max_batch):
+    """A context whose bounded head's buffers cannot be had is made all the
+    same and takes the full head: the same tokens, one embedding after
+    another."""
+    from bfp import Dims, synth
+    from bfp.model import BfpModel
+    d = Dims(D=192, H_Q=3, H_KV=1, HD=64, FFN=256, NL=1, MAX_CTX=16, VOCAB=1040)
+    rng = np.random.default_rng(max_batch)
+    hm = rng.integers(-20000, 20000, size=(max_batch, d.D)).astype(np.int16)
+    he = np.zeros((max_batch, d.D // 16), np.int8)
+    P = rng.integers(0, d.VOCAB, size=(max_batch, 3)).astype(np.int32)
+    got = []
+    for held in (True, False):
+        monkeypatch.setenv("BFP_OPTIONAL_MEMORY", str(int(held)))
+        gm = BfpModel(d, max_batch=max_batch)
+        assert ("head" in gm.optional_memory()) == (held and max_batch > 1)
+        for seed in (1, 2):
+            gm.load_fp32(synth.make_model(d, seed=seed))
+            full, lg = gm.head(hm, he, logits=True)
+            am, _ = gm.head(hm, he)
+            assert list(am) == list(full) == [int(np.argmax(r)) for r in lg]
+            got.append((list(am), gm.decode(P, 8)[0].tolist()))
+        gm.close()
+    assert got[:2] == got[2:]

@@ -303,10 +303,11 @@ class BfpModel:
 
     def optional_memory(self):
         """What this context holds of the memory it can do without
-        (include/bfp.h, bfp_optional_memory): a set of 'history'.  The
-        environment variable BFP_OPTIONAL_MEMORY=0 at construction: none."""
+        (include/bfp.h, bfp_optional_memory): a set of 'history' and
+        'head'.  The environment variable BFP_OPTIONAL_MEMORY=0 at
+        construction: none."""
         f = lib().bfp_optional_memory(self._h)
-        return {n for b, n in ((1, "history"),) if f & b}
+        return {n for b, n in ((1, "history"), (2, "head")) if f & b}
 
     def decode_path(self):
         """'persist', 'graph' or 'eager': how the last decode ran."""

@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <cmath>
 #include <deque>
+#include <initializer_list>
 #include <vector>
 
 #include "bfp.h"
@@ -152,6 +153,33 @@ struct bfp_ctx {
     }
     allocs.push_back(*p);
     return BFP_OK;
+  }
+  // Device memory that the context can do without, all parts in one block:
+  // false, with the parts null, when there is none (or it is not to be asked
+  // for), with no error left behind.
+  struct Part {
+    void **p;
+    size_t bytes;
+  };
+  bool alloc_optional(std::initializer_list<Part> parts) {
+    auto padded = [](size_t n) { return (n + 255) & ~(size_t)255; };
+    size_t total = 0;
+    for (const Part &q : parts) {
+      *q.p = nullptr;
+      total += padded(q.bytes);
+    }
+    uint8_t *block = nullptr;
+    if (!optional) return false;
+    if (hipMalloc((void **)&block, total) != hipSuccess) {
+      (void)hipGetLastError();   // not the next launch's error
+      return false;
+    }
+    allocs.push_back(block);
+    for (const Part &q : parts) {
+      *q.p = block;
+      block += padded(q.bytes);
+    }
+    return true;
   }
   // Pinned memory that the context can do without: null when there is none
   // (or it is not to be asked for), with no error left behind.
@@ -580,31 +608,16 @@ bool prefill_ready(bfp_ctx *c, int rows) {
   const size_t R = (size_t)std::min<long long>(PF_ROWS, (long long)c->max_batch * c->max_ctx);
   const size_t D = d.D, nq = D + 2 * (size_t)d.H_KV * d.HD, F = d.FFN;
   if ((size_t)rows > R || prepare_prefill_kernels()) return false;
-  struct Part {
-    void **p;
-    size_t bytes;
-  };
-  const Part parts[] = {
-      {(void **)&c->pf_q, sizeof(double) * R * D},
-      {(void **)&c->pf_h_m, 2 * R * D},     {(void **)&c->pf_h_e, R * D / 16},
-      {(void **)&c->pf_h1_m, 2 * R * D},    {(void **)&c->pf_h1_e, R * D / 16},
-      {(void **)&c->pf_qkv_m, 2 * R * nq},  {(void **)&c->pf_qkv_e, R * nq / 16},
-      {(void **)&c->pf_att_m, 2 * R * D},   {(void **)&c->pf_att_e, R * D / 16},
-      {(void **)&c->pf_mlp_m, 2 * R * F},   {(void **)&c->pf_mlp_e, R * F / 16},
-      {(void **)&c->pf_xn_m, 2 * R * D},    {(void **)&c->pf_xn_e, R * D / 16},
-  };
-  auto padded = [](size_t n) { return (n + 255) & ~(size_t)255; };
-  size_t total = 0;
-  for (const Part &q : parts) total += padded(q.bytes);
-  uint8_t *block = nullptr;
-  if (c->alloc((void **)&block, total)) {
-    (void)hipGetLastError();   // not the next launch's error
+  if (!c->alloc_optional({
+          {(void **)&c->pf_q, sizeof(double) * R * D},
+          {(void **)&c->pf_h_m, 2 * R * D},     {(void **)&c->pf_h_e, R * D / 16},
+          {(void **)&c->pf_h1_m, 2 * R * D},    {(void **)&c->pf_h1_e, R * D / 16},
+          {(void **)&c->pf_qkv_m, 2 * R * nq},  {(void **)&c->pf_qkv_e, R * nq / 16},
+          {(void **)&c->pf_att_m, 2 * R * D},   {(void **)&c->pf_att_e, R * D / 16},
+          {(void **)&c->pf_mlp_m, 2 * R * F},   {(void **)&c->pf_mlp_e, R * F / 16},
+          {(void **)&c->pf_xn_m, 2 * R * D},    {(void **)&c->pf_xn_e, R * D / 16},
+      }))
     return false;
-  }
-  for (const Part &q : parts) {
-    *q.p = block;
-    block += padded(q.bytes);
-  }
   c->pf_rows = (int)R;
   return true;
 }
@@ -843,12 +856,6 @@ bfp_ctx *bfp_create(const bfp_dims *dims, int device, int max_batch) {
       (rc = c->alloc((void **)&c->embed, sizeof(float) * (size_t)d.VOCAB * d.D)) ||
       (max_batch >= HEAD_SEQ_MIN && d.D % 64 == 0 && d.D <= 576 &&
        (rc = c->alloc((void **)&c->embedp, sizeof(float) * (size_t)d.VOCAB * d.D))) ||
-      (max_batch >= HEADQ_MIN && d.D % 64 == 0 && d.D <= 576 &&
-       ((rc = c->alloc((void **)&c->embq, (size_t)d.VOCAB * d.D * 2)) ||
-        (rc = c->alloc((void **)&c->embq_meta, sizeof(HeadQRow) * (size_t)d.VOCAB)) ||
-        (rc = c->alloc((void **)&c->hq_x, (size_t)(B + 15) / 16 * (d.D / 64) * 64 * 32)) ||
-        (rc = c->alloc((void **)&c->hq_seq, sizeof(HeadQSeq) * B)) ||
-        (rc = c->alloc((void **)&c->hq_blk, sizeof(double2) * B * (d.VOCAB / 16))))) ||
       (rc = c->alloc((void **)&c->h_m, 2 * B * d.D)) || (rc = c->alloc((void **)&c->h_e, B * d.D / 16)) ||
       (rc = c->alloc((void **)&c->h1_m, 2 * B * d.D)) ||
       (rc = c->alloc((void **)&c->h1_e, B * d.D / 16)) ||
@@ -877,6 +884,13 @@ bfp_ctx *bfp_create(const bfp_dims *dims, int device, int max_batch) {
     delete c;
     return nullptr;
   }
+  // the bounded head's, after all that the context cannot do without
+  if (max_batch >= HEADQ_MIN && d.D % 64 == 0 && d.D <= 576)
+    c->alloc_optional({{(void **)&c->embq, (size_t)d.VOCAB * d.D * 2},
+                       {(void **)&c->embq_meta, sizeof(HeadQRow) * (size_t)d.VOCAB},
+                       {(void **)&c->hq_x, (size_t)(B + 15) / 16 * (d.D / 64) * 64 * 32},
+                       {(void **)&c->hq_seq, sizeof(HeadQSeq) * B},
+                       {(void **)&c->hq_blk, sizeof(double2) * B * (d.VOCAB / 16)}});
   if (prepare_layer_kernels(c->max_ctx, d.D, d.FFN) || prepare_head_kernels(d.D)) {
     delete c;
     return nullptr;
@@ -904,7 +918,7 @@ int bfp_get_dims(const bfp_ctx *c, bfp_dims *out) {
 }
 
 int bfp_optional_memory(const bfp_ctx *c) {
-  return c ? (c->hist_pin ? BFP_MEM_HISTORY : 0) : 0;
+  return c ? (c->hist_pin ? BFP_MEM_HISTORY : 0) | (c->embq ? BFP_MEM_HEAD : 0) : 0;
 }
 
 // Load one weight tensor.  Matrices: from float32 (quantize_W on the device,
