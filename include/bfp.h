@@ -235,11 +235,15 @@ int bfp_get_dims(const bfp_ctx *ctx, bfp_dims *out);
  *                    first use); else one copy after it;
  *   BFP_MEM_HEAD     the bounded head's copy of the embedding and its
  *                    buffers (2 bytes an element and 24 a row; contexts for
- *                    2 sequences and more, D at most 576); else the full head.
+ *                    2 sequences and more, D at most 576); else the full head;
+ *   BFP_MEM_PROMPT   the rows of bfp_decode's prompt passes (at most 1024,
+ *                    about 18 D + 4 KV + 2 FFN bytes each, made on first use);
+ *                    else the prompt runs step by step.
  * With the environment variable BFP_OPTIONAL_MEMORY=0 when the context is
  * made, it asks for none of it. */
 #define BFP_MEM_HISTORY 1
 #define BFP_MEM_HEAD 2
+#define BFP_MEM_PROMPT 4
 int bfp_optional_memory(const bfp_ctx *ctx);
 
 /* Load one tensor (which = enum bfp_which).  Matrices (rows x cols as in
@@ -432,6 +436,13 @@ int bfp_decode_path(const bfp_ctx *ctx);
 #define BFP_FORM_PIPE 32
 #define BFP_FORM_ATT_GROUP 64
 int bfp_decode_form(const bfp_ctx *ctx);
+/* How many of the last bfp_decode's steps ran as passes over the prompt's
+ * positions (no reference counterpart; for tests and tuning): n_prompt, or 0
+ * where every position was a step (prompts of 1 position, or of at most 3 on
+ * the persistent path; more sequences than a pass takes; flags that ask for
+ * each step on its own; no memory for the passes' rows); -1 before any
+ * decode. */
+int bfp_decode_prompt_pass(const bfp_ctx *ctx);
 /* The stage trace of the last decode run with BFP_DECODE_TRACE on the
  * persistent path: per (step, layer) 20 stamps -- 0/1 Q|K|V input ready /
  * output stored, 2 the first attention job's q|k|v input in, 3 attention

@@ -1,6 +1,7 @@
 """GPU: a decode whose prompt goes through the layers as passes over many
 positions (bfp_prefill.hip) against the same decode step by step (direct
-launches, which never take a pass) -- tokens, every layer's output at every
+launches, which never take a pass; the number of steps that ran as passes is
+checked on both sides) -- tokens, every layer's output at every
 step, the cache rows and the tokens generated from them, bit for bit: at the
 edges of the attention's tiles (positions a workgroup, 32-row V blocks,
 256-row K blocks), over several passes, for ragged and split head groups, and
@@ -50,10 +51,42 @@ def test_prompt_pass_equals_steps(gpu, name):
             return toks, hm, he, kv
 
         want = both(graph=False)
+        assert gm.prompt_pass_steps() == 0
         got = both()
+        # at batch 1 these contexts decode persistently, where a pass is made from 4 positions
+        taken = n_prompt >= (4 if gm.decode_path() == "persist" else 2)
+        assert gm.prompt_pass_steps() == (n_prompt if taken else 0)
         for a, b in zip(want[:3], got[:3]):
             assert np.array_equal(a, b)
         for (wk, wv), (gk, gv) in zip(want[3], got[3]):
             for a, b in zip((*wk, *wv), (*gk, *gv)):
                 assert np.array_equal(a, b)
     gm.close()
+
+
+@pytest.mark.parametrize("batch", [1, 3, 17])
+def test_prompt_steps_without_memory_for_a_pass(gpu, monkeypatch, batch):
+    """Where there is no memory for a pass's rows the prompt runs step by
+    step: the same tokens, history and cache rows, call after call."""
+    from bfp import Dims, synth
+    from bfp.model import BfpModel
+    d = Dims(D=192, H_Q=3, H_KV=1, HD=64, FFN=256, NL=2, MAX_CTX=40, VOCAB=512)
+    fm = synth.make_model(d, seed=7)
+    P = np.random.default_rng(batch).integers(0, d.VOCAB, size=(batch, 11)).astype(np.int32)
+    got = []
+    for held in (True, False):
+        monkeypatch.setenv("BFP_OPTIONAL_MEMORY", str(int(held)))
+        gm = BfpModel(d, max_batch=batch)
+        gm.load_fp32(fm)
+        assert gm.prompt_pass_steps() is None
+        for _ in range(2):
+            gm.reset_kv()
+            toks, (hm, he) = gm.decode(P, 5, hist=True)
+            assert gm.prompt_pass_steps() == (11 if held else 0)
+            assert ("prompt" in gm.optional_memory()) == held
+            got.append([toks, hm, he] + [x for li in range(d.NL) for b in range(batch)
+                                         for t in gm.kv_io(li, b, 0, 16) for x in t])
+        gm.close()
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            assert np.array_equal(a, b)

@@ -93,6 +93,7 @@ SIGNATURES = {
     "bfp_decode_step_times": (i32, [vp, vp, i32]),
     "bfp_decode_path": (i32, [vp]),
     "bfp_decode_form": (i32, [vp]),
+    "bfp_decode_prompt_pass": (i32, [vp]),
     "bfp_optional_memory": (i32, [vp]),
     "bfp_decode_trace": (i32, [vp, vp, sz]),
     "bfp_vocab_open": (i32, [C.c_char_p, C.POINTER(vp)]),

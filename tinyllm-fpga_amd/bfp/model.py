@@ -303,11 +303,11 @@ class BfpModel:
 
     def optional_memory(self):
         """What this context holds of the memory it can do without
-        (include/bfp.h, bfp_optional_memory): a set of 'history' and
-        'head'.  The environment variable BFP_OPTIONAL_MEMORY=0 at
+        (include/bfp.h, bfp_optional_memory): a set of 'history',
+        'head' and 'prompt'.  The environment variable BFP_OPTIONAL_MEMORY=0 at
         construction: none."""
         f = lib().bfp_optional_memory(self._h)
-        return {n for b, n in ((1, "history"), (2, "head")) if f & b}
+        return {n for b, n in ((1, "history"), (2, "head"), (4, "prompt")) if f & b}
 
     def decode_path(self):
         """'persist', 'graph' or 'eager': how the last decode ran."""
@@ -330,6 +330,12 @@ class BfpModel:
             return ("single", "multi")[f]
         return ("mx" + ("+qkv_attn" if f & 4 else "") + ("+attn_group" if f & 64 else "")
                 + ("+norm_fused" if f & 8 else ""))
+
+    def prompt_pass_steps(self):
+        """How many of the last decode's steps ran as passes over the
+        prompt's positions: its prompt's length, or 0 (None before any)."""
+        n = lib().bfp_decode_prompt_pass(self._h)
+        return None if n < 0 else n
 
     def decode_trace(self):
         """Stamps (device clock, 100 MHz) of the last decode(trace=True): on

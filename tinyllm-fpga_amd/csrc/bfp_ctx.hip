@@ -140,6 +140,7 @@ struct bfp_ctx {
   size_t hist_slot = 0;
   int last_path = -1;   // BFP_PATH_* of the last decode
   int last_form = -1;   // BFP_FORM_* of the last decode
+  int last_pass = -1;   // steps of the last decode that ran as prompt passes
   float last_decode_ms = 0.f, last_gen_ms = 0.f;
   std::vector<float> step_ms;   // per-step device time of the last decode (BFP_DECODE_STEP_TIMES)
   std::vector<unsigned long long> trace;   // stage stamps of the last traced persistent decode
@@ -607,7 +608,11 @@ bool prefill_ready(bfp_ctx *c, int rows) {
   const bfp_dims &d = c->d;
   const size_t R = (size_t)std::min<long long>(PF_ROWS, (long long)c->max_batch * c->max_ctx);
   const size_t D = d.D, nq = D + 2 * (size_t)d.H_KV * d.HD, F = d.FFN;
-  if ((size_t)rows > R || prepare_prefill_kernels()) return false;
+  if ((size_t)rows > R) return false;
+  if (prepare_prefill_kernels()) {
+    (void)hipGetLastError();   // not the next launch's error
+    return false;
+  }
   if (!c->alloc_optional({
           {(void **)&c->pf_q, sizeof(double) * R * D},
           {(void **)&c->pf_h_m, 2 * R * D},     {(void **)&c->pf_h_e, R * D / 16},
@@ -670,9 +675,11 @@ int prefill(bfp_ctx *c, const int *dprompt, int n_prompt, int batch, int16_t *dh
 int prefill_steps(bfp_ctx *c, int batch, int n_prompt, int flags, bool persist) {
   const int per_step = BFP_DECODE_RTL_LOOP | BFP_DECODE_NO_GRAPH | BFP_DECODE_STEP_TIMES | BFP_DECODE_TRACE |
                        BFP_DECODE_ABORT_TEST;
+  c->last_pass = 0;
   if (flags & per_step) return 0;
   const int n = prefill_chunk(batch, n_prompt);
-  return n >= (persist ? PF_MIN_PERSIST : PF_MIN) && prefill_ready(c, batch * n) ? n_prompt : 0;
+  if (n < (persist ? PF_MIN_PERSIST : PF_MIN) || !prefill_ready(c, batch * n)) return 0;
+  return c->last_pass = n_prompt;
 }
 
 // The whole batch-1 decode as one persistent launch (bfp_persist.hip);
@@ -918,7 +925,8 @@ int bfp_get_dims(const bfp_ctx *c, bfp_dims *out) {
 }
 
 int bfp_optional_memory(const bfp_ctx *c) {
-  return c ? (c->hist_pin ? BFP_MEM_HISTORY : 0) | (c->embq ? BFP_MEM_HEAD : 0) : 0;
+  if (!c) return 0;
+  return (c->hist_pin ? BFP_MEM_HISTORY : 0) | (c->embq ? BFP_MEM_HEAD : 0) | (c->pf_rows ? BFP_MEM_PROMPT : 0);
 }
 
 // Load one weight tensor.  Matrices: from float32 (quantize_W on the device,
@@ -1752,6 +1760,7 @@ int bfp_decode(bfp_ctx *c, const int32_t *prompt, int n_prompt, int n_gen, int b
 
 int bfp_decode_path(const bfp_ctx *c) { return c ? c->last_path : -1; }
 int bfp_decode_form(const bfp_ctx *c) { return c ? c->last_form : -1; }
+int bfp_decode_prompt_pass(const bfp_ctx *c) { return c ? c->last_pass : -1; }
 
 int bfp_decode_trace(const bfp_ctx *c, uint64_t *out, size_t n) {
   if (!c || (!out && n > 0)) return set_err(BFP_EINVAL, "null argument");
