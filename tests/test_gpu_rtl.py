@@ -171,3 +171,22 @@ def test_rmsnorm_exponent_rises(gpu, D):
         want = ort.rtl_rmsnorm(xm, xe, gm, ge)
         for a, b in zip(got, want):
             assert np.array_equal(np.asarray(a).reshape(-1), np.asarray(b).reshape(-1)), order
+
+
+@pytest.mark.parametrize("D", [64, 176, 192, 208, 384, 400, 752, 768, 784])
+def test_rmsnorm_workgroup_sizes(gpu, D):
+    """The norm's workgroup has as many waves as its elements fill (three a
+    thread, at most four waves): at the edges of each size, several vectors
+    a launch, every exponent its own."""
+    from bfp import rtl
+    rng = np.random.default_rng(D)
+    B = 5
+    xm = rng.integers(-32768, 32768, (B, D)).astype(np.int16)
+    xe = rng.integers(-9, 10, (B, D // 16)).astype(np.int8)
+    gm = rng.integers(-32768, 32768, D).astype(np.int16)
+    ge = rng.integers(-2, 3, D // 16).astype(np.int8)
+    ym, ye = rtl.golden_rmsnorm(xm, xe, gm, ge)
+    for b in range(B):
+        wm, we = ort.rtl_rmsnorm(xm[b], xe[b], gm, ge)
+        assert np.array_equal(np.asarray(ym)[b].reshape(-1), np.asarray(wm).reshape(-1)), b
+        assert np.array_equal(np.asarray(ye)[b].reshape(-1), np.asarray(we).reshape(-1)), b
