@@ -190,3 +190,15 @@ def test_rmsnorm_workgroup_sizes(gpu, D):
         wm, we = ort.rtl_rmsnorm(xm[b], xe[b], gm, ge)
         assert np.array_equal(np.asarray(ym)[b].reshape(-1), np.asarray(wm).reshape(-1)), b
         assert np.array_equal(np.asarray(ye)[b].reshape(-1), np.asarray(we).reshape(-1)), b
+
+
+@pytest.mark.parametrize("n", [16, 64, 16 * 64, 16 * 65, 16 * 1023, 16 * 1024, 16 * 1025])
+def test_argmax_rows(gpu, n):
+    """Several rows a launch, at the edges of the workgroup's size (a thread a
+    chunk, 64 to 1024)."""
+    from bfp import rtl
+    rng = np.random.default_rng(n)
+    m = rng.integers(-32768, 32768, (9, n)).astype(np.int16)
+    e = rng.integers(-4, 5, (9, n)).astype(np.int8)
+    got = rtl.argmax(m, e)
+    assert list(got) == [ort.rtl_argmax(m[b], e[b]) for b in range(9)]
