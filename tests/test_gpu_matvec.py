@@ -266,10 +266,12 @@ def test_bad_shapes_raise(gpu):
         call("bfp_matvec_d", 0, 0, 15, 16, 1, 0, 0, 0, 0, 0, 0, 0, 0, 0, _dev.stream())
 
 
-@pytest.mark.parametrize("n_out,n_in", [(16, 16), (16, 48), (48, 32), (80, 144), (176, 1536)])
+@pytest.mark.parametrize("n_out,n_in", [(16, 16), (16, 48), (48, 32), (80, 144), (176, 1536), (80, 16), (4112, 16),
+                                        (112, 80), (48, 1712)])
 def test_quantize_pack_values(gpu, n_out, n_in):
     """The packing quantizer against the tile quantizer of float64 values,
-    bit for bit: odd tile counts, partial wave units, zero tiles, denormals,
+    bit for bit: odd tile counts (pairs of tiles that run on into the next 16
+    rows, and an odd number of tiles in all), zero tiles, denormals,
     values at and beside powers of two, the largest floats, infinities; the
     bytes behind both outputs are left alone."""
     import torch

@@ -16,6 +16,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <climits>
 
 #include "bfp.h"
@@ -150,18 +151,19 @@ __global__ void tile_quantize_kernel(const T *__restrict__ v, long long n_tiles,
 }
 
 // quantize_W straight into the device layout.  Bound by memory: 4 bytes in
-// and 2 1/16 out an element.  A wave takes QP_UNITS units of 16 rows (a chunk)
-// by two tiles with four elements a lane, so that each instruction covers
-// whole lines on both sides: a load 8 rows of 128 bytes, a store four runs of
-// 8 rows by 16 bytes (one tile's half of 8 columns).  49152 x 576: 29.8 us
-// (5.8 TB/s); a thread a tile, with lanes 64 bytes apart on the way in and 512
-// on the way out, took 49.6.
+// and 2 1/16 out an element.  A wave takes two tiles of 16 rows (a chunk), in
+// the layout's order, with four elements a lane, so that each instruction
+// covers whole lines on both sides: a load 8 rows of 128 bytes, a store four
+// runs of 8 rows by 16 bytes (one tile's half of 8 columns).  With an odd
+// number of tiles a row a pair runs on into the next chunk.  49152 x 576: 28.5
+// us a call (6.0 TB/s); a thread a tile, with lanes 64 bytes apart on the way
+// in and 512 on the way out, took 32.6.  Small tables want the waves: with
+// four pairs a wave 49152 x 80 took 6.1 us and x 400 24.4, so 4.9 and 22.1
+// (every call back to back has 4 us of launch in it).
 // The arithmetic is tile_exp_of's and tile_mant_of's on float32 values, in
 // float32 and bit for bit the same: scaling by a power of two is exact (a
 // result below the normal range rounds to 0 either way), and no float32 amax
 // lies within 709 * 2^-53 below a power of two, so the exponent is frexp's.
-constexpr int QP_UNITS = 4;
-
 __device__ __forceinline__ float quad_max(float v) {
   const int i = __float_as_int(v);
   v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, i, 0xB1, 0xf, 0xf, false)));   // lane ^ 1
@@ -169,54 +171,45 @@ __device__ __forceinline__ float quad_max(float v) {
   return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, j, 0x4E, 0xf, 0xf, false)));  // lane ^ 2
 }
 
-__global__ __launch_bounds__(256) void quantize_pack_f32_kernel(const float *__restrict__ W, unsigned units,
-                                                                int nT, int cstride, uint2 *__restrict__ Pm,
+__global__ __launch_bounds__(256) void quantize_pack_f32_kernel(const float *__restrict__ W, unsigned tiles,
+                                                                unsigned nT, int cstride, uint2 *__restrict__ Pm,
                                                                 int8_t *__restrict__ Pe) {
   const int l = threadIdx.x & 63;
-  const unsigned npair = (nT + 1) / 2;
-  const unsigned u0 = __builtin_amdgcn_readfirstlane((blockIdx.x * 4 + (threadIdx.x >> 6)) * QP_UNITS);
-  // lane: row 8j + (l >> 3) of the chunk, elements 4 (l & 3) .. of tile 2p + ((l >> 2) & 1)
-  float4 f[QP_UNITS][2];
+  // lane: row 8j + (l >> 3) of the chunk, elements 4 (l & 3) .. of the pair's tile (l >> 2) & 1
+  const unsigned blk = blockIdx.y * gridDim.x + blockIdx.x;
+  const unsigned q = 2 * __builtin_amdgcn_readfirstlane(blk * 4 + (threadIdx.x >> 6)), odd = (l >> 2) & 1;
+  const unsigned c0 = q / nT, t0 = q - c0 * nT + odd;
+  const unsigned c = t0 < nT ? c0 : c0 + 1, t = t0 < nT ? t0 : 0;
+  const bool live = q + odd < tiles;
+  float4 f[2];
 #pragma unroll
-  for (int i = 0; i < QP_UNITS; ++i) {
-    const unsigned c = (u0 + i) / npair;
-    const int t = 2 * (int)((u0 + i) % npair) + ((l >> 2) & 1);
-    const bool live = u0 + i < units && t < nT;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      f[i][j] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (live)
-        f[i][j] = ld_nt(reinterpret_cast<const float4 *>(W + (((long long)c * 16 + 8 * j + (l >> 3)) * nT + t) * TILE +
-                                                         4 * (l & 3)));
-    }
+  for (int j = 0; j < 2; ++j) {
+    f[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (live)
+      f[j] = ld_nt(reinterpret_cast<const float4 *>(W + (((long long)c * 16 + 8 * j + (l >> 3)) * nT + t) * TILE +
+                                                    4 * (l & 3)));
   }
+  const long long ct = (long long)c * cstride * nT + t;
 #pragma unroll
-  for (int i = 0; i < QP_UNITS; ++i) {
-    const unsigned c = (u0 + i) / npair;
-    const int t = 2 * (int)((u0 + i) % npair) + ((l >> 2) & 1);
-    const bool live = u0 + i < units && t < nT;
-    const long long ct = (long long)c * cstride * nT + t;
+  for (int j = 0; j < 2; ++j) {
+    const float x[4] = {f[j].x, f[j].y, f[j].z, f[j].w};
+    float amax = 0.f;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const float x[4] = {f[i][j].x, f[i][j].y, f[i][j].z, f[i][j].w};
-      float amax = 0.f;
+    for (int k = 0; k < 4; ++k) amax = fmaxf(amax, fabsf(x[k]));
+    amax = quad_max(amax);
+    int ex = -127;
+    if (amax > 0.f) {
+      frexp((double)amax, &ex);
+      ex = ex < -127 ? -127 : (ex > 127 ? 127 : ex);
+    }
+    int mm[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) amax = fmaxf(amax, fabsf(x[k]));
-      amax = quad_max(amax);
-      int ex = -127;
-      if (amax > 0.f) {
-        frexp((double)amax, &ex);
-        ex = ex < -127 ? -127 : (ex > 127 ? 127 : ex);
-      }
-      int mm[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) mm[k] = (int)fminf(fmaxf(rintf(ldexpf(x[k], 15 - ex)), -32768.f), 32767.f);
-      const int r = 8 * j + (l >> 3), h = (l >> 1) & 1;
-      if (live) {
-        Pm[((ct * 2 + h) * 16 + r) * 2 + (l & 1)] =
-            make_uint2((mm[0] & 0xffff) | (mm[1] << 16), (mm[2] & 0xffff) | (mm[3] << 16));
-        if ((l & 3) == 0) Pe[ct * 16 + r] = (int8_t)ex;
-      }
+    for (int k = 0; k < 4; ++k) mm[k] = (int)fminf(fmaxf(rintf(ldexpf(x[k], 15 - ex)), -32768.f), 32767.f);
+    const int r = 8 * j + (l >> 3), h = (l >> 1) & 1;
+    if (live) {
+      Pm[((ct * 2 + h) * 16 + r) * 2 + (l & 1)] =
+          make_uint2((mm[0] & 0xffff) | (mm[1] << 16), (mm[2] & 0xffff) | (mm[3] << 16));
+      if ((l & 3) == 0) Pe[ct * 16 + r] = (int8_t)ex;
     }
   }
 }
@@ -561,10 +554,12 @@ int quantize_pack_f32(const float *W, int n_out, int n_in, void *P_m, void *P_e,
   if (n_out <= 0 || n_in <= 0 || n_out % 16 || n_in % 16 || !W || !P_m || !P_e)
     return set_err(BFP_EINVAL, "quantize_pack: bad arguments (n_out=%d n_in=%d)", n_out, n_in);
   int nT = n_in / 16;
-  const long long units = (long long)(n_out / 16) * ((nT + 1) / 2);
-  if (units > (1LL << 31)) return set_err(BFP_EINVAL, "quantize_pack: n_out=%d n_in=%d", n_out, n_in);
-  hipLaunchKernelGGL(quantize_pack_f32_kernel, dim3(nblk(units, 4 * QP_UNITS)), dim3(256), 0, s, W,
-                     (unsigned)units, nT, cstride, reinterpret_cast<uint2 *>(P_m),
+  const long long tiles = (long long)(n_out / 16) * nT;   // of 16 rows
+  if (tiles > (1LL << 31)) return set_err(BFP_EINVAL, "quantize_pack: n_out=%d n_in=%d", n_out, n_in);
+  // a grid row stays below 2^32 threads
+  const unsigned blocks = nblk((tiles + 1) / 2, 4), gx = std::min(blocks, 1u << 22);
+  hipLaunchKernelGGL(quantize_pack_f32_kernel, dim3(gx, (blocks + gx - 1) / gx), dim3(256), 0, s, W,
+                     (unsigned)tiles, (unsigned)nT, cstride, reinterpret_cast<uint2 *>(P_m),
                      reinterpret_cast<int8_t *>(P_e));
   return launch_status("quantize_pack");
 }
