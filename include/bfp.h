@@ -419,7 +419,8 @@ int bfp_decode(bfp_ctx *ctx, const int32_t *prompt, int n_prompt, int n_gen, int
 int bfp_decode_path(const bfp_ctx *ctx);
 /* The launch form of the last bfp_decode's layers (no reference
  * counterpart; for tests and tuning): BFP_FORM_SINGLE (per-sequence stage
- * kernels, batches below 16), or BFP_FORM_MX (int8 matrix-core matvecs) with
+ * kernels: batches below 16 sequences, and of wide layers, from about D = 704
+ * on, fewer), or BFP_FORM_MX (int8 matrix-core matvecs) with
  * BFP_FORM_QKV_ATTN when Q|K|V and attention ran as one launch (with
  * BFP_FORM_ATT_GROUP when its attention workgroups each took a whole KV
  * group's query heads: contexts of at most 256, the default; the environment

@@ -524,3 +524,22 @@ def test_head_without_bounded_buffers(gpu, monkeypatch, max_batch):
             got.append((list(am), gm.decode(P, 8)[0].tolist()))
         gm.close()
     assert got[:2] == got[2:]
+
+
+@pytest.mark.parametrize("D,H_KV,FFN,single,mx", [(704, 11, 1408, 11, 12), (1024, 4, 1728, 10, 11), (1088, 1, 1728, 9, 10),
+                                                  (1280, 5, 1536, 8, 9), (1728, 27, 512, 3, 4)])
+def test_decode_wide_layers(gpu, D, H_KV, FFN, single, mx):
+    """Wide layers go to the matrix cores below 16 sequences, once Q|K|V and
+    G/U are past two rounds of workgroups (their norm a pair of elements a
+    thread up to D = 1024, block-wide in 6, 8 or 9 waves above): on both sides
+    of the line layer outputs at every step and tokens equal the oracle's."""
+    d, om, gm = _setup(dict(D=D, H_Q=D // 64, H_KV=H_KV, HD=64, FFN=FFN, NL=1, MAX_CTX=8, VOCAB=256), D, max_batch=mx)
+    prompts = np.random.default_rng(D).integers(0, d.VOCAB, size=(mx, 1)).astype(np.int32)
+    want = {b: _oracle_decode(om, prompts[b], 3) for b in (0, single - 1, mx - 1)}
+    for n, form in ((2, "single"), (single, "single"), (mx, "mx")):
+        toks, (hm, he) = gm.decode(prompts[:n], 3, hist=True)
+        assert gm.decode_form().startswith(form), n
+        for b in (b for b in want if b < n):
+            wt, wm, we = want[b]
+            assert list(toks[b]) == list(wt) and np.array_equal(hm[b], wm) and np.array_equal(he[b], we), (n, b)
+    gm.close()

@@ -315,7 +315,8 @@ class BfpModel:
 
     def decode_form(self):
         """How the last decode's layers were launched: 'persist', 'pipe' (the
-        pipelined batched step), 'single' (batches below 16), or 'mx' followed by
+        pipelined batched step), 'single' (the per-sequence kernels: batches
+        below 16 sequences, fewer of wide layers), or 'mx' followed by
         '+qkv_attn' (Q|K|V and attention in one launch), '+attn_group' (its
         attention a KV group per workgroup) and '+norm_fused' (RMSNorms
         inside the O and D launches)."""

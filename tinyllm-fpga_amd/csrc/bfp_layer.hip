@@ -998,20 +998,6 @@ __global__ __launch_bounds__(256) void k_ctl_embed(CtlArgs a, EmbedArgs e) {
 // --------------------------------------------------------------- launchers
 typedef void (*lk_fn)(LayerArgs);
 
-// Batches from this size on (a whole group of 16 sequences) run the matvecs
-// on the matrix cores with the RMSNorms once per sequence; below, every
-// (chunk, sequence) is a workgroup of the per-sequence kernels.  At SmolLM2's
-// 30 layers, 23 + 25 tokens, per-sequence against matrix-core launches: 5
-// sequences 26.8 / 38.2 ms, 8 31.0 / 41.1, 12 35.9 / 43.0, 16 41.0 / 45.9, 20
-// 46.4 / 47.6, 24 51.6 / 50.6 -- the crossing is near 22, where the rows are
-// ragged; 16 keeps whole groups on the matrix cores.  (A vector form with 8
-// sequences per workgroup, weights read once for them, took 46.5 ms at 5.)
-// env BFP_MX_MIN_BATCH overrides.
-static int MX_MIN_BATCH = [] {
-  const char *v = getenv("BFP_MX_MIN_BATCH");
-  return v ? atoi(v) : 16;
-}();
-
 // The (waves, tiles per lane) pairs default_waves() produces for
 // 4 <= in/16 <= 108, i.e. every supported D and FFN.
 #define BFP_LAYER_SHAPES(X, KER) \
@@ -1020,10 +1006,17 @@ static int MX_MIN_BATCH = [] {
 #define BFP_CASE(KER, NW, TPT) \
   if (nw == NW && tpt == TPT) return KER<NW, TPT>;
 
+// Waves and tiles per lane of a matvec over nT input tiles.
+static void shape_for(int nT, int &nw, int &tpt) {
+  nw = default_waves(nT);
+  tpt = (nT + 4 * nw - 1) / (4 * nw);
+}
+
 // k_qkv and k_gu: up to D = 1024 a thread per pair of elements (D / 128 waves,
 // at most two tiles a lane), so the RMSNorm prologue is one division pair and
 // one quantisation a thread and every wave sums the squares itself; above, the
-// matvec's own shape with the block-wide norm.
+// matvec's own shape (6, 8 or 9 waves, three tiles a lane) with the block-wide
+// norm.
 static bool norm_pairs_shape(int D, int &nw, int &tpt) {
   if (D > 1024) return false;
   nw = (D + 127) / 128;
@@ -1041,20 +1034,15 @@ static bool norm_pairs_shape(int D, int &nw, int &tpt) {
     lds = (size_t)norm_prologue_doubles(true, D) * 8 + (size_t)(D / 16) * 17 * 4;                     \
     return (tpt == 1 ? k1 : k2)[nw - 1];                                                              \
   }                                                                                                   \
-  threads = 64 * 9;                                                                                   \
+  shape_for(D / 16, nw, tpt);                                                                         \
+  threads = 64 * nw;                                                                                  \
   lds = (size_t)norm_prologue_doubles(false, D) * 8 + (size_t)(D / 16) * 17 * 4;                      \
-  return KER<9, 3, false>;
+  return nw == 6 ? KER<6, 3, false> : (nw == 8 ? KER<8, 3, false> : KER<9, 3, false>);
 static lk_fn pick_qkv(int D, int &threads, size_t &lds) { BFP_NORM_CASES(k_qkv) }
 static lk_fn pick_gu(int D, int &threads, size_t &lds) { BFP_NORM_CASES(k_gu) }
 
 static lk_fn pick_ores(int nw, int tpt) { BFP_LAYER_SHAPES(BFP_CASE, k_o_res) return nullptr; }
 static lk_fn pick_dres(int nw, int tpt) { BFP_LAYER_SHAPES(BFP_CASE, k_d_res) return nullptr; }
-
-// Waves and tiles per lane of a matvec over nT input tiles.
-static void shape_for(int nT, int &nw, int &tpt) {
-  nw = default_waves(nT);
-  tpt = (nT + 4 * nw - 1) / (4 * nw);
-}
 
 static lk_fn attn_kernel(int ppw) {
   // max_ctx <= 512 = 64 * ATT_WAVES for ppw 2, 3 and 4: the short forms
@@ -1160,8 +1148,42 @@ static bool mx_joined_qkv_attn(const LayerArgs &a) {
          mx_waves(a.D / 16, bq * G) == ATT_WAVES;
 }
 
-// The matrix-core path (its norm buffer is the context's).
-static bool mx_path(const LayerArgs &a) { return a.batch >= MX_MIN_BATCH && a.batch > 1 && a.xn_m; }
+// Which layers run their matvecs on the matrix cores with the RMSNorms once
+// per sequence; the others run the per-sequence kernels, in which every
+// (chunk, sequence) is a workgroup and those of Q|K|V and G/U each form the
+// norm.  The matrix-core launches take about the same time from 2 sequences
+// to 16; the per-sequence ones grow with the rounds of workgroups that the
+// chip needs for Q|K|V and G/U, and are overtaken at about two rounds of the
+// pair form (D <= 1024) and 1 3/4 of the block-wide norm's.  Per-sequence /
+// matrix-core launches, ms for 30 steps of 4 layers:
+//   D 704, H_KV 11, FFN 1408   9 sequences 6.07 / 6.89, 12 7.04 / 7.04, 15 7.68 / 7.20
+//   D 1024, H_KV 4, FFN 1728   9 7.01 / 7.61, 11 7.80 / 7.77, 15 9.13 / 7.94
+//   D 1088, H_KV 17, FFN 1728  4 7.17 / 8.50, 6 8.63 / 8.65, 8 10.7 / 8.78, 15 15.3 / 9.31
+//   D 1152, H_KV 6, FFN 512    8 6.73 / 8.29, 12 8.57 / 8.65, 15 9.51 / 8.80
+//   D 1728, H_KV 27, FFN 512   3 8.93 / 10.5, 4 10.8 / 10.6, 8 16.1 / 11.0, 15 25.9 / 11.8
+// (D 1536 crosses later than the rule, near 9 sequences against 7.)
+// Whole groups of 16 sequences are on the matrix cores at every width.  At
+// D <= 768 that is earlier than the crossing, and the batches from 16 up to it
+// are slower for it: SmolLM2's 30 layers, 23 + 25 tokens, 16 sequences 34.4 /
+// 39.2, 20 38.8 / 40.4, 22 41.1 / 40.5; 60 + 1000 tokens, 16 sequences 1904 /
+// 2225; D 256 of 12 layers, 24 sequences 10.5 / 12.4.
+// env BFP_MX_MIN_BATCH: from that many sequences at every width.
+static int MX_MIN_BATCH = [] {
+  const char *v = getenv("BFP_MX_MIN_BATCH");
+  return v ? atoi(v) : 0;
+}();
+static bool mx_path(const LayerArgs &a) {
+  if (a.batch < 2 || !a.xn_m) return false;   // (the norm buffer is the context's)
+  if (MX_MIN_BATCH > 0) return a.batch >= MX_MIN_BATCH;
+  if (a.batch >= MX_SEQ) return true;
+  int threads;
+  size_t lds;
+  pick_gu(a.D, threads, lds);
+  const int nw = threads / 64, chunks = (a.D + 2 * a.KV + a.FFN) / 16;
+  const int held = std::min(32 / nw, (int)(160 * 1024 / (lds + 2 * nw * 16 * 12)));   // workgroups a CU, with k_gu's static LDS
+  const int quarter_rounds = a.D <= 1024 ? 8 : 7;
+  return 4 * chunks * a.batch > quarter_rounds * 256 * held;
+}
 
 int layer_form(const LayerArgs &a) {
   if (!mx_path(a)) return BFP_FORM_SINGLE;
