@@ -234,8 +234,9 @@ int bfp_get_dims(const bfp_ctx *ctx, bfp_dims *out);
  *                    reaches the host while the decode runs (4.3 MB, made on
  *                    first use); else one copy after it;
  *   BFP_MEM_HEAD     the bounded head's copy of the embedding and its
- *                    buffers (2 bytes an element and 24 a row; contexts for
- *                    2 sequences and more, D at most 576); else the full head;
+ *                    buffers (2 bytes an element and 24 a row; contexts
+ *                    whose max_batch takes it, see bfp_head); else the full
+ *                    head;
  *   BFP_MEM_PROMPT   the rows of bfp_decode's prompt passes (at most 1024,
  *                    about 18 D + 4 KV + 2 FFN bytes each, made on first use);
  *                    else the prompt runs step by step.
@@ -353,12 +354,14 @@ int bfp_rtl_decode(bfp_ctx *ctx, const int32_t *prompt, int n_prompt, int n_gen,
                    int16_t *hist_m, int8_t *hist_e);
 
 /* Decode head (full.py:438-440): final norm, float64 logits over the raw
- * embedding, first-index argmax.  logits may be NULL: then, from 2
- * sequences on (D at most 576), the argmax comes from
- * the bounded head, which forms float64 logits only for the rows that can
- * hold the largest (an exact int16 dot product brackets every logit) and
- * returns the same index; the environment variable BFP_HEAD_BOUNDED=0
- * keeps the full head. */
+ * embedding, first-index argmax.  logits may be NULL: then, from 10
+ * sequences on or where sequences x vocabulary is past 65536 (D at most 576,
+ * 2 sequences and more), the argmax comes from the bounded head, which forms
+ * float64 logits only for the rows that can hold the largest (an exact int16
+ * dot product brackets every logit) and returns the same index.  The
+ * environment variable BFP_HEAD_BOUNDED=0 keeps the full head; with another
+ * value, set when the context is made and after, the bounded one is taken
+ * from 2 sequences. */
 int bfp_head(bfp_ctx *ctx, int batch, const int16_t *h_m, const int8_t *h_e, double *logits,
              int32_t *argmax);
 

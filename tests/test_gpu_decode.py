@@ -406,13 +406,14 @@ def test_batched_trace(gpu):
 
 
 @pytest.mark.parametrize("batch", [2, 15, 16, 17, 31])
-def test_head_bounded_small_batches(gpu, batch):
+def test_head_bounded_small_batches(gpu, monkeypatch, batch):
     """The bounded head below 32 sequences (one sequence group up to 16, four
     above) against the full head's logits, with ties within and across
     blocks, a zero block, an all-zero hidden state and a short last block of
     workgroups."""
     from bfp import Dims, synth
     from bfp.model import BfpModel
+    monkeypatch.setenv("BFP_HEAD_BOUNDED", "1")   # at this vocabulary it is the rule from 10 sequences only
     d = Dims(D=192, H_Q=3, H_KV=1, HD=64, FFN=256, NL=1, MAX_CTX=8, VOCAB=1040)
     fm = synth.make_model(d, seed=batch)
     E = fm.embed
@@ -421,6 +422,7 @@ def test_head_bounded_small_batches(gpu, batch):
     E[200:216] = 0.0
     E[101] = np.nextafter(E[100], np.float32(np.inf))
     gm = BfpModel(d, max_batch=batch)
+    assert "head" in gm.optional_memory()
     gm.load_fp32(fm)
     rng = np.random.default_rng(batch)
     hs = [rng.standard_normal(d.D) * (0.3 + 0.1 * b) for b in range(batch)]
@@ -499,7 +501,7 @@ def test_history_without_pinned_memory(gpu, monkeypatch, batch, n_prompt, n_gen)
         assert np.array_equal(hm, got[0][1][0]) and np.array_equal(he, got[0][1][1])
 
 
-@pytest.mark.parametrize("max_batch", [1, 2, 15, 33])
+@pytest.mark.parametrize("max_batch", [1, 9, 10, 33])
 def test_head_without_bounded_buffers(gpu, monkeypatch, max_batch):
     """A context whose bounded head's buffers cannot be had is made all the
     same and takes the full head: the same tokens, one embedding after
@@ -515,7 +517,7 @@ def test_head_without_bounded_buffers(gpu, monkeypatch, max_batch):
     for held in (True, False):
         monkeypatch.setenv("BFP_OPTIONAL_MEMORY", str(int(held)))
         gm = BfpModel(d, max_batch=max_batch)
-        assert ("head" in gm.optional_memory()) == (held and max_batch > 1)
+        assert ("head" in gm.optional_memory()) == (held and max_batch >= 10)
         for seed in (1, 2):
             gm.load_fp32(synth.make_model(d, seed=seed))
             full, lg = gm.head(hm, he, logits=True)
@@ -542,4 +544,23 @@ def test_decode_wide_layers(gpu, D, H_KV, FFN, single, mx):
         for b in (b for b in want if b < n):
             wt, wm, we = want[b]
             assert list(toks[b]) == list(wt) and np.array_equal(hm[b], wm) and np.array_equal(he[b], we), (n, b)
+    gm.close()
+
+
+@pytest.mark.parametrize("batch,vocab,bounded", [(1, 131072, False), (2, 32768, False), (2, 32784, True), (9, 7280, False),
+                                                 (9, 7296, True), (10, 512, True)])
+def test_head_bounded_where_it_pays(gpu, batch, vocab, bounded):
+    """The bounded head from 10 sequences, or past 65536 rows over all of
+    them: the argmax on both sides of the line equals the full head's."""
+    from bfp import Dims, synth
+    from bfp.model import BfpModel
+    d = Dims(D=64, H_Q=1, H_KV=1, HD=64, FFN=64, NL=1, MAX_CTX=8, VOCAB=vocab)
+    gm = BfpModel(d, max_batch=batch)
+    assert ("head" in gm.optional_memory()) == bounded
+    gm.load_fp32(synth.make_model(d, seed=batch))
+    rng = np.random.default_rng(batch)
+    hm = rng.integers(-20000, 20000, size=(batch, d.D)).astype(np.int16)
+    he = rng.integers(-2, 3, size=(batch, d.D // 16)).astype(np.int8)
+    full, lg = gm.head(hm, he, logits=True)
+    assert list(gm.head(hm, he)[0]) == list(full) == [int(np.argmax(r)) for r in lg]
     gm.close()

@@ -60,7 +60,7 @@ struct bfp_ctx {
   float *embed = nullptr;
   float *embedp = nullptr;     // the embedding permuted per row for the batched head
                                // (made when max_batch >= HEAD_SEQ_MIN)
-  // the bounded head (made when max_batch >= HEADQ_MIN): the embedding as split int16 with
+  // the bounded head (made where max_batch sequences take it): the embedding as split int16 with
   // per-row meta, and per step the quantised hidden, its per-sequence
   // record and the per-block bounds
   uint4 *embq = nullptr, *hq_x = nullptr;
@@ -276,13 +276,18 @@ int head_part_max(const bfp_ctx *c) {
   return m;
 }
 
-// The bounded head (argmax only) where its copy exists and no logits are
-// asked for, from HEADQ_MIN sequences; BFP_HEAD_BOUNDED=0 keeps the full
-// head.  (Below HEAD_SEQ_MIN sequences a vocabulary too large for the pick's
-// candidate list takes the full head too.)
-bool head_bounded(const bfp_ctx *c, int batch, const double *logits) {
+// The bounded head's batches (headq_batch); BFP_HEAD_BOUNDED=0 keeps the full
+// head, another value takes the bounded one from 2 sequences.
+bool headq_takes(int batch, int VOCAB) {
   const char *v = getenv("BFP_HEAD_BOUNDED");
-  return c->embq && !logits && batch >= HEADQ_MIN && !(v && atoi(v) == 0) &&
+  return v ? atoi(v) != 0 && batch >= 2 : headq_batch(batch, VOCAB);
+}
+
+// The bounded head (argmax only) where its copy exists and no logits are
+// asked for.  (Below HEAD_SEQ_MIN sequences a vocabulary too large for the
+// pick's candidate list takes the full head too.)
+bool head_bounded(const bfp_ctx *c, int batch, const double *logits) {
+  return c->embq && !logits && headq_takes(batch, c->d.VOCAB) &&
          (batch >= HEAD_SEQ_MIN || headq_pick_lds(c->d.D, c->d.VOCAB) <= 64 * 1024);
 }
 
@@ -892,7 +897,7 @@ bfp_ctx *bfp_create(const bfp_dims *dims, int device, int max_batch) {
     return nullptr;
   }
   // the bounded head's, after all that the context cannot do without
-  if (max_batch >= HEADQ_MIN && d.D % 64 == 0 && d.D <= 576)
+  if (headq_takes(max_batch, d.VOCAB) && d.D % 64 == 0 && d.D <= 576)
     c->alloc_optional({{(void **)&c->embq, (size_t)d.VOCAB * d.D * 2},
                        {(void **)&c->embq_meta, sizeof(HeadQRow) * (size_t)d.VOCAB},
                        {(void **)&c->hq_x, (size_t)(B + 15) / 16 * (d.D / 64) * 64 * 32},

@@ -144,11 +144,16 @@ struct HeadArgs {
   double2 *hq_blk;                         // (batch, VOCAB / 16) per 16-row block: max lower, max upper bound
 };
 
-// The bounded head runs from HEADQ_MIN sequences (D % 64 == 0 and D <= 576)
-// unless logits are asked for.  Against the full head over all rows, 30 layers
-// and 23 + 25 tokens: 2 sequences 23.6 / 24.1 ms, 5 26.1 / 27.2, 16 44.6 / 45.9,
-// 24 48.5 / 50.0.
-constexpr int HEADQ_MIN = 2;
+// The bounded head runs (D % 64 == 0 and D <= 576, no logits asked for) where
+// a step's full head reads enough to pay for one launch more: from 10 sequences,
+// or where sequences x vocabulary is past 65536.  Full / bounded, us a decode
+// step of one small layer at D 576: vocabulary 1024, 2 sequences 42.4 / 49.9, 8
+// 49.9 / 52.2, 12 55.9 / 53.1, 31 90.5 / 74.4; 16384, 2 48.0 / 52.1, 5 52.1 /
+// 52.8, 8 56.1 / 53.3; 49152, 2 70.0 / 55.8, 8 89.2 / 57.3, 31 177 / 81.0 (D 64
+// to 320 cross at the same places).  Its time grows with the blocks that can
+// hold the largest logit, about one a sequence; a hidden state of zeros, which
+// ties every row, takes 1.1 ms at 49152 (full: 0.12).
+inline bool headq_batch(int batch, int VOCAB) { return batch >= 10 || (batch >= 2 && (long long)batch * VOCAB > 65536); }
 constexpr int HEADQ_SEQ = 64;   // most sequences per k_headq_mx workgroup
 inline size_t headq_pick_lds(int D, int VOCAB) { return (size_t)D * 8 + (size_t)(VOCAB / 16) * 4; }
 
