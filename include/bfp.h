@@ -232,7 +232,8 @@ int bfp_get_dims(const bfp_ctx *ctx, bfp_dims *out);
  * reference counterpart; for tests and tuning).
  *   BFP_MEM_HISTORY  the pinned pieces through which bfp_decode's history
  *                    reaches the host while the decode runs (4.3 MB, made on
- *                    first use); else one copy after it;
+ *                    first use, by a history of more than 64 KB); else one
+ *                    copy after it;
  *   BFP_MEM_HEAD     the bounded head's copy of the embedding and its
  *                    buffers (2 bytes an element and 24 a row; contexts
  *                    whose max_batch takes it, see bfp_head); else the full

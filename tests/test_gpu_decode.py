@@ -477,14 +477,16 @@ def test_history_pieces(gpu, batch, n_prompt, n_gen):
     gm.close()
 
 
-@pytest.mark.parametrize("batch,n_prompt,n_gen", [(1, 3, 4), (1, 12, 4), (3, 5, 6), (17, 2, 9)])
-def test_history_without_pinned_memory(gpu, monkeypatch, batch, n_prompt, n_gen):
+@pytest.mark.parametrize("batch,n_prompt,n_gen,pieces", [(1, 3, 53, False), (1, 3, 54, True), (1, 12, 60, True),
+                                                         (3, 5, 30, True), (17, 2, 9, True)])
+def test_history_without_pinned_memory(gpu, monkeypatch, batch, n_prompt, n_gen, pieces):
     """Without pinned memory for its pieces the history comes in one copy
-    after the decode: the same bits, batch 1 on the persistent launch and
-    batches, with and without a prompt pass before."""
+    after the decode, as one of at most 64 KB does with it: the same bits,
+    batch 1 on the persistent launch and batches, with and without a prompt
+    pass before."""
     from bfp import Dims, synth
     from bfp.model import BfpModel
-    d = Dims(D=192, H_Q=3, H_KV=1, HD=64, FFN=272, NL=3, MAX_CTX=32, VOCAB=512)
+    d = Dims(D=192, H_Q=3, H_KV=1, HD=64, FFN=272, NL=3, MAX_CTX=80, VOCAB=512)
     fm = synth.make_model(d, seed=2)
     P = np.stack([synth.make_prompt(d, n_prompt, seed=b) for b in range(batch)])
     got = []
@@ -494,7 +496,7 @@ def test_history_without_pinned_memory(gpu, monkeypatch, batch, n_prompt, n_gen)
         gm.load_fp32(fm)
         for _ in range(2):
             got.append(gm.decode(P, n_gen, hist=True))
-        assert ("history" in gm.optional_memory()) == held
+        assert ("history" in gm.optional_memory()) == (held and pieces)
         gm.close()
     for toks, (hm, he) in got[1:]:
         assert np.array_equal(toks, got[0][0])

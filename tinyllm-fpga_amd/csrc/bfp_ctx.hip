@@ -482,12 +482,15 @@ constexpr int HIST_LAG = 8;   // steps
 // the last step only the last marks' steps are left to copy.  64 sequences x
 // 32 steps x 30 layers x 576 (73 MB): the call's time past the decode's last
 // kernel 4.0 ms, 10.3 with one copy at the end; the decode itself takes the same.
-// Without pinned memory for the pieces it is that one copy.
+// Without pinned memory for the pieces it is that one copy, and for a history
+// of at most WHOLE bytes, where the second stream and its events cost 12 us
+// more than the copy (230 / 242 us for 2 steps of one layer; from about 76 KB
+// the pieces are level or ahead).
 class HistOut {
  public:
   HistOut(bfp_ctx *c, int batch, int steps, const int16_t *dm, const int8_t *de, int16_t *m, int8_t *e)
       : c_(c), batch_(batch), steps_(steps), dm_(dm), de_(de), m_(m), e_(e),
-        row_((size_t)c->d.NL * c->d.D * 2) {}
+        row_((size_t)c->d.NL * c->d.D * 2), whole_(row_ * batch * steps <= WHOLE) {}
   ~HistOut() {
     if (on()) (void)hipStreamSynchronize(c_->hist_stream);   // no copy outlives the buffers
     for (const Mark &k : marks_) (void)hipEventDestroy(k.ev);
@@ -549,7 +552,7 @@ class HistOut {
   struct Piece {
     int b0, nb, s0, ns;
   };
-  static constexpr size_t PIECE = 2 << 20;
+  static constexpr size_t PIECE = 2 << 20, WHOLE = 64 << 10;
 
   int prepare() {
     if (c_->hist_ev[1]) return BFP_OK;
@@ -599,7 +602,7 @@ class HistOut {
   int16_t *m_;
   int8_t *e_;
   const size_t row_;   // bytes of a step's mantissas, one sequence
-  bool whole_ = false;   // no pinned pieces: one copy at the end
+  bool whole_;   // one copy at the end, no pinned pieces
   int done_ = 0, next_ = 0;
   Piece slot_[2] = {};
   std::deque<Mark> marks_;
