@@ -204,13 +204,13 @@ int bfp_rtl_residual_d(const int16_t *a_m, const int8_t *a_e, const int16_t *b_m
                        const int8_t *b_e, int n, int16_t *y_m, int8_t *y_e, void *stream);
 /* The decode head's bfp_gt running argmax (smollm_decode_head_bfp.sv:
  * 253-274,322-324,399-430) over batch rows of n (m, e) pairs (one exponent
- * per element); work: 3*batch*n/16 int32 of device scratch. */
+ * per element); work: batch*n/16 int32 of device scratch. */
 int bfp_rtl_argmax_d(const int16_t *m, const int8_t *e, int n, int batch, int32_t *work,
                      int32_t *idx, void *stream);
 /* No counterpart in the reference: bfp_rtl_argmax_d for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  The same kernel and result; its
- * workspace is the library's static device scratch (3 MiB per GPU, held
+ * workspace is the library's static device scratch (1 MiB per GPU, held
  * until the process ends), so it calls no allocator.  batch * n/16 must be
  * at most 262144 (e.g. 64 rows of a 65536-entry vocabulary), else
  * BFP_EINVAL.  Calls that overlap on one GPU share the scratch and race. */

@@ -327,8 +327,8 @@ class BfpModel:
             return "persist"
         if f == 32:
             return "pipe"
-        if f < 2:
-            return ("single", "multi")[f]
+        if f == 0:
+            return "single"
         return ("mx" + ("+qkv_attn" if f & 4 else "") + ("+attn_group" if f & 64 else "")
                 + ("+norm_fused" if f & 8 else ""))
 

@@ -120,7 +120,7 @@ def argmax(m, e):
     """bfp_gt running argmax over rows of (m, e) pairs: m, e (batch, n) or (n,)."""
     m = np.atleast_2d(np.asarray(m))
     batch, n = m.shape
-    work = _dev.empty(3 * batch * n // TILE, "int32")
+    work = _dev.empty(batch * n // TILE, "int32")
     out = _dev.empty(batch, "int32")
     dm, de = _d(m, np.int16), _d(e, np.int8)
     call("bfp_rtl_argmax_d", dm.data_ptr(), de.data_ptr(), n, batch, work.data_ptr(),

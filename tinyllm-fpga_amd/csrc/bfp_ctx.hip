@@ -1375,7 +1375,7 @@ static int rtl_head_ready(bfp_ctx *c, RtlHeadArgs &ha) {
     BFP_TRY(c->alloc((void **)&c->rtl_lg_e, (size_t)d.VOCAB));
     BFP_TRY(c->alloc((void **)&c->rtl_xn_m, (size_t)d.D * 2));
     BFP_TRY(c->alloc((void **)&c->rtl_xn_e, (size_t)d.D / 16));
-    BFP_TRY(c->alloc((void **)&c->rtl_work, sizeof(int) * 3 * (size_t)(d.VOCAB / 16)));
+    BFP_TRY(c->alloc((void **)&c->rtl_work, sizeof(int) * (size_t)(d.VOCAB / 16)));
     BFP_TRY(c->alloc((void **)&c->rtl_tok, sizeof(int)));
   }
   BFP_TRY(bfp_quantize_pack_f32_d(c->embed, d.VOCAB, d.D, c->rtl_emb_m, c->rtl_emb_e, c->stream));
@@ -1673,8 +1673,8 @@ int bfp_decode(bfp_ctx *c, const int32_t *prompt, int n_prompt, int n_gen, int b
   hipGraph_t gr[2] = {nullptr, nullptr};
   int rc = BFP_OK;
   if (use_graph) {
-    // k = 0: a step without the head (before the prompt's end)
-    for (int k = step0 > 0 || rtl_loop ? 1 : 0; k < 2 && !rc; ++k) {
+    // k = 0: a step without the head (before the prompt's last position)
+    for (int k = step0 >= n_prompt - 1 || rtl_loop ? 1 : 0; k < 2 && !rc; ++k) {
       HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
       rc = enqueue_step(k == 1);
       hipError_t e1 = hipStreamEndCapture(s, &gr[k]);

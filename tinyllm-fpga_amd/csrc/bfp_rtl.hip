@@ -1196,16 +1196,17 @@ __global__ __launch_bounds__(64) void k_rtl_ctl(RtlCtlArgs a) {
 }  // namespace bfp
 
 // ---------------------------------------------- allocation-free argmax
-// Scratch of bfp_rtl_argmax_static_d: the per-chunk bests (mantissa,
-// exponent, index) of at most ARGMAX_STATIC_CHUNKS chunks (batch * n/16),
-// in one device-global array per GPU: 3 MiB, held until the process ends.
+// Scratch of bfp_rtl_argmax_static_d: the per-chunk bests (a word of
+// mantissa, exponent and lane each) of at most ARGMAX_STATIC_CHUNKS chunks
+// (batch * n/16), in one device-global array per GPU: 1 MiB, held until the
+// process ends.
 // Host code never passes the array's name to a kernel (on the host it is a
 // stand-in, not a device address): argmax_scratch() looks its address up
 // once per device with hipGetSymbolAddress and hands that out.
 namespace bfp {
 namespace {
 constexpr long long ARGMAX_STATIC_CHUNKS = 262144;
-static __device__ __align__(256) int scratch[3 * ARGMAX_STATIC_CHUNKS];
+static __device__ __align__(256) int scratch[ARGMAX_STATIC_CHUNKS];
 constexpr int SCRATCH_MAX_DEVICES = 64;
 std::mutex g_scratch_mu;
 int *g_scratch[SCRATCH_MAX_DEVICES] = {};
@@ -1345,7 +1346,7 @@ int bfp_rtl_argmax_static_d(const int16_t *m, const int8_t *e, int n, int batch,
   return launch_status("rtl_argmax_static");
 }
 
-// work: 3 * batch * n/16 ints of device scratch supplied by the caller.
+// work: batch * n/16 ints of device scratch supplied by the caller.
 int bfp_rtl_argmax_d(const int16_t *m, const int8_t *e, int n, int batch, int32_t *work,
                      int32_t *idx, void *stream) {
   if (n <= 0 || n % 16 || batch <= 0 || !work) return set_err(BFP_EINVAL, "rtl_argmax: n=%d", n);
