@@ -74,16 +74,16 @@ def test_layer_batched_sequences(gpu):
     gm.close()
 
 
-@pytest.mark.parametrize("cfg,batch", [(MID, 5), (FULL, 6), (MID, 9), (MID, 33), (FULL, 40),
-                                       (FULL_LONG, 9)],
-                         ids=["mid-b5", "full-b6", "mfma-mid-b9", "mfma-mid-b33", "mfma-full-b40",
-                              "mfma-full-long-b9"])
+@pytest.mark.parametrize("cfg,batch", [(MID, 5), (FULL, 6), (MID, 9), (FULL_LONG, 9), (MID, 16), (MID, 17), (MID, 33),
+                                       (FULL, 40), (FULL_LONG, 17)],
+                         ids=["seq-mid-b5", "seq-full-b6", "seq-mid-b9", "seq-full-long-b9", "mfma-mid-b16",
+                              "mfma-mid-b17", "mfma-mid-b33", "mfma-full-b40", "mfma-full-long-b17"])
 def test_layer_multi_sequence_path(gpu, cfg, batch):
-    """Batches of 4 or more run the multi-sequence kernels (separate norm,
-    weight chunks reused across a group of sequences), from 8 on with the
-    tile sums on the int8 matrix cores in blocks of 16 sequences (9: one
-    partial block; 33: a last block of one sequence): every stage of every
-    sequence still equals its own oracle run."""
+    """Several sequences a launch: below 16 the per-sequence kernels, from 16
+    on the norm once per sequence and the tile sums on the int8 matrix cores
+    in blocks of 16 sequences (16: one whole block; 17, 33: a last block of
+    one sequence), with the short and the long attention form: every stage of
+    every sequence still equals its own oracle run."""
     d, om, gm = _setup(cfg, seed=7, max_batch=batch)
     rng = np.random.default_rng(9)
     kvs = [sim.new_kv(om.dims, d.MAX_CTX) for _ in range(batch)]
@@ -210,4 +210,34 @@ def test_long_attention_forms(gpu, cfg):
             assert all(np.array_equal(x, y) for p, q in zip(k0[b], k1) for x, y in zip(p, q)), pos
         one = gm.layer_step_bfp(0, pos + 3, hm[0], he[0], kv_pos=pos)
         assert np.array_equal(one[0][0], got[0][0]) and np.array_equal(one[1][0], got[1][0]), pos
+    gm.close()
+
+
+@pytest.mark.parametrize("batch", [15, 17])
+def test_long_attention_one_workgroup_a_head(gpu, batch):
+    """Capacities past 512 without a stage dump, from 512 / 4 heads a launch:
+    one workgroup per head (below and on the matrix cores otherwise), against
+    the oracle, at the ends of the K and V blocks and with RoPE position and
+    slot apart."""
+    d, om, gm = _setup(dict(FULL, MAX_CTX=1100), seed=11, max_batch=batch)
+    rng = np.random.default_rng(batch)
+    seqs = (0, batch // 2, batch - 1)
+    kvs = {b: sim.new_kv(om.dims, d.MAX_CTX) for b in seqs}
+    for b in range(batch):
+        rows = []
+        for _ in range(2):
+            m, e = sim.tile_quantize(rng.standard_normal(d.MAX_CTX * d.KV) * (0.3 + 0.1 * b))
+            rows.append((m.reshape(d.MAX_CTX, d.KV), e.reshape(d.MAX_CTX, d.KV // 16)))
+        gm.kv_io(0, b, 0, d.MAX_CTX, k=rows[0], v=rows[1])
+        if b in seqs:
+            for name, (m, e) in zip("kv", rows):
+                kvs[b][name][:] = sim.tile_decode(m.reshape(-1, 16), e.reshape(-1)).reshape(d.MAX_CTX, d.H_KV, d.HD)
+    for pos, slot in ((0, 0), (33, 31), (511, 511), (512, 512), (1090, 1099)):
+        hs = [sim.fp_quantize_vec(rng.standard_normal(d.D) * (0.5 + b)) for b in range(batch)]
+        q = [sim.tile_quantize(h) for h in hs]
+        om_, oe_, _ = gm.layer_step_bfp(0, pos, np.stack([x[0].reshape(-1) for x in q]), np.stack([x[1] for x in q]),
+                                        kv_pos=slot)
+        for b in seqs:
+            want = sim.fwd_layer(hs[b], om.layers[0], pos=pos, kv=kvs[b], kv_pos=slot, dims=om.dims)
+            assert (sim.tile_decode(om_[b].reshape(-1, 16), oe_[b]) == want).all(), (pos, slot, b)
     gm.close()
