@@ -5,15 +5,19 @@
 // pairwise sum, the ascending-t AV chain -- so the outputs are bit-identical
 // to its long form's (k_attn<8, false>), which gives a head to four
 // workgroups that each form every score and a quarter of the dimensions.
-//   K    blocks of 512 rows through LDS (coalesced 16-byte loads, the next
-//        block's in flight); each wave scores 64 of them, a decoded row a
-//        lane against the head's q (ddot64_rows);
+//   K    blocks of 512 rows through LDS (coalesced 16-byte loads); each wave
+//        scores 64 of them, a decoded row a lane against the head's q
+//        (ddot64_rows).  The next block's loads are issued before the scores,
+//        but the compiler keeps them in scratch memory (the choice between
+//        them and the current row is one of addresses, and so generic loads
+//        one after another), so a block waits for them before its scores;
 //   V    blocks of 32 rows decoded to float64 in LDS by waves 4-7, the loads
 //        of four blocks in flight; wave 0 runs the 64 chains (av_block).
 // A workgroup is a chain of dependent steps: about a third of it wave 0's
-// 1500 products and adds at position 1500, the rest the K blocks' loads and
-// scores and the softmax.  16 sequences at position 1500 (9 heads): 55.4 us a
-// launch against 69.6.
+// 1500 products and adds at position 1500 (some 29 cycles a position: wave 0
+// forms the products too, waves 1-3 are idle), the rest the K blocks' loads
+// and scores and the softmax.  16 sequences at position 1500 (9 heads): 55.4
+// us a launch against 69.6.
 #include <stdint.h>
 
 #include <algorithm>

@@ -1097,7 +1097,10 @@ int prepare_layer_kernels(int max_ctx, int D, int FFN) {
 // is the shorter one; one workgroup a head past that, which forms the scores
 // once and not four times.  Two layer calls, four / one, us: 1 sequence at
 // position 1500 118 / 172, 4 at 600 109 / 137, 16 at 100 185 / 168, 16 at 1500
-// 272 / 239, 64 at 600 392 / 328.
+// 272 / 239, 64 at 600 392 / 328.  One workgroup a head is one workgroup a CU,
+// so 257 heads take two rounds: from there to about 288 the four are ahead at
+// late positions (29 sequences of 9 heads at 1500 180 / 173, at 2047 199 / 209,
+// at 4095 301 / 328, one call).
 constexpr int ATT_LONG_SPLIT_MAX = 512;
 static int launch_attn(const LayerArgs &a, hipStream_t s) {
   const int ppw = attn_ppw(a.max_ctx);

@@ -84,7 +84,9 @@ __global__ __launch_bounds__(64 * PF_ROPE_WAVES) void k_pf_rope(PrefillArgs a) {
 // heads of one KV group: NP = QT * GH (position, head) pairs over the same K
 // and V rows.
 //   scores   a block of 256 K rows goes through LDS (coalesced 16-byte
-//            loads, the next block's in flight); lane t of a wave decodes K
+//            loads; the next block's are issued before the scores, but the
+//            compiler keeps them in scratch memory, so they are waited for
+//            there); lane t of a wave decodes K
 //            row t once and forms that row's SkylakeX ddot with half of the
 //            pairs' q (ddot64_rows);
 //   softmax  one wave per pair, the whole row of scores in LDS, numpy's
